@@ -1,8 +1,8 @@
 // Host orchestration of the energy/force pipeline and the C ABI (include/nnp_capi.h).
 //
 // Pipeline for a batch of structures (all kernels cover every atom of every structure):
-//   1. neighbour list      k_zero, k_bin_atoms / k_scan_excl / k_fill_bins / k_neigh_cells
-//                          (large cells), k_neigh_allpairs (small cells)
+//   1. neighbour list      k_bins_small or k_bin_atoms / k_bin_scan / k_fill_bins, then
+//                          k_neigh_cells_bits (large cells), k_neigh_allpairs (small cells)
 //   2. descriptors         k_symm<T, NE, NC>                 -> G
 //   3. networks            k_net_f64 | k_net_mixed, all species' 16-atom tiles -> E_i, dE/dG
 //   4. force terms         k_force<T, NE, NC>                 -> X (per neighbour entry)
@@ -382,7 +382,7 @@ Engine::Engine(const Engine& o, int) : host(o.host), pb(o.pb), shape(o.shape) {
 size_t Engine::workspace_bytes() const {
     size_t b = 0;
     for (const DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
-                            &d_bfill, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount,
+                            &d_brank, &d_bpos, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount,
                             &d_rlist, &d_out, &d_mom})
         b += m->cap;
     return b;
@@ -400,7 +400,7 @@ Engine::~Engine() {
     if (owns_model)
         for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi}) m->release();
     for (DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
-                      &d_bfill, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})
+                      &d_brank, &d_bpos, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})
         m->release();
     h_up.release();
     h_down.release();
@@ -615,7 +615,8 @@ void Engine::bind_scratch(void* base, size_t bytes, const nnp_structure& s) {
     for (DevMem* m : {&d_cnt, &d_abin, &d_rcount}) take(*m, N * 4);
     take(d_eatom, N * 8);
     take(d_F, N * 24);
-    for (DevMem* m : {&d_bcount, &d_bstart, &d_bfill}) take(*m, nb * 4);
+    take(d_bcount, nb * 4);
+    take(d_bstart, (nb + 1) * 4);
     take(d_G, N * ldg * 8);
     take(d_dEdG, N * ldg * 8);
     // per row slot: neighbour index 4, metadata 4, displacement 32, FP64 force term 32, receiver
@@ -631,6 +632,10 @@ void Engine::bind_scratch(void* base, size_t bytes, const nnp_structure& s) {
     take(d_meta, N * fit * 4);
     take(d_nbrr, N * fit * 32);
     take(d_X, N * fit * 32);
+    // the search's scratch: the force terms are written after it has been read
+    d_bpos.bind(d_X.p, N * sizeof(float4));
+    d_brank.bind((char*)d_X.p + N * sizeof(float4), N * 4);
+    HIPCHK(hipMemsetAsync(d_bcount.p, 0, nb * 4, stream));
     take(d_rlist, N * fit * 4);
     HIPCHK(hipMemsetAsync(d_maxcnt.p, 0, 64, stream));  // counters the mode does not write read as zero
     maxp = 0;
@@ -656,9 +661,13 @@ void Engine::build_neighbors(bool all_images) {
         d_work.reserve(64);
         if (nbins > 0) {
             d_abin.reserve((size_t)ntot * 4);
+            const size_t count_cap = d_bcount.cap;
             d_bcount.reserve((size_t)nbins * 4);
-            d_bstart.reserve((size_t)nbins * 4);
-            d_bfill.reserve((size_t)nbins * 4);
+            // the bin counters are zero between passes: the scan clears what it has read
+            if (d_bcount.cap != count_cap) HIPCHK(hipMemsetAsync(d_bcount.p, 0, d_bcount.cap, stream));
+            d_bstart.reserve((size_t)(nbins + 1) * 4);
+            d_brank.reserve((size_t)ntot * 4);
+            d_bpos.reserve((size_t)ntot * sizeof(float4));
         }
         // serving lanes check the count at the download instead (one host sync per batch), staging
         // full rows in LDS; when full rows do not fit, the count is read here and the rows staged
@@ -916,7 +925,7 @@ void Engine::net_dims(int& maxw, int& dersum) const {
 }
 
 // Enqueue the fused persistent kernel over the current batch (work counter must be zero:
-// k_zero in the neighbour launch clears it).
+// the neighbour launch clears it).
 void Engine::fused(bool mixed, uint32_t flags, int nblocks) {
     int maxw, dersum;
     net_dims(maxw, dersum);
@@ -1130,7 +1139,8 @@ NeighborArgs Engine::neighbor_args(bool all_images) const {
     a.atom_bin = (int*)d_abin.p;
     a.bin_count = (int*)d_bcount.p;
     a.bin_start = (int*)d_bstart.p;
-    a.bin_fill = (int*)d_bfill.p;
+    a.bin_rank = (int*)d_brank.p;
+    a.bin_pos = (float4*)d_bpos.p;
     // the binning writes the cell-list atoms in bin order over the first ncell centres, so every
     // per-centre kernel walking the centres in XCD-local order takes spatially compact runs
     a.bin_atoms = (int*)d_centres.p;

@@ -90,10 +90,11 @@ struct NeighborArgs {
     int npair;
     int nbins;
     int* atom_bin = nullptr;
-    int* bin_count = nullptr;
-    int* bin_start = nullptr;
-    int* bin_fill = nullptr;
+    int* bin_count = nullptr;  // zero between passes (the scan clears what it reads)
+    int* bin_start = nullptr;  // nbins + 1
+    int* bin_rank = nullptr;  // place of each atom inside its bin (batches binned by several blocks)
     int* bin_atoms = nullptr;
+    float4* bin_pos = nullptr;  // bin-ordered fractional coordinates (FP32) and atom index
     int all_images;
     int cell_natoms_max = 0;  // atoms of the largest cell-list structure (LDS bitmap size)
     bool count_max = true;    // fold the largest neighbour count into maxcnt after the search
@@ -255,7 +256,7 @@ class Engine {
     HostPinned h_up, h_down;
     DevView d_pos, d_type, d_astruc, d_strucs, d_centres, d_spatoms;
     DevMem d_cnt, d_nbrj, d_meta, d_nbrr, d_maxcnt;
-    DevMem d_abin, d_bcount, d_bstart, d_bfill;
+    DevMem d_abin, d_bcount, d_bstart, d_brank, d_bpos;
     DevMem d_G, d_dEdG, d_X, d_eatom, d_F;
     // per-centre moment tables [S][NE][35] the moment-only descriptor kernel leaves for the
     // force-term kernel of the same rows (which then skips its own moment sums); mom_fresh is the

@@ -74,14 +74,18 @@ __device__ __forceinline__ void image_vec(const DevStruc& s, int n, double& x, d
     z = (double)a * s.Rv[2] + (double)b * s.Rv[5] + (double)c * s.Rv[8];
 }
 
+// Exclusive prefix sum over the wavefront in six DPP adds: shifts by 1, 2, 4 and 8 inside each row of 16
+// lanes, then the last lane of row 0 (2) onto row 1 (3), then lane 31 onto rows 2 and 3.
 __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
+    (void)lane;
     int x = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(x, o, kWave);
-        if (lane >= o) x += y;
-    }
-    total = __shfl(x, kWave - 1, kWave);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    total = __builtin_amdgcn_readlane(x, kWave - 1);
     return x - v;
 }
 
@@ -122,13 +126,28 @@ __device__ __forceinline__ ImgRange img_range(const DevStruc& s, double bx, doub
     return g;
 }
 
+// The per-pass counters (neighbour maximum, missed reactions, work counter of the fused kernel), cleared by
+// the first block of the neighbour kernels: nothing else touches them before the force assembly.
+struct PassCounters {
+    int* maxcnt;
+    int* work;
+};
+__device__ __forceinline__ void clear_counters(const PassCounters& pc) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        pc.maxcnt[0] = 0;  // neighbour maximum
+        pc.maxcnt[1] = 0;  // reactions missed by the force assembly's gather
+        if (pc.work) *pc.work = 0;
+    }
+}
+
 // ------------------------------------------------------------------ all-pairs search
 __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                           const double* __restrict__ pos, const int* __restrict__ type,
                                                           const int* __restrict__ centres, double rc2, int maxp,
                                                           int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                           int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                          int* __restrict__ maxcnt) {
+                                                          PassCounters pc) {
+    clear_counters(pc);
     const int i = centres[blockIdx.x];
     const DevStruc& s = S[atom_struc[i]];
     const int lane = threadIdx.x;
@@ -237,54 +256,83 @@ __device__ __forceinline__ int bin_xyz(const SG& s, double x, double y, double z
     }
     return s.bin0 + (b[0] * s.nbin[1] + b[1]) * s.nbin[2] + b[2];
 }
+// An atom's entry in the bin-ordered candidate array: its fractional coordinates in [0, 1] rounded to
+// FP32 and its index, what the cell-list search's distance filter reads.
+template <class SG>
+__device__ __forceinline__ float4 bin_entry(const SG& s, double x, double y, double z, int i) {
+    float f[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const double v = s.RInv[3 * r] * x + s.RInv[3 * r + 1] * y + s.RInv[3 * r + 2] * z;
+        f[r] = (float)(v - floor(v));
+    }
+    return make_float4(f[0], f[1], f[2], __int_as_float(i));
+}
 __device__ __forceinline__ int bin_of(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                       const double* __restrict__ pos, int i) {
     return bin_xyz(S[atom_struc[i]], pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]);
 }
 
+// Binning of the cell-list atoms: each atom's bin, every bin's first slot (nbins + 1 starts, so a bin ends
+// where the next begins), and in bin order the atoms and their filter entries.  The order inside a bin is set by
+// atomics and does not matter: the search places its entries by index.
+//
+// Up to kBinsSmallAtoms atoms of one structure (half as many of several, whose cells are looked up per atom)
+// one workgroup does it all with the counters in LDS, each thread's atoms in registers between the count
+// and the fill; larger batches take three launches (count with each atom's place in its bin, scan, fill).
+// Kernel times, one workgroup against the three launches: 2048 atoms 7.8 / 10.1 us, 4096 atoms 9.4-11.5 / 10.9 us
+// (and two launch gaps), 8192 atoms 18.8 / 11.2 us; 8192 atoms of 16 structures 25.9 / 11.6 us, 32768
+// atoms of 16 structures 75 us / 14 us.
+// ONE: a single structure, whose cell is read once per wavefront (scalar loads) instead of per atom.
 __global__ void k_bin_atoms(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                             const double* __restrict__ pos, int natoms_total, int* __restrict__ atom_bin,
-                            int* __restrict__ bin_count) {
+                            int* __restrict__ bin_count, int* __restrict__ bin_rank) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= natoms_total) return;
     const int bin = bin_of(S, atom_struc, pos, i);
     atom_bin[i] = bin;
-    if (bin >= 0) atomicAdd(&bin_count[bin], 1);
+    if (bin >= 0) bin_rank[i] = atomicAdd(&bin_count[bin], 1);
 }
 
-// Small batches: the counter reset, binning, bin scan and scatter of the four kernels below in
-// one workgroup with the bin counters in LDS (one launch instead of four at a few thousand atoms).
-// ONE: a single structure, whose cell is read once per wavefront (scalar loads) instead of per atom.
-constexpr int kBinsSmallAtoms = 32768;
+constexpr int kBinsSmallAtoms = 4096;
 constexpr int kBinsSmallBins = 4096;
+constexpr int kBinsPerThread = kBinsSmallAtoms / 1024;
+
+// Exclusive scan of one value per thread over 1024 threads, and the block's total.
+__device__ __forceinline__ int block_excl_scan(int v, int* part, int& total) {
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    int wtot;
+    int x = wave_excl_scan(v, lane, wtot);
+    if (lane == 0) part[wv] = wtot;
+    __syncthreads();
+    total = 0;
+#pragma unroll
+    for (int k = 0; k < 1024 / kWave; ++k) {
+        x += k < wv ? part[k] : 0;
+        total += part[k];
+    }
+    return x;
+}
+
 template <bool ONE>
 __global__ __launch_bounds__(1024) void k_bins_small(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                      const double* __restrict__ pos, int ntot, int nbins,
-                                                     int* __restrict__ maxcnt, int* __restrict__ work,
-                                                     int* __restrict__ atom_bin, int* __restrict__ bin_count,
-                                                     int* __restrict__ bin_start, int* __restrict__ bin_atoms) {
+                                                     int* __restrict__ atom_bin, int* __restrict__ bin_start,
+                                                     int* __restrict__ bin_atoms, float4* __restrict__ bin_pos) {
     __shared__ int cnt_l[kBinsSmallBins];
-    __shared__ int start_l[kBinsSmallBins];
     __shared__ int part[1024 / kWave];
     const int t = threadIdx.x;
-    if (t == 0) {
-        maxcnt[0] = 0;  // neighbour maximum
-        maxcnt[1] = 0;  // reactions missed by the force assembly's gather
-        if (work) *work = 0;
-    }
     for (int b = t; b < nbins; b += 1024) cnt_l[b] = 0;
-    __syncthreads();
-    // each thread's atoms i = t + 1024 k keep their bins in registers for the fill below
-    int mybin[kBinsSmallAtoms / 1024];
-#pragma unroll
-    for (int k = 0; k < kBinsSmallAtoms / 1024; ++k) mybin[k] = -1;
     BinGeom g1{};
     if constexpr (ONE) g1 = bin_geom(S[0]);
-    // groups of four atoms per thread; the positions of a group are loaded unconditionally at
-    // clamped (in-bounds) indices, so the four loads go out together (a guarded load becomes a
-    // branch with a full wait after it); the exit test is the same for the whole block
+    __syncthreads();
+    // each thread's atoms i = t + 1024 k, in groups of four; the positions of a group are loaded
+    // unconditionally at clamped (in-bounds) indices, so the four loads go out together (a guarded load
+    // becomes a branch with a full wait after it); the exit test is the same for the whole block
+    int mybin[kBinsPerThread], rank[kBinsPerThread];
+    float4 entry[kBinsPerThread];
 #pragma unroll
-    for (int k0 = 0; k0 < kBinsSmallAtoms / 1024; k0 += 4) {
+    for (int k0 = 0; k0 < kBinsPerThread; k0 += 4) {
         if (k0 * 1024 >= ntot) break;
         double px[4], py[4], pz[4];
 #pragma unroll
@@ -296,17 +344,26 @@ __global__ __launch_bounds__(1024) void k_bins_small(const DevStruc* __restrict_
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int i = t + 1024 * (k0 + q);
+            const int k = k0 + q, i = t + 1024 * k;
+            mybin[k] = -1;
             if (i < ntot) {
-                const int bin = ONE ? bin_xyz(g1, px[q], py[q], pz[q]) : bin_of(S, atom_struc, pos, i);
+                int bin;
+                if constexpr (ONE) {
+                    bin = bin_xyz(g1, px[q], py[q], pz[q]);
+                    entry[k] = bin_entry(g1, px[q], py[q], pz[q], i);
+                } else {
+                    const DevStruc& s = S[atom_struc[i]];
+                    bin = bin_xyz(s, px[q], py[q], pz[q]);
+                    if (bin >= 0) entry[k] = bin_entry(s, px[q], py[q], pz[q], i);
+                }
                 atom_bin[i] = bin;
-                mybin[k0 + q] = bin;
-                if (bin >= 0) atomicAdd(&cnt_l[bin], 1);
+                mybin[k] = bin;
+                if (bin >= 0) rank[k] = atomicAdd(&cnt_l[bin], 1);
             }
         }
     }
     __syncthreads();
-    // exclusive scan: four consecutive bins per thread, then a scan of the 1024 thread sums
+    // exclusive scan in place: four consecutive bins per thread, then a scan of the 1024 thread sums
     int loc[4], sum = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -314,49 +371,70 @@ __global__ __launch_bounds__(1024) void k_bins_small(const DevStruc* __restrict_
         loc[k] = sum;
         sum += b < nbins ? cnt_l[b] : 0;
     }
-    // inclusive scan inside each wavefront (shuffles), then the 16 wavefront totals
-    const int lane = t & (kWave - 1), wv = t / kWave;
-    int inc = sum;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(inc, o, kWave);
-        if (lane >= o) inc += y;
-    }
-    if (lane == kWave - 1) part[wv] = inc;
-    __syncthreads();
-    int excl = inc - sum;
-    for (int k = 0; k < wv; ++k) excl += part[k];
+    int total;
+    const int excl = block_excl_scan(sum, part, total);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int b = 4 * t + k;
         if (b < nbins) {
-            const int st = excl + loc[k];
-            bin_start[b] = st;
-            bin_count[b] = cnt_l[b];
-            start_l[b] = st;
+            bin_start[b] = excl + loc[k];
+            cnt_l[b] = excl + loc[k];
         }
     }
-    __syncthreads();
-    for (int b = t; b < nbins; b += 1024) cnt_l[b] = 0;  // now the fill counters
+    if (t == 0) bin_start[nbins] = total;
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kBinsSmallAtoms / 1024; ++k) {
+    for (int k = 0; k < kBinsPerThread; ++k) {
+        if (k * 1024 >= ntot) break;
         const int b = mybin[k];
         if (b < 0) continue;
-        const int slot = atomicAdd(&cnt_l[b], 1);
-        bin_atoms[start_l[b] + slot] = t + 1024 * k;
+        const int slot = cnt_l[b] + rank[k];
+        bin_atoms[slot] = t + 1024 * k;
+        bin_pos[slot] = entry[k];
     }
 }
 
-// Scatter atoms into their bins.  Order inside a bin does not matter: candidates are sorted.
-__global__ void k_fill_bins(const int* __restrict__ atom_bin, int natoms_total, const int* __restrict__ bin_start,
-                            int* __restrict__ bin_fill, int* __restrict__ bin_atoms) {
+// Bin starts (exclusive scan of the counts, the total last) by one block, four bins per thread and step; the
+// counts are cleared behind it for the next pass.
+__global__ __launch_bounds__(1024) void k_bin_scan(int* __restrict__ count, int* __restrict__ start, int nbins) {
+    __shared__ int part[1024 / kWave];
+    const int t = threadIdx.x;
+    int carry = 0;
+    for (int base = 0; base < nbins; base += 4096) {
+        const int b0 = base + 4 * t;
+        int v[4], sum = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = b0 + k < nbins ? count[b0 + k] : 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += v[k];
+        int total;
+        int at = carry + block_excl_scan(sum, part, total);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (b0 + k < nbins) {
+                start[b0 + k] = at;
+                count[b0 + k] = 0;
+            }
+            at += v[k];
+        }
+        carry += total;
+        __syncthreads();  // part is rewritten by the next step
+    }
+    if (t == 0) start[nbins] = carry;
+}
+
+// Scatter atoms into their bins.
+__global__ void k_fill_bins(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
+                            const double* __restrict__ pos, const int* __restrict__ atom_bin, int natoms_total,
+                            const int* __restrict__ bin_start, const int* __restrict__ bin_rank,
+                            int* __restrict__ bin_atoms, float4* __restrict__ bin_pos) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= natoms_total) return;
     const int b = atom_bin[i];
     if (b < 0) return;
-    const int slot = atomicAdd(&bin_fill[b], 1);
-    bin_atoms[bin_start[b] + slot] = i;
+    const int slot = bin_start[b] + bin_rank[i];
+    bin_atoms[slot] = i;
+    bin_pos[slot] = bin_entry(S[atom_struc[i]], pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], i);
 }
 
 // One wavefront per centre: gather candidates from the 27 neighbouring bins, keep those with
@@ -365,12 +443,13 @@ __global__ void k_fill_bins(const int* __restrict__ atom_bin, int natoms_total, 
 __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                        const double* __restrict__ pos, const int* __restrict__ type,
                                                        const int* __restrict__ centres, const int* __restrict__ atom_bin,
-                                                       const int* __restrict__ bin_start, const int* __restrict__ bin_count,
+                                                       const int* __restrict__ bin_start,
                                                        const int* __restrict__ bin_atoms, double rc2, int maxp, int n2cap,
                                                        int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                        int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                       int* __restrict__ maxcnt) {
+                                                       PassCounters pc) {
     extern __shared__ double lds_cells[];
+    clear_counters(pc);
     const int cap = maxp;
     double* vals = lds_cells;
     int* keys = (int*)(vals + 4 * cap);
@@ -394,7 +473,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
         const int cz = s.nbin[2] < 3 ? o2 : (bz + o2 - 1 + s.nbin[2]) % s.nbin[2];
         const int b = s.bin0 + (cx * s.nbin[1] + cy) * s.nbin[2] + cz;
         bstart = bin_start[b];
-        bcount = bin_count[b];
+        bcount = bin_start[b + 1] - bstart;
     }
     int ncand;
     const int bfirst = wave_excl_scan(bcount, lane, ncand);  // first flat candidate of bin `lane`
@@ -468,52 +547,189 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
     }
 }
 
-// Cell list without a sort: kept neighbours are marked in an LDS bitmap over the structure's
-// atoms (one bit each, set with an LDS atomic OR, so the result does not depend on the order
-// the candidates are visited in), then read out in ascending index order, which is the
-// reference's order; each kept entry's displacement is recomputed by the same Cell::diff.
-// LDS: one 32-bit word per 32 atoms of the largest cell-list structure of the batch.
+// Cell list without a sort.  One wavefront per centre:
+//  1. the 27 neighbouring bins are at most 18 runs of consecutive bins (three bins along the last
+//     axis, two runs where they wrap), one flat candidate list;
+//  2. filter: every candidate's distance from the bin-ordered FP32 fractional coordinates (one
+//     coalesced 16-byte load), against rc plus a bound on the FP32 error; what may be within rc
+//     (45-70 of some 320 candidates) goes to a short list in LDS;
+//  3. the listed candidates take the reference's Cell::diff and its inclusive test in FP64; kept ones set
+//     their bit in an LDS bitmap over the structure's atoms (an atomic OR, so the visiting order does
+//     not matter) and stay in registers;
+//  4. each kept entry's place in its row is the number of set bits before its own (a prefix count
+//     per word, a popcount inside it): ascending index, the reference's order.
+// Bound by the VALU instructions it issues and the latency of its loads.  Cell::diff is about 60 FP64
+// operations; on every candidate and again on every set bit (a lane per bitmap word, most lanes idle) the
+// search took 18.0 us on 4096 atoms (2 species, rc 6) and 205 us on 16 x 4096 atoms (rc 6.5); with the filter
+// 10.9 us and 102 us (728 instead of 1516 VALU instructions per centre).
+//
+// The filter must keep everything Cell::diff would.  A cell-list structure has every height > 2 rc, so an
+// entry within rc has fractional components |f| <= rc / h < 1/2 and is the image that rounding picks; the FP32
+// coordinates (in [0, 1], error 2^-25) put the distance off by less than 4e-7 ||R||_F, and the filter adds
+// 1e-6 ||R||_F.  Where some rc / h is within 1e-4 of 1/2 the rounding could take the other image, and
+// where a row could hold more than the register batches (maxp > 192) or the filter lists more than they
+// hold, every candidate takes Cell::diff and the kept set is read out of the bitmap instead.
+// LDS: bitmap, one 32-bit word per 32 atoms of the largest cell-list structure (nwords_max); 16-bit prefix
+// counts per word.
+constexpr int kNeighList = 2 * kWave;  // two register batches
+struct NeighEntry {  // a candidate's Cell::diff, j < 0 when it is not kept
+    double x, y, z, d2;
+    int j, t;
+};
 __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
     const DevStruc* __restrict__ S, const int* __restrict__ atom_struc, const double* __restrict__ pos,
     const int* __restrict__ type, int ncell, const int* __restrict__ atom_bin,
-    const int* __restrict__ bin_start, const int* __restrict__ bin_count, const int* __restrict__ bin_atoms,
-    double rc2, int maxp, int* __restrict__ cnt, int* __restrict__ nbr_j, int* __restrict__ nbr_meta,
-    double4* __restrict__ nbr_r) {
+    const int* __restrict__ bin_start, const float4* __restrict__ bin_pos, int one_struc, double rc2, int maxp,
+    int* __restrict__ cnt, int* __restrict__ nbr_j, int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
+    int nwords_max, PassCounters pc) {
     extern __shared__ unsigned int lds_bits[];
+    clear_counters(pc);
+    unsigned short* pre = reinterpret_cast<unsigned short*>(lds_bits + nwords_max);
+    __shared__ int list[kNeighList];
     // centres in the XCD-local order of the cell-list atoms in bin order: the blocks of one XCD
-    // cover one contiguous, spatially compact run of centres, whose candidates' positions and bin
+    // cover one contiguous, spatially compact run of centres, whose candidates' coordinates and bin
     // lists they then share in that XCD's L2 (the centre a block computes does not change any row)
     const int slot = xcd_slot(ncell);
     if (slot < 0) return;
-    const int i = bin_atoms[slot];
-    const DevStruc& s = S[atom_struc[i]];
+    const float4 own = bin_pos[slot];
+    const int i = __builtin_amdgcn_readfirstlane(__float_as_int(own.w));
+    const DevStruc& s = S[one_struc ? 0 : atom_struc[i]];
     const int lane = threadIdx.x;
     const int nwords = (s.natoms + 31) >> 5;
     for (int w = lane; w < nwords; w += kWave) lds_bits[w] = 0u;
-    __syncthreads();
     const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int myb = atom_bin[i] - s.bin0;
-    const int bz = myb % s.nbin[2], by = (myb / s.nbin[2]) % s.nbin[1], bx = myb / (s.nbin[2] * s.nbin[1]);
-    const int n0 = s.nbin[0] < 3 ? s.nbin[0] : 3, n1 = s.nbin[1] < 3 ? s.nbin[1] : 3, n2 = s.nbin[2] < 3 ? s.nbin[2] : 3;
-    const int nb = n0 * n1 * n2;  // <= 27
-    int bstart = 0, bcount = 0;
-    if (lane < nb) {
-        const int o2 = lane % n2, o1 = (lane / n2) % n1, o0 = lane / (n2 * n1);
-        const int cx = s.nbin[0] < 3 ? o0 : (bx + o0 - 1 + s.nbin[0]) % s.nbin[0];
-        const int cy = s.nbin[1] < 3 ? o1 : (by + o1 - 1 + s.nbin[1]) % s.nbin[1];
-        const int cz = s.nbin[2] < 3 ? o2 : (bz + o2 - 1 + s.nbin[2]) % s.nbin[2];
-        const int b = s.bin0 + (cx * s.nbin[1] + cy) * s.nbin[2] + cz;
-        bstart = bin_start[b];
-        bcount = bin_count[b];
+    const int nb0 = s.nbin[0], nb1 = s.nbin[1], nb2 = s.nbin[2];
+    const unsigned myb = (unsigned)(atom_bin[i] - s.bin0), byx = myb / (unsigned)nb2, bx_ = byx / (unsigned)nb1;
+    const int bz = (int)(myb - byx * nb2), by = (int)(byx - bx_ * nb1), bx = (int)bx_;
+    // lane r owns run r: an (x, y) pair of neighbouring bins (an axis with fewer than 3 bins is covered
+    // once) and one of the one or two stretches of bins along z
+    const int n0 = min(nb0, 3), n1 = min(nb1, 3);
+    const int nz = nb2 > 3 && (bz == 0 || bz == nb2 - 1) ? 2 : 1;
+    const int nruns = n0 * n1 * nz;
+    int first = 0, rcount = 0;
+    if (lane < nruns) {
+        const int hf = nz == 2 ? (lane & 1) : 0, xy = nz == 2 ? (lane >> 1) : lane;
+        const int ox = (xy >= n1) + (xy >= 2 * n1), oy = xy - ox * n1;
+        int cx = ox, cy = oy, z0, z1;
+        if (nb0 >= 3) {
+            cx = bx + ox - 1;
+            cx = cx < 0 ? cx + nb0 : (cx >= nb0 ? cx - nb0 : cx);
+        }
+        if (nb1 >= 3) {
+            cy = by + oy - 1;
+            cy = cy < 0 ? cy + nb1 : (cy >= nb1 ? cy - nb1 : cy);
+        }
+        if (nb2 <= 3) {
+            z0 = 0;
+            z1 = nb2 - 1;
+        } else if (nz == 1) {
+            z0 = bz - 1;
+            z1 = bz + 1;
+        } else if (hf == 0) {  // the stretch at the low end
+            z0 = 0;
+            z1 = bz == 0 ? 1 : 0;
+        } else {
+            z0 = bz == 0 ? nb2 - 1 : nb2 - 2;
+            z1 = nb2 - 1;
+        }
+        const int b = s.bin0 + (cx * nb1 + cy) * nb2;
+        first = bin_start[b + z0];
+        rcount = bin_start[b + z1 + 1] - first;
     }
     int ncand;
-    const int bfirst = wave_excl_scan(bcount, lane, ncand);
-    for (int c0 = 0; c0 < ncand; c0 += kWave) {
+    const int rfirst = wave_excl_scan(rcount, lane, ncand);  // first flat candidate of run `lane`
+    // The bin-order slot of flat candidate c = c0 + lane, for chunks c0 taken in order: the runs that start in
+    // the chunk are walked (the same for every lane), each taking over the candidates from its start on;
+    // empty runs are taken over by the next one.  run: the last run that starts at or before the chunk.
+    const int shift = first - rfirst;
+    int run = 0;
+    auto chunk_slot = [&](int c0) {
         const int c = c0 + lane;
-        const int ob = owner_bin(bfirst, nb, c);
-        const int ostart = __shfl(bstart, ob, kWave), ofirst = __shfl(bfirst, ob, kWave);
+        int d = __builtin_amdgcn_readlane(shift, run);
+        while (run + 1 < nruns) {
+            const int f = __builtin_amdgcn_readlane(rfirst, run + 1);
+            if (f > c0 + kWave - 1) break;
+            ++run;
+            d = c >= f ? __builtin_amdgcn_readlane(shift, run) : d;
+        }
+        return c < ncand ? c + d : slot;  // past the list: any valid slot
+    };
+    int nlist = 0;
+    bool full = maxp > 192 || fmax(fmax(s.reach[0], s.reach[1]), s.reach[2]) > 0.4999;
+    if (!full) {
+        float R[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) R[q] = (float)s.R[q];
+        const double rlim = sqrt(rc2) + 1e-6 * s.fro;
+        const float lim = (float)(rlim * rlim * (1.0 + 2e-6));
+        for (int c0 = 0; c0 < ncand; c0 += kWave) {
+            const int c = c0 + lane;
+            const float4 v = bin_pos[chunk_slot(c0)];
+            float dx = own.x - v.x, dy = own.y - v.y, dz = own.z - v.z;
+            dx -= rintf(dx);
+            dy -= rintf(dy);
+            dz -= rintf(dz);
+            const float x = R[0] * dx + R[1] * dy + R[2] * dz, y = R[3] * dx + R[4] * dy + R[5] * dz,
+                        z = R[6] * dx + R[7] * dy + R[8] * dz;
+            const int gj = __float_as_int(v.w);
+            const bool near = c < ncand && gj != i && x * x + y * y + z * z <= lim;
+            const unsigned long long m = __ballot(near);
+            const int at = nlist + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            if (near && at < kNeighList) list[at] = gj;
+            nlist += __popcll(m);
+        }
+        full = nlist > kNeighList;
+    }
+    __syncthreads();
+    const int64_t row = (int64_t)i * maxp;
+    const int per = (nwords + kWave - 1) / kWave;  // lanes own contiguous word ranges
+    const int w0 = min(lane * per, nwords), w1 = min(w0 + per, nwords);
+    if (!full) {
+        auto take = [&](int p) {
+            NeighEntry e{0.0, 0.0, 0.0, 0.0, -1, 0};
+            if (p < nlist) {
+                const int gj = list[p];
+                e.t = type[gj];
+                cell_diff(s, xi - pos[3 * gj], yi - pos[3 * gj + 1], zi - pos[3 * gj + 2], e.x, e.y, e.z);
+                e.d2 = e.x * e.x + e.y * e.y + e.z * e.z;
+                if (e.d2 <= rc2) {
+                    e.j = gj - s.atom0;
+                    atomicOr(&lds_bits[e.j >> 5], 1u << (e.j & 31));
+                }
+            }
+            return e;
+        };
+        auto put = [&](const NeighEntry& e) {
+            if (e.j < 0) return;
+            const int w = e.j >> 5;
+            const int p = pre[w] + __popc(lds_bits[w] & ((1u << (e.j & 31)) - 1u));
+            const double d = sqrt(e.d2);
+            // one image per j: it is the minimum image when below ||R||_F (neighbor.cpp:132-140)
+            if (p < maxp) put_entry(row + p, e.j, 0, e.t, d < s.fro, e.x, e.y, e.z, d, nbr_j, nbr_meta, nbr_r);
+        };
+        const NeighEntry e0 = take(lane);
+        NeighEntry e1{0.0, 0.0, 0.0, 0.0, -1, 0};
+        if (nlist > kWave) e1 = take(kWave + lane);
+        __syncthreads();
+        int mine = 0;
+        for (int w = w0; w < w1; ++w) mine += __popc(lds_bits[w]);
+        int kept;
+        int at = wave_excl_scan(mine, lane, kept);
+        for (int w = w0; w < w1; ++w) {
+            pre[w] = (unsigned short)at;
+            at += __popc(lds_bits[w]);
+        }
+        __syncthreads();
+        put(e0);
+        if (nlist > kWave) put(e1);
+        if (lane == 0) cnt[i] = kept;
+        return;
+    }
+    run = 0;
+    for (int c0 = 0; c0 < ncand; c0 += kWave) {
+        const int c = c0 + lane, sl = chunk_slot(c0);
         if (c < ncand) {
-            const int gj = bin_atoms[ostart + (c - ofirst)];
+            const int gj = __float_as_int(bin_pos[sl].w);
             if (gj != i) {
                 double rx, ry, rz;
                 cell_diff(s, xi - pos[3 * gj], yi - pos[3 * gj + 1], zi - pos[3 * gj + 2], rx, ry, rz);
@@ -525,14 +741,10 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
         }
     }
     __syncthreads();
-    // lanes own contiguous word ranges; a wave prefix sum of their popcounts gives the slots
-    const int per = (nwords + kWave - 1) / kWave;
-    const int w0 = min(lane * per, nwords), w1 = min(w0 + per, nwords);
     int mine = 0;
     for (int w = w0; w < w1; ++w) mine += __popc(lds_bits[w]);
     int kept;
     int at = wave_excl_scan(mine, lane, kept);
-    const int64_t row = (int64_t)i * maxp;
     for (int w = w0; w < w1; ++w) {
         unsigned int m = lds_bits[w];
         while (m) {
@@ -543,7 +755,6 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
                 double rx, ry, rz;
                 cell_diff(s, xi - pos[3 * gj], yi - pos[3 * gj + 1], zi - pos[3 * gj + 2], rx, ry, rz);
                 const double d = sqrt(rx * rx + ry * ry + rz * rz);
-                // one image per j: it is the minimum image when below ||R||_F (neighbor.cpp:132-140)
                 put_entry(row + at, lj, 0, type[gj], d < s.fro, rx, ry, rz, d, nbr_j, nbr_meta, nbr_r);
             }
             ++at;
@@ -569,47 +780,6 @@ __global__ __launch_bounds__(256) void k_count_max(const int* __restrict__ cnt, 
     }
 }
 
-// Clears the per-pass counters (max entry count, missed reactions and the cell-list bin counters)
-// in one launch.
-__global__ void k_zero(int* __restrict__ maxcnt, int* __restrict__ work, int* __restrict__ bin_count,
-                       int* __restrict__ bin_fill, int nbins) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) {
-        maxcnt[0] = 0;  // neighbour maximum
-        maxcnt[1] = 0;  // reactions missed by the force assembly's gather
-        if (work) *work = 0;
-    }
-    if (t < nbins) {
-        bin_count[t] = 0;
-        bin_fill[t] = 0;
-    }
-}
-
-// Exclusive scan of n ints by one block (bin starts of the cell list).
-__global__ __launch_bounds__(1024) void k_scan_excl(const int* __restrict__ in, int* __restrict__ out, int n) {
-    // blocks of 1024: inclusive scans inside each wavefront (shuffles), then the 16 wavefront
-    // totals, then the running carry of the blocks before
-    __shared__ int part[1024 / kWave];
-    const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
-    int carry = 0;
-    for (int base = 0; base < n; base += 1024) {
-        const int v = base + t < n ? in[base + t] : 0;
-        int inc = v;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const int y = __shfl_up(inc, o, kWave);
-            if (lane >= o) inc += y;
-        }
-        if (lane == kWave - 1) part[wv] = inc;
-        __syncthreads();
-        int off = carry;
-        for (int k = 0; k < wv; ++k) off += part[k];
-        if (base + t < n) out[base + t] = off + inc - v;
-        for (int k = 0; k < 1024 / kWave; ++k) carry += part[k];
-        __syncthreads();  // part is rewritten by the next block
-    }
-}
-
 }  // namespace atomnn
 
 #include "engine.hpp"
@@ -620,45 +790,42 @@ hipError_t launch_count_max(const int* cnt, int n, int* maxcnt, hipStream_t st);
 
 hipError_t launch_neighbors(const NeighborArgs& a, hipStream_t st) {
     hipError_t e;
-    const bool small = a.ncell > 0 && a.ntot <= kBinsSmallAtoms && a.nbins <= kBinsSmallBins;
-    if (small) {
-        if (a.nstruc == 1)
-            hipLaunchKernelGGL(k_bins_small<true>, dim3(1), dim3(1024), 0, st, a.S, a.atom_struc, a.pos, a.ntot,
-                               a.nbins, a.maxcnt, a.work, a.atom_bin, a.bin_count, a.bin_start, a.bin_atoms);
-        else
-            hipLaunchKernelGGL(k_bins_small<false>, dim3(1), dim3(1024), 0, st, a.S, a.atom_struc, a.pos, a.ntot,
-                               a.nbins, a.maxcnt, a.work, a.atom_bin, a.bin_count, a.bin_start, a.bin_atoms);
-    } else {
-        const int nz = a.ncell > 0 ? a.nbins : 0;
-        hipLaunchKernelGGL(k_zero, dim3((nz + 255) / 256 + 1), dim3(256), 0, st, a.maxcnt, a.work, a.bin_count,
-                           a.bin_fill, nz);
-    }
+    const PassCounters pc{a.maxcnt, a.work};
     if (a.ncell > 0) {
-        if (!small) {
-            hipLaunchKernelGGL(k_bin_atoms, dim3((a.ntot + 255) / 256), dim3(256), 0, st, a.S, a.atom_struc, a.pos,
-                               a.ntot, a.atom_bin, a.bin_count);
-            hipLaunchKernelGGL(k_scan_excl, dim3(1), dim3(1024), 0, st, a.bin_count, a.bin_start, a.nbins);
-            hipLaunchKernelGGL(k_fill_bins, dim3((a.ntot + 255) / 256), dim3(256), 0, st, a.atom_bin, a.ntot,
-                               a.bin_start, a.bin_fill, a.bin_atoms);
+        if (a.ntot <= (a.nstruc == 1 ? kBinsSmallAtoms : kBinsSmallAtoms / 2) && a.nbins <= kBinsSmallBins) {
+            if (a.nstruc == 1)
+                hipLaunchKernelGGL(k_bins_small<true>, dim3(1), dim3(1024), 0, st, a.S, a.atom_struc, a.pos, a.ntot,
+                                   a.nbins, a.atom_bin, a.bin_start, a.bin_atoms, a.bin_pos);
+            else
+                hipLaunchKernelGGL(k_bins_small<false>, dim3(1), dim3(1024), 0, st, a.S, a.atom_struc, a.pos, a.ntot,
+                                   a.nbins, a.atom_bin, a.bin_start, a.bin_atoms, a.bin_pos);
+        } else {
+            const dim3 grid((a.ntot + 255) / 256);
+            hipLaunchKernelGGL(k_bin_atoms, grid, dim3(256), 0, st, a.S, a.atom_struc, a.pos, a.ntot, a.atom_bin,
+                               a.bin_count, a.bin_rank);
+            hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, a.bin_count, a.bin_start, a.nbins);
+            hipLaunchKernelGGL(k_fill_bins, grid, dim3(256), 0, st, a.S, a.atom_struc, a.pos, a.atom_bin, a.ntot,
+                               a.bin_start, a.bin_rank, a.bin_atoms, a.bin_pos);
         }
         const size_t bits_lds = (size_t)((a.cell_natoms_max + 31) / 32) * 4;
-        if (bits_lds <= 32768) {
-            hipLaunchKernelGGL(k_neigh_cells_bits, dim3(xcd_grid(a.ncell)), dim3(kWave), bits_lds, st, a.S,
-                               a.atom_struc, a.pos, a.type, a.ncell, a.atom_bin, a.bin_start, a.bin_count,
-                               a.bin_atoms, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r);
+        if (bits_lds <= 32768) {  // the bitmap, then its prefix counts (16 bits per word)
+            hipLaunchKernelGGL(k_neigh_cells_bits, dim3(xcd_grid(a.ncell)), dim3(kWave),
+                               bits_lds + (bits_lds / 2 + 3) / 4 * 4, st, a.S, a.atom_struc, a.pos, a.type, a.ncell,
+                               a.atom_bin, a.bin_start, a.bin_pos, a.nstruc == 1, a.rc2, a.maxp, a.cnt, a.nbr_j,
+                               a.nbr_meta, a.nbr_r, (int)(bits_lds / 4), pc);
         } else {  // very large structures: sort the kept candidates instead
             int n2cap = 1;
             while (n2cap < a.maxp) n2cap <<= 1;
             const size_t lds = (size_t)a.maxp * 32 + (size_t)a.maxp * 4 + (size_t)n2cap * 8;
             hipLaunchKernelGGL(k_neigh_cells, dim3(a.ncell), dim3(kWave), lds, st, a.S, a.atom_struc, a.pos, a.type,
-                               a.cell_centres, a.atom_bin, a.bin_start, a.bin_count, a.bin_atoms, a.rc2, a.maxp, n2cap,
-                               a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.maxcnt);
+                               a.cell_centres, a.atom_bin, a.bin_start, a.bin_atoms, a.rc2, a.maxp, n2cap, a.cnt,
+                               a.nbr_j, a.nbr_meta, a.nbr_r, pc);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.npair > 0) {
         hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave), 0, st, a.S, a.atom_struc, a.pos, a.type,
-                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.maxcnt);
+                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, pc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.ntot > 0 && a.count_max) return launch_count_max(a.cnt, a.ntot, a.maxcnt, st);
