@@ -33,6 +33,17 @@ int grid_shape(int ne, int nc);
 int shape_ne(int shape);  // exponents per centre of a grid shape
 constexpr int kMomK = 35;  // monomials of degree <= 4: the moment table's row length
 constexpr int kMomZ = 4;   // their highest degree
+constexpr int kPowL = 10;  // levels of powers.hpp (lambda = +-1, zeta = 1, 2, 4, 8, 16)
+size_t symm_pow_lds(int ne, bool fp64, int lmaxp, int ldg);
+size_t force_pow_lds(int ne, bool fp64, int lmaxp, int ldg, int ntypes);
+template <typename T>
+hipError_t launch_symm_pow(int ne, const DevPlan* plan, const double* rfe, const double* rfr, const int* atom_type,
+                           const int* centres, int ncentres, const int* cnt, const int* meta, const double4* r, int maxp,
+                           int lmaxp, T* G, int ldg, hipStream_t st);
+template <typename T>
+hipError_t launch_force_pow(int ne, const DevPlan* plan, const double* rfe, const double* rfr, const int* atom_type,
+                            const int* centres, int ncentres, const int* cnt, const int* meta, const double4* r, int maxp,
+                            int lmaxp, const T* dEdG, int ldg, T* X, int ntypes, hipStream_t st);
 size_t symm_lds(int shape, bool fp64, bool ns, int lmaxp, int ldg);
 size_t force_lds(int shape, bool fp64, bool ns, int lmaxp, int ldg);
 size_t net_lds_bytes(const DevNet& n, bool fp64);
@@ -274,6 +285,7 @@ Engine::Engine(HostModel&& hm) : host(std::move(hm)) {
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev));
     build_adjoint_table();
+    build_power_index();
     d_plan.reserve(sizeof(DevPlan));
     HIPCHK(hipMemcpy(d_plan.p, &pb.plan, sizeof(DevPlan), hipMemcpyHostToDevice));
     d_rfe.reserve(pb.rfun_eta.size() * 8);
@@ -360,6 +372,29 @@ void Engine::build_adjoint_table() {
     pb.plan.ang_index = (const int*)d_angi.p;
 }
 
+// Function of each (block, exponent, level) of a model in the domain of powers.hpp: level k for lambda = +1 and
+// zeta = 2^k, 5 + k for lambda = -1.
+void Engine::build_power_index() {
+    const DevPlan& P = pb.plan;
+    if (!P.pow_ne) return;
+    const int T = P.T, nblk = T * (T + 1) / 2;
+    std::vector<int> index((size_t)T * nblk * P.pow_ne * kPowL, -1);
+    for (int t = 0; t < T; ++t)
+        for (int blk = 0; blk < nblk; ++blk) {
+            const DevAngular& A = P.ang[t][blk];
+            for (int e = 0; e < A.ne; ++e)
+                for (int c = 0; c < A.nc; ++c) {
+                    int k = 0;
+                    while ((1 << k) < A.zint[c]) ++k;
+                    if (A.lambda[c] < 0) k += kPowL / 2;
+                    index[(((size_t)t * nblk + blk) * P.pow_ne + e) * kPowL + k] = A.fmap[e * kMaxC + c];
+                }
+        }
+    d_powi.reserve(index.size() * 4);
+    HIPCHK(hipMemcpy(d_powi.p, index.data(), index.size() * 4, hipMemcpyHostToDevice));
+    pb.plan.pow_index = (const int*)d_powi.p;
+}
+
 Engine::Engine(const Engine& o, int) : host(o.host), pb(o.pb), shape(o.shape) {
     owns_model = false;
     pipeline = o.pipeline;
@@ -398,7 +433,8 @@ Engine::~Engine() {
     d_sstart.release();
     d_work.release();
     if (owns_model)
-        for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi}) m->release();
+        for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi, &d_powi})
+            m->release();
     for (DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
                       &d_brank, &d_bpos, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})
         m->release();
@@ -715,6 +751,16 @@ int Engine::mom_flag(size_t base_lds, bool fp64, int bits) {
 
 template <typename T>
 void Engine::descriptors() {
+    // models with zeta up to 16 (powers.hpp); rows that do not fit go on to the generic kernel's own check
+    if (pb.plan.pow_ne && symm_pow_lds(pb.plan.pow_ne, sizeof(T) == 8, lmaxp, pb.plan.ldg) <= 65536) {
+        d_G.reserve((size_t)ntot * pb.plan.ldg * sizeof(T));
+        mom_fresh = 0;
+        HIPCHK(launch_symm_pow<T>(pb.plan.pow_ne, (const DevPlan*)d_plan.p, (const double*)d_rfe.p,
+                                  (const double*)d_rfr.p, (const int*)d_type.p, (const int*)d_centres.p, ntot,
+                                  (const int*)d_cnt.p, (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp,
+                                  (T*)d_G.p, pb.plan.ldg, stream));
+        return;
+    }
     const size_t lds = symm_lds(shape, sizeof(T) == 8, pb.plan.generic, lmaxp, pb.plan.ldg);
     if (lds > 65536) throw unsupported_error("too many neighbours per atom for the descriptor kernel's LDS");
     // mom = 2 when every species takes the moments: no triplet blocks, so the reduction buffer
@@ -814,6 +860,13 @@ void Engine::force_terms() {
                                    (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp, (const T*)d_dEdG.p,
                                    pb.plan.ldg, (T*)d_X.p, pb.plan.T, stream,
                                    mom_fresh == (int)sizeof(T) ? (const T*)d_mom.p : nullptr));
+        return;
+    }
+    if (pb.plan.pow_ne && force_pow_lds(pb.plan.pow_ne, fp64, lmaxp, pb.plan.ldg, pb.plan.T) <= 65536) {
+        HIPCHK(launch_force_pow<T>(pb.plan.pow_ne, (const DevPlan*)d_plan.p, (const double*)d_rfe.p,
+                                   (const double*)d_rfr.p, (const int*)d_type.p, (const int*)d_centres.p, ntot,
+                                   (const int*)d_cnt.p, (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp,
+                                   (const T*)d_dEdG.p, pb.plan.ldg, (T*)d_X.p, pb.plan.T, stream));
         return;
     }
     const size_t lds = force_lds(shape, fp64, pb.plan.generic, lmaxp, pb.plan.ldg);

@@ -281,6 +281,7 @@ PlanBuffers build_plan(const HostModel& m) {
     P.ne_max = 1;
     P.nc_max = 1;
     const int nblk = m.T * (m.T + 1) / 2;
+    bool pow_ok = true, all_mom = true;
     for (int i = 0; i < m.T; ++i) {
         const SpeciesSpec& s = m.sp[i];
         P.nG[i] = s.nG;
@@ -372,6 +373,18 @@ PlanBuffers build_plan(const HostModel& m) {
             P.ang_shared[i] = shared ? 1 : 0;
             P.mom_ok[i] = (shared && ok) ? 1 : 0;
         }
+        // the domain of powers.hpp: GAUSSIAN radial functions, GAUSS angular factors over one exponent table,
+        // lambda = +-1 and zeta a power of two up to 16
+        pow_ok = pow_ok && P.ang_shared[i];
+        all_mom = all_mom && P.mom_ok[i];
+        for (int j = 0; j < m.T; ++j) pow_ok = pow_ok && P.rad[i][j].phi == RAD_GAUSSIAN;
+        for (int b = 0; b < nblk; ++b) {
+            const DevAngular& A = P.ang[i][b];
+            pow_ok = pow_ok && A.phi == ANG_GAUSS;
+            for (int c = 0; c < A.nc; ++c)
+                pow_ok = pow_ok && std::fabs(A.lambda[c]) == 1.0 && A.zint[c] >= 1 && A.zint[c] <= 16 &&
+                         (A.zint[c] & (A.zint[c] - 1)) == 0;
+        }
         // network: weights padded (outputs to 16, inputs to 16) and stored row-major
         const NetSpec& net = s.net;
         DevNet& dn = P.net[i];
@@ -443,6 +456,7 @@ PlanBuffers build_plan(const HostModel& m) {
         pb.rfun_eta.push_back(0.0);
         pb.rfun_rs.push_back(0.0);
     }
+    if (pow_ok && !all_mom && P.ne_max <= 4) P.pow_ne = P.ne_max <= 2 ? 2 : 4;
     return pb;
 }
 

@@ -168,6 +168,11 @@ struct DevPlan {
     // G = sum_p coefficient_p X_p over the powers p of the block's moment products
     const double* ang_coef;
     const int* ang_index;
+    // models in the domain of powers.hpp (pow_ne = 2 or 4 exponents per block, 0 for the others): for centre
+    // species t and item (block, exponent e < pow_ne, level) the function's index within the block, or -1
+    // (device array, set by the engine)
+    int pow_ne;
+    const int* pow_index;
 };
 
 struct PlanBuffers {

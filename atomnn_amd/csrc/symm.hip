@@ -32,6 +32,7 @@
 #include "model.hpp"
 #include "basis.hpp"
 #include "moments.hpp"
+#include "powers.hpp"
 
 namespace atomnn {
 
@@ -330,14 +331,13 @@ __device__ __forceinline__ double4 load_x4<float>(const float* src) {
 }
 
 // ------------------------------------------------------------------ per-atom bodies
-// Descriptors of one staged centre into Grow (LDS, zeroed by the caller).
-template <typename T, int NE, int NC, bool GEN>
-__device__ __forceinline__ void symm_body(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
-                                          const double* __restrict__ rfun_rs, int ti, int ntypes, int P, int maxp,
-                                          const T* su, T* Rf, T* red, int red_elems, T* Grow, const Segs& sg,
-                                          T* nsx, T* mom, int lane, T* mom_out = nullptr) {
-    // radial: cutoff once per neighbour, then (function, part) items over 64 lanes; the parts of
-    // a function are summed in a fixed order
+// Radial descriptors of one staged centre into Grow.  Rf and red are scratch (a value per entry, one per lane).
+template <typename T, bool GEN>
+__device__ __forceinline__ void symm_radial(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
+                                            const double* __restrict__ rfun_rs, int ti, int ntypes, const T* su,
+                                            T* Rf, T* red, T* Grow, const Segs& sg, int lane) {
+    // once per neighbour, then (function, part) items over 64 lanes; the parts of a function
+    // are summed in a fixed order
     {
         T* fcr = Rf;    // [maxp] cutoff values (Rf is free until the angular blocks)
         T* part = red;  // [64] partial sums
@@ -389,6 +389,15 @@ __device__ __forceinline__ void symm_body(const DevPlan* __restrict__ plan, cons
             __syncthreads();
         }
     }
+}
+
+// Descriptors of one staged centre into Grow (LDS, zeroed by the caller).
+template <typename T, int NE, int NC, bool GEN>
+__device__ __forceinline__ void symm_body(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
+                                          const double* __restrict__ rfun_rs, int ti, int ntypes, int P, int maxp,
+                                          const T* su, T* Rf, T* red, int red_elems, T* Grow, const Segs& sg,
+                                          T* nsx, T* mom, int lane, T* mom_out = nullptr) {
+    symm_radial<T, GEN>(plan, rfun_eta, rfun_rs, ti, ntypes, su, Rf, red, Grow, sg, lane);
 
     // angular blocks: moment expansion when the centre species allows it
     if (mom && plan->mom_ok[ti]) {
@@ -1463,6 +1472,152 @@ static hipError_t launch_force_mom_t(const DevPlan* plan, const double* rfe, con
                        rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, dEdG, ldg, X, Min);
     return hipGetLastError();
 }
+
+// ------------------------------------------------------------------ models with zeta up to 16
+// Descriptor and force kernels of the models whose every angular block is in the domain of powers.hpp (and not
+// all in the moment expansion's): one wavefront per centre.  Such models took the generic (8, 8) kernels: an
+// 8 x 8 grid of accumulators for a few exponents and terms, each term by selects, at one wavefront per SIMD.
+// Bound by VALU instructions (FP64 products of the pairs).  1500 atoms, 2 species, 2 exponents, zeta 1, 2, 4,
+// 16, P = 45: descriptors 160 -> 23.5 us, force terms 282 -> 27.4 us.
+template <typename T, int NE>
+__host__ __device__ constexpr size_t symm_pow_lds_bytes(int lmaxp, int ldg) {
+    return sizeof(T) * (size_t)(4 * lmaxp + NE * lmaxp + pow_red_elems() + ((ldg + 1) & ~1));
+}
+template <typename T, int NE>
+__host__ __device__ constexpr size_t force_pow_lds_bytes(int lmaxp, int ldg, int ntypes) {
+    return sizeof(T) * (size_t)(4 * lmaxp + 2 * NE * lmaxp + ((ldg + 1) & ~1) + pow_weight_elems<NE>(ntypes)) +
+           sizeof(int) * (size_t)lmaxp;
+}
+
+template <typename T, int NE>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(NE <= 2 ? 4 : 2, 8))) void k_symm_pow(
+    const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta, const double* __restrict__ rfun_rs,
+    const int* __restrict__ atom_type, const int* __restrict__ centres, int ncentres, const int* __restrict__ cnt,
+    const int* __restrict__ nbr_meta, const double4* __restrict__ nbr_r, int maxp, int lmaxp, T* __restrict__ G,
+    int ldg) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    T* su = (T*)lds_raw;
+    T* Rf = su + 4 * lmaxp;
+    T* red = Rf + NE * lmaxp;
+    T* Grow = red + pow_red_elems();
+    const int slot = xcd_slot(ncentres);  // the XCD-local order of the neighbour kernel
+    if (slot < 0) return;
+    const int i = centres[slot];
+    const int lane = threadIdx.x;
+    const int ti = atom_type[i];
+    const int P = min(cnt[i], lmaxp);
+    const int ntypes = plan->T;
+    __shared__ int seg_lds[kMaxSpecies + 1];
+    Segs sg{seg_lds};
+    stage_entries<T>(i, P, maxp, ntypes, nbr_meta, nbr_r, su, nullptr, sg, lane);
+    for (int k = lane; k < ldg; k += kWave) Grow[k] = T(0);
+    __syncthreads();
+    symm_radial<T, false>(plan, rfun_eta, rfun_rs, ti, ntypes, su, Rf, red, Grow, sg, lane);
+    radial_tables<T, NE, false>(plan->ang[ti][0], su, 0, P, Rf, nullptr, lane);
+    __syncthreads();
+    symm_angular_powers<T, NE>(plan, ti, ntypes, su, Rf, sg.start, red, Grow, lane);
+    for (int k = lane; k < ldg; k += kWave) G[(int64_t)i * ldg + k] = Grow[k];
+}
+
+template <typename T, int NE>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(NE <= 2 && sizeof(T) == 4 ? 4 : 2, 8))) void k_force_pow(
+    const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta, const double* __restrict__ rfun_rs,
+    const int* __restrict__ atom_type, const int* __restrict__ centres, int ncentres, const int* __restrict__ cnt,
+    const int* __restrict__ nbr_meta, const double4* __restrict__ nbr_r, int maxp, int lmaxp,
+    const T* __restrict__ dEdG, int ldg, T* __restrict__ Xout) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int ntypes = plan->T;
+    T* su = (T*)lds_raw;
+    T* Rf = su + 4 * lmaxp;
+    T* Rd = Rf + NE * lmaxp;
+    T* W = Rd + NE * lmaxp;
+    T* wtab = W + ((ldg + 1) & ~1);
+    int* orig = (int*)(wtab + pow_weight_elems<NE>(ntypes));
+    const int slot = xcd_slot(ncentres);  // the XCD-local order of the neighbour kernel
+    if (slot < 0) return;
+    const int i = centres[slot];
+    const int lane = threadIdx.x;
+    const int ti = atom_type[i];
+    const int P = min(cnt[i], lmaxp);
+    __shared__ int seg_lds[kMaxSpecies + 1];
+    Segs sg{seg_lds};
+    stage_entries<T>(i, P, maxp, ntypes, nbr_meta, nbr_r, su, orig, sg, lane);
+    for (int k = lane; k < ldg; k += kWave) W[k] = dEdG[(int64_t)i * ldg + k];
+    __syncthreads();
+    pow_weights<T, NE>(plan, ti, ntypes, W, wtab, lane);
+    radial_tables<T, NE, false>(plan->ang[ti][0], su, 0, P, Rf, Rd, lane);
+    __syncthreads();
+    const int64_t row = (int64_t)i * maxp;
+    for (int p = lane; p < P; p += kWave) {
+        int s = 0;
+        while (s + 1 < ntypes && p >= sg.start[s + 1]) ++s;
+        const DevRadial& R = plan->rad[ti][s];
+        const T d = su[4 * p + 3];
+        T fc, gc;
+        cutoff_fg<T>(R.cut, d, T(R.rc), T(R.rci), T(R.pirci), fc, gc);
+        T sr = T(0);
+        for (int f = 0; f < R.n; ++f) {
+            const T eta = T(rfun_eta[R.fbase + f]), rs = T(rfun_rs[R.fbase + f]);
+            const T x = d - rs;
+            sr += W[R.goff + f] * kexp(-eta * x * x) * (T(-2) * eta * x * fc + gc);
+        }
+        sr *= T(R.norm);
+        T gx = sr * su[4 * p], gy = sr * su[4 * p + 1], gz = sr * su[4 * p + 2];
+        force_powers_entry<T, NE>(ntypes, su, Rf, Rd, sg.start, wtab, p, s, gx, gy, gz);
+        store_x4<T>(Xout + 4 * (row + orig[p]), -gx, -gy, -gz);
+    }
+}
+
+size_t symm_pow_lds(int ne, bool fp64, int lmaxp, int ldg) {
+    if (ne <= 2) return fp64 ? symm_pow_lds_bytes<double, 2>(lmaxp, ldg) : symm_pow_lds_bytes<float, 2>(lmaxp, ldg);
+    return fp64 ? symm_pow_lds_bytes<double, 4>(lmaxp, ldg) : symm_pow_lds_bytes<float, 4>(lmaxp, ldg);
+}
+size_t force_pow_lds(int ne, bool fp64, int lmaxp, int ldg, int ntypes) {
+    if (ne <= 2)
+        return fp64 ? force_pow_lds_bytes<double, 2>(lmaxp, ldg, ntypes) : force_pow_lds_bytes<float, 2>(lmaxp, ldg, ntypes);
+    return fp64 ? force_pow_lds_bytes<double, 4>(lmaxp, ldg, ntypes) : force_pow_lds_bytes<float, 4>(lmaxp, ldg, ntypes);
+}
+
+template <typename T>
+hipError_t launch_symm_pow(int ne, const DevPlan* plan, const double* rfe, const double* rfr, const int* atom_type,
+                           const int* centres, int ncentres, const int* cnt, const int* meta, const double4* r, int maxp,
+                           int lmaxp, T* G, int ldg, hipStream_t st) {
+    const size_t lds = symm_pow_lds(ne, sizeof(T) == 8, lmaxp, ldg);
+    if (lds > 65536) return hipErrorInvalidConfiguration;
+    const dim3 grid(xcd_grid(ncentres)), block(kWave);
+    if (ne <= 2)
+        hipLaunchKernelGGL((k_symm_pow<T, 2>), grid, block, lds, st, plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta,
+                           r, maxp, lmaxp, G, ldg);
+    else
+        hipLaunchKernelGGL((k_symm_pow<T, 4>), grid, block, lds, st, plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta,
+                           r, maxp, lmaxp, G, ldg);
+    return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_force_pow(int ne, const DevPlan* plan, const double* rfe, const double* rfr, const int* atom_type,
+                            const int* centres, int ncentres, const int* cnt, const int* meta, const double4* r, int maxp,
+                            int lmaxp, const T* dEdG, int ldg, T* X, int ntypes, hipStream_t st) {
+    const size_t lds = force_pow_lds(ne, sizeof(T) == 8, lmaxp, ldg, ntypes);
+    if (lds > 65536) return hipErrorInvalidConfiguration;
+    const dim3 grid(xcd_grid(ncentres)), block(kWave);
+    if (ne <= 2)
+        hipLaunchKernelGGL((k_force_pow<T, 2>), grid, block, lds, st, plan, rfe, rfr, atom_type, centres, ncentres, cnt,
+                           meta, r, maxp, lmaxp, dEdG, ldg, X);
+    else
+        hipLaunchKernelGGL((k_force_pow<T, 4>), grid, block, lds, st, plan, rfe, rfr, atom_type, centres, ncentres, cnt,
+                           meta, r, maxp, lmaxp, dEdG, ldg, X);
+    return hipGetLastError();
+}
+template hipError_t launch_symm_pow<double>(int, const DevPlan*, const double*, const double*, const int*, const int*, int,
+                                            const int*, const int*, const double4*, int, int, double*, int, hipStream_t);
+template hipError_t launch_symm_pow<float>(int, const DevPlan*, const double*, const double*, const int*, const int*, int,
+                                           const int*, const int*, const double4*, int, int, float*, int, hipStream_t);
+template hipError_t launch_force_pow<double>(int, const DevPlan*, const double*, const double*, const int*, const int*,
+                                             int, const int*, const int*, const double4*, int, int, const double*, int,
+                                             double*, int, hipStream_t);
+template hipError_t launch_force_pow<float>(int, const DevPlan*, const double*, const double*, const int*, const int*, int,
+                                            const int*, const int*, const double4*, int, int, const float*, int, float*,
+                                            int, hipStream_t);
 
 template <typename T, int NE, int NC, bool GEN>
 __host__ __device__ constexpr size_t fused_lds_bytes(int maxp, int ldg, int maxw, int dersum) {
