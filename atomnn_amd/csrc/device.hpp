@@ -10,6 +10,7 @@
 //     nbr_j    int32 [Ntot*maxp]    neighbour atom (index inside its structure)
 //     nbr_meta int32 [Ntot*maxp]    image << 8 | species << 1 | min-image flag
 //     nbr_r    double4[Ntot*maxp]   (r_i - r_j - T, |r|): points from neighbour to centre
+//   row_tab    uint16[Ntot][32]     index table of each row
 //   G          T[Ntot][ldg]          descriptors, dEdG same shape
 //   X          TX4[Ntot*maxp]       per-entry force term  -dE_i/dr_ij
 #pragma once
@@ -52,6 +53,12 @@ __device__ __forceinline__ int xcd_slot(int n) {
 }
 inline int xcd_grid(int n) { return kXcds * ((n + kXcds - 1) / kXcds); }
 
+// Index table of a neighbour row (rows ascend in the neighbour's index): entry q < kRowTab is the number of row
+// entries with an index below q row_tab_width(natoms), so the entries of one neighbour are found in a stretch of
+// P / 32 entries without a search.  Written with the rows, read by the force assembly.
+constexpr int kRowTab = 32;
+__host__ __device__ __forceinline__ int row_tab_width(int natoms) { return (natoms + kRowTab - 1) / kRowTab; }
+
 // Force assembly (k_assemble).  react points at two per-pass counters beside the neighbour
 // maximum: react[0] = reactions the gather from the neighbours' rows missed (mode 0; cleared by
 // the neighbour launch), react[1] = longest receiver row (mode 1; cleared by that mode's own
@@ -70,6 +77,7 @@ struct AssembleArgs {
     const int* cnt;
     const int* nbr_j;
     const int* meta;
+    const unsigned short* row_tab;
     int maxp;
     int ntot;
     int all_images;
@@ -100,16 +108,24 @@ struct EnergyTail {
     int* maxcnt;
 };
 
-// Block b of the tail (one wavefront).  Energy: lane t sums its contiguous chunk of the
-// structure's E_i in order, then a fixed shuffle tree; the sum depends only on that structure's
-// E_i, so batch and single passes agree bit for bit.  Count: strided slices, one atomicMax each.
+// Block b of the tail (one wavefront).  Energy: lane t sums the E_i t, t + 64, ... of its structure in four
+// interleaved chains (coalesced loads, sixteen in flight), then a fixed shuffle tree; the sum depends only on
+// that structure's E_i, so batch and single passes agree bit for bit.  Count: strided slices, one atomicMax
+// each.
 __device__ __forceinline__ void energy_tail_block(const EnergyTail& t, int b, int lane) {
     if (b < t.nstruc) {
         const int a0 = t.sstart[b], a1 = t.sstart[b + 1];
-        const int n = a1 - a0, chunk = (n + kWave - 1) / kWave;
-        const int i0 = a0 + lane * chunk, i1 = a0 + min(n, (lane + 1) * chunk);
-        double acc = 0.0;
-        for (int i = i0; i < i1; ++i) acc += t.eatom[i];
+        double c[4] = {0.0, 0.0, 0.0, 0.0};
+        int i = a0 + lane;
+        for (; i + 15 * kWave < a1; i += 16 * kWave) {
+            double v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[k] = t.eatom[i + k * kWave];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) c[k & 3] += v[k];
+        }
+        for (; i < a1; i += kWave) c[0] += t.eatom[i];
+        double acc = (c[0] + c[1]) + (c[2] + c[3]);
 #pragma unroll
         for (int o = kWave / 2; o > 0; o >>= 1) acc += __shfl_down(acc, o);
         if (lane == 0) t.E[b] = acc;

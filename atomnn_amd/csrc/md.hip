@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kWave) void k_md_refresh(const DevStruc* __restrict
                                                      int built, double rc2, double half_skin2,
                                                      int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                      int* __restrict__ nbr_meta, double4* __restrict__ nbr_r, int maxp,
-                                                     int* __restrict__ maxcnt, const int* __restrict__ list_maxcnt,
+                                                     unsigned short* __restrict__ row_tab, int* __restrict__ maxcnt, const int* __restrict__ list_maxcnt,
                                                      int* __restrict__ maxseen) {
     extern __shared__ __align__(8) unsigned char md_lds[];
     double* dk = (double*)md_lds;          // [maxp] kept distances
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kWave) void k_md_refresh(const DevStruc* __restrict
     }
     __syncthreads();
     // min flags over the kept entries (runs of one neighbour are contiguous)
-    const int K = min(kept, maxp);
+    const int K = min(kept, maxp), tw = row_tab_width(s.natoms);
     for (int k = lane; k < K; k += kWave) {
         const int j = jk[k];
         const double d = dk[k];
@@ -234,7 +234,10 @@ __global__ __launch_bounds__(kWave) void k_md_refresh(const DevStruc* __restrict
         for (int q = k - 1; mn && q >= 0 && jk[q] == j; --q) mn = dk[q] > d;
         for (int q = k + 1; mn && q < K && jk[q] == j; ++q) mn = dk[q] >= d;
         nbr_meta[row + k] = mk[k] | (mn ? 1 : 0);
+        // the row's index table: an entry opens the slots after its predecessor's up to its own
+        for (int q = k > 0 ? jk[k - 1] / tw + 1 : 0; q <= j / tw; ++q) row_tab[(int64_t)i * kRowTab + q] = (unsigned short)k;
     }
+    if (lane < kRowTab && lane >= (K > 0 ? jk[K - 1] / tw + 1 : 0)) row_tab[(int64_t)i * kRowTab + lane] = (unsigned short)K;
     if (lane == 0) cnt[i] = kept;
 }
 
@@ -307,7 +310,7 @@ struct Md {
                            (const int*)L.d_meta.p, (const double4*)L.d_nbrr.p, L.maxp, (double4*)d_T.p,
                            (double*)d_xb.p, built, E.host.rc * E.host.rc, half * half * (1.0 - 1e-9),
                            (int*)E.d_cnt.p, (int*)E.d_nbrj.p, (int*)E.d_meta.p, (double4*)E.d_nbrr.p, E.maxp,
-                           (int*)E.d_maxcnt.p, (const int*)L.d_maxcnt.p, (int*)d_maxseen.p);
+                           (unsigned short*)E.d_rowtab.p, (int*)E.d_maxcnt.p, (const int*)L.d_maxcnt.p, (int*)d_maxseen.p);
         HIPCHK(hipGetLastError());
     }
 

@@ -89,6 +89,18 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
     return x - v;
 }
 
+// Index table of row i from its ascending entries in LDS or registers' order: entry p with neighbour index j opens
+// every table slot after its predecessor's (index jp, -1 for the first entry) up to its own.
+__device__ __forceinline__ void row_tab_open(unsigned short* tab, int width, int jp, int j, int p) {
+    const int q0 = jp < 0 ? 0 : jp / width + 1, q1 = j / width;
+    for (int q = q0; q <= q1; ++q) tab[q] = (unsigned short)p;
+}
+// the slots after the last entry (index j, -1 in an empty row) of a row of P entries
+__device__ __forceinline__ void row_tab_close(unsigned short* tab, int width, int j, int P, int lane) {
+    const int q0 = j < 0 ? 0 : j / width + 1;
+    if (lane >= q0 && lane < kRowTab) tab[lane] = (unsigned short)P;
+}
+
 __device__ __forceinline__ void put_entry(int64_t slot, int j, int img, int typ, bool mn, double x, double y, double z,
                                           double d, int* nbr_j, int* nbr_meta, double4* nbr_r) {
     nbr_j[slot] = j;
@@ -146,7 +158,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
                                                           const int* __restrict__ centres, double rc2, int maxp,
                                                           int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                           int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                          PassCounters pc) {
+                                                          unsigned short* __restrict__ row_tab, PassCounters pc) {
     clear_counters(pc);
     const int i = centres[blockIdx.x];
     const DevStruc& s = S[atom_struc[i]];
@@ -154,6 +166,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
     const int li = i - s.atom0;
     const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
     const int64_t row = (int64_t)i * maxp;
+    const int tw = row_tab_width(s.natoms);
     int written = 0;
     for (int j0 = 0; j0 < s.natoms; j0 += kWave) {
         const int j = j0 + lane;
@@ -199,6 +212,8 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
                 }
         int tot;
         int at = written + wave_excl_scan(mine, lane, tot);
+        // the row's index table: atom j opens slot j / width when it is the slot's first
+        if (valid && j % tw == 0) row_tab[(int64_t)i * kRowTab + j / tw] = (unsigned short)min(at, maxp);
         if (mine > 0) {
             for (int a = g.lo[0]; a <= g.hi[0]; ++a)
                 for (int b = g.lo[1]; b <= g.hi[1]; ++b)
@@ -218,6 +233,8 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
         }
         written += tot;
     }
+    const int q0 = (s.natoms + tw - 1) / tw;  // slots past the last atom
+    if (lane >= q0 && lane < kRowTab) row_tab[(int64_t)i * kRowTab + lane] = (unsigned short)min(written, maxp);
     if (lane == 0) {
         cnt[i] = written;
     }
@@ -447,7 +464,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
                                                        const int* __restrict__ bin_atoms, double rc2, int maxp, int n2cap,
                                                        int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                        int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                       PassCounters pc) {
+                                                       unsigned short* __restrict__ row_tab, PassCounters pc) {
     extern __shared__ double lds_cells[];
     clear_counters(pc);
     const int cap = maxp;
@@ -541,7 +558,9 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
         // one image per j: it is the minimum image when below ||R||_F (neighbor.cpp:132-140)
         put_entry(row + q, j, 0, type[s.atom0 + j], d < s.fro, vals[4 * src], vals[4 * src + 1], vals[4 * src + 2], d,
                   nbr_j, nbr_meta, nbr_r);
+        row_tab_open(row_tab + (int64_t)i * kRowTab, row_tab_width(s.natoms), q > 0 ? skey[q - 1] : -1, j, q);
     }
+    row_tab_close(row_tab + (int64_t)i * kRowTab, row_tab_width(s.natoms), P > 0 ? skey[P - 1] : -1, P, lane);
     if (lane == 0) {
         cnt[i] = kept;
     }
@@ -581,7 +600,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
     const int* __restrict__ type, int ncell, const int* __restrict__ atom_bin,
     const int* __restrict__ bin_start, const float4* __restrict__ bin_pos, int one_struc, double rc2, int maxp,
     int* __restrict__ cnt, int* __restrict__ nbr_j, int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-    int nwords_max, PassCounters pc) {
+    unsigned short* __restrict__ row_tab, int nwords_max, PassCounters pc) {
     extern __shared__ unsigned int lds_bits[];
     clear_counters(pc);
     unsigned short* pre = reinterpret_cast<unsigned short*>(lds_bits + nwords_max);
@@ -722,6 +741,11 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
         __syncthreads();
         put(e0);
         if (nlist > kWave) put(e1);
+        if (lane < kRowTab) {  // the row's index table: set bits before each slot's first atom
+            const int j = lane * row_tab_width(s.natoms), w = j >> 5;
+            const int p = j < s.natoms ? pre[w] + __popc(lds_bits[w] & ((1u << (j & 31)) - 1u)) : kept;
+            row_tab[(int64_t)i * kRowTab + lane] = (unsigned short)min(p, maxp);
+        }
         if (lane == 0) cnt[i] = kept;
         return;
     }
@@ -745,8 +769,13 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
     for (int w = w0; w < w1; ++w) mine += __popc(lds_bits[w]);
     int kept;
     int at = wave_excl_scan(mine, lane, kept);
+    const int tw = row_tab_width(s.natoms);
     for (int w = w0; w < w1; ++w) {
         unsigned int m = lds_bits[w];
+        // slots of the row's index table whose first atom is among this word's 32 (the bits before it)
+        for (int q = ((w << 5) + tw - 1) / tw; q < kRowTab && q * tw < (w << 5) + 32; ++q)
+            row_tab[(int64_t)i * kRowTab + q] =
+                (unsigned short)min(at + __popc(m & ((1u << (q * tw - (w << 5))) - 1u)), maxp);
         while (m) {
             const int bit = __ffs(m) - 1;
             m &= m - 1;
@@ -760,6 +789,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
             ++at;
         }
     }
+    if (lane < kRowTab && lane * tw >= nwords * 32) row_tab[(int64_t)i * kRowTab + lane] = (unsigned short)min(kept, maxp);
     if (lane == 0) cnt[i] = kept;
 }
 
@@ -812,20 +842,20 @@ hipError_t launch_neighbors(const NeighborArgs& a, hipStream_t st) {
             hipLaunchKernelGGL(k_neigh_cells_bits, dim3(xcd_grid(a.ncell)), dim3(kWave),
                                bits_lds + (bits_lds / 2 + 3) / 4 * 4, st, a.S, a.atom_struc, a.pos, a.type, a.ncell,
                                a.atom_bin, a.bin_start, a.bin_pos, a.nstruc == 1, a.rc2, a.maxp, a.cnt, a.nbr_j,
-                               a.nbr_meta, a.nbr_r, (int)(bits_lds / 4), pc);
+                               a.nbr_meta, a.nbr_r, a.row_tab, (int)(bits_lds / 4), pc);
         } else {  // very large structures: sort the kept candidates instead
             int n2cap = 1;
             while (n2cap < a.maxp) n2cap <<= 1;
             const size_t lds = (size_t)a.maxp * 32 + (size_t)a.maxp * 4 + (size_t)n2cap * 8;
             hipLaunchKernelGGL(k_neigh_cells, dim3(a.ncell), dim3(kWave), lds, st, a.S, a.atom_struc, a.pos, a.type,
                                a.cell_centres, a.atom_bin, a.bin_start, a.bin_atoms, a.rc2, a.maxp, n2cap, a.cnt,
-                               a.nbr_j, a.nbr_meta, a.nbr_r, pc);
+                               a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, pc);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.npair > 0) {
         hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave), 0, st, a.S, a.atom_struc, a.pos, a.type,
-                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, pc);
+                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, pc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.ntot > 0 && a.count_max) return launch_count_max(a.cnt, a.ntot, a.maxcnt, st);

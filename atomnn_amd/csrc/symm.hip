@@ -1770,8 +1770,8 @@ template hipError_t launch_fused<float>(int, int, int, const DevPlan*, const dou
 // when that entry, in centre i's own row, carries the min flag (every entry with all_images).
 // One wavefront per atom a, lanes over its own entries.  The reactions are gathered from the
 // rows of a's neighbours: for the first entry of each neighbour j in a's row (rows are sorted by
-// neighbour index, then image), the run of entries with index a in j's row is located (lower
-// bound of a) and every entry of that run that carries a reaction is subtracted.  No image
+// neighbour index, then image), the run of entries with index a in j's row is located (through the row's
+// index table) and every entry of that run that carries a reaction is subtracted.  No image
 // correspondence is assumed, so images that tie in distance (half-lattice offsets, where both
 // differences wrap to -1/2) take exactly the entries the reference takes.
 //
@@ -1790,6 +1790,11 @@ template hipError_t launch_fused<float>(int, int, int, const DevPlan*, const dou
 //
 // Lane partials are summed in a fixed tree order (deterministic, no atomics on F).
 //
+// Bound by its chain of dependent look-ups (a's row, the neighbour's table, the stretch of its row, the
+// term).  With a guess at the position and an 8-ary search where it missed (some lane of every wavefront did) the
+// launch took 13.9 us on 4096 atoms, 31 us on 11003 and 155 us on 16 x 4096 (FP32 terms); with the index table
+// 8.8, 25 and 130 us.
+//
 // Block order: workgroups are dealt to the 8 XCDs round-robin, each XCD with its own L2.  Block b
 // (after the tail blocks, padded to a multiple of 8) takes position (b mod 8) * chunk + b / 8 of the
 // processing order (cell-list atoms by bin, then the rest), so the blocks an XCD runs at any time
@@ -1807,55 +1812,12 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
-// First index in [0, P) of row `rowj` whose neighbour index is >= want (P if none).  The row's
-// indices ascend, so the entry sits near want / natoms of the way along it: the 16 indices around
-// that guess come in four aligned 16-byte loads and, when they bracket want, their count places
-// it; otherwise an 8-ary search (7 independent probes per level, a short dependent chain) takes
-// the side that holds it and the last <= 16 indices are counted.
-__device__ __forceinline__ int row_lower_bound(const int* __restrict__ nbr_j, int64_t rowj, int P, int want,
-                                               int natoms) {
-    int lo = 0, hi = P;
-    if (P >= 16) {
-        const int g = (int)(((int64_t)want * P) / max(natoms, 1));
-        const int w0 = min(max(0, g - 8), P - 16) & ~3;  // 4-aligned, and w0 + 16 <= P
-        const int4* kv = reinterpret_cast<const int4*>(nbr_j + rowj + w0);
-        int c = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int4 k4 = kv[q];
-            c += (k4.x < want) + (k4.y < want) + (k4.z < want) + (k4.w < want);
-        }
-        const int w1 = w0 + 16;
-        if (c > 0 && (c < 16 || w1 == P)) {
-            lo = hi = w0 + c;
-        } else if (c == 0) {
-            hi = w0;
-        } else {
-            lo = w1;
-        }
-    }
-    while (hi - lo > 16) {
-        const int len = hi - lo;
-        int c = 0;
-#pragma unroll
-        for (int m = 1; m < 8; ++m) c += nbr_j[rowj + lo + (len * m) / 8] < want ? 1 : 0;
-        const int nlo = c == 0 ? lo : lo + (len * c) / 8 + 1;
-        const int nhi = c == 7 ? hi : lo + (len * (c + 1)) / 8;
-        lo = nlo;
-        hi = nhi;
-    }
-    int c = 0;
-#pragma unroll
-    for (int m = 0; m < 16; ++m) c += (lo + m < hi && nbr_j[rowj + lo + m] < want) ? 1 : 0;
-    return lo + c;
-}
-
-
 template <typename T, int MODE>
 __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                     const int* __restrict__ cnt, const int* __restrict__ nbr_j,
-                                                    const int* __restrict__ nbr_meta, const T* __restrict__ X, int maxp,
-                                                    int all_images, double* __restrict__ F, EnergyTail tail,
+                                                    const int* __restrict__ nbr_meta,
+                                                    const unsigned short* __restrict__ row_tab, const T* __restrict__ X,
+                                                    int maxp, int all_images, double* __restrict__ F, EnergyTail tail,
                                                     int* __restrict__ react, const int* __restrict__ rcount,
                                                     const int* __restrict__ rlist, int rcap,
                                                     const int* __restrict__ bin_atoms,
@@ -1880,27 +1842,47 @@ __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__
     if (MODE == 0) {
         const DevStruc& st = S[atom_struc[a]];
         const int la = a - st.atom0;
+        const int slot = la / row_tab_width(st.natoms);  // the table slot of this atom in every row
         int own = 0, used = 0;
         for (int s = lane; s < P; s += kWave) {
             const int64_t e = row + s;
+            const int j = nbr_j[e];
+            own += (all_images || (nbr_meta[e] & 1)) ? 1 : 0;
+            // one lane per neighbour: the first of its entries.  Self entries carry no min flag
+            // (neighbor.cpp:131), so under the min-image rule the atom's own row is skipped.
+            const bool first = (s == 0 || nbr_j[e - 1] != j) && (all_images || j != la);
+            const int gj = st.atom0 + j;
+            const int64_t rowj = (int64_t)gj * maxp;
+            int q0 = 0, q1 = 0;
+            if (first) {
+                const unsigned short* tab = row_tab + (int64_t)gj * kRowTab + slot;
+                q0 = tab[0];
+                q1 = slot + 1 < kRowTab ? tab[1] : min(cnt[gj], maxp);
+            }
             {
                 const double4 v = load_x4<T>(X + 4 * e);
                 fx += v.x;
                 fy += v.y;
                 fz += v.z;
             }
-            const int j = nbr_j[e];
-            own += (all_images || (nbr_meta[e] & 1)) ? 1 : 0;
-            // one lane per neighbour: the first of its entries.  Self entries carry no min flag
-            // (neighbor.cpp:131), so under the min-image rule the atom's own row is skipped.
-            const bool first = s == 0 || nbr_j[e - 1] != j;
-            if (first && (all_images || j != la)) {
-                const int gj = st.atom0 + j;
-                const int64_t rowj = (int64_t)gj * maxp;
-                const int Pj = min(cnt[gj], maxp);
-                for (int q = row_lower_bound(nbr_j, rowj, Pj, la, st.natoms); q < Pj && nbr_j[rowj + q] == la; ++q) {
-                    if (all_images || (nbr_meta[rowj + q] & 1)) {
-                        const double4 v = load_x4<T>(X + 4 * (rowj + q));
+            // the stretch [q0, q1) of j's row, twelve entries at a time by aligned 16-byte loads
+            for (int w = min(q0 & ~3, maxp - 12); w < q1; w += 12) {
+                const int wc = min(w, maxp - 12);
+                const int4* kv = reinterpret_cast<const int4*>(nbr_j + rowj + wc);
+                unsigned m = 0;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const int4 k4 = kv[k];
+                    m |= ((k4.x == la) | ((k4.y == la) << 1) | ((k4.z == la) << 2) | ((k4.w == la) << 3)) << (4 * k);
+                }
+                const int lo = max(q0, w) - wc, hi = min(q1 - wc, 12);
+                m &= (1u << hi) - (1u << lo);
+                while (m) {
+                    const int64_t f = rowj + wc + __ffs(m) - 1;
+                    m &= m - 1;
+                    const int meta = nbr_meta[f];
+                    const double4 v = load_x4<T>(X + 4 * f);
+                    if (all_images || (meta & 1)) {
                         fx -= v.x;
                         fy -= v.y;
                         fz -= v.z;
@@ -2148,8 +2130,8 @@ hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* 
     const dim3 grid(ntail_pad + kXcds * chunk);
     const int ncell = a.bin_atoms ? a.ncell : 0;
     if (a.mode == 0) {
-        hipLaunchKernelGGL((k_assemble<T, 0>), grid, dim3(kWave), 0, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta, X,
-                           a.maxp, a.all_images, a.F, t, a.react, nullptr, nullptr, 0, a.bin_atoms, a.pair_centres,
+        hipLaunchKernelGGL((k_assemble<T, 0>), grid, dim3(kWave), 0, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta,
+                           a.row_tab, X, a.maxp, a.all_images, a.F, t, a.react, nullptr, nullptr, 0, a.bin_atoms, a.pair_centres,
                            ncell, a.ntot, chunk);
         return hipGetLastError();
     }
@@ -2158,7 +2140,7 @@ hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* 
     hipLaunchKernelGGL(k_react_zero, dim3((a.ntot + 255) / 256), dim3(256), 0, st, a.rcount, a.ntot, a.react);
     hipLaunchKernelGGL(k_react_fill, dim3(a.ntot), dim3(kWave), 0, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta,
                        a.maxp, a.all_images, a.rcount, a.rlist, a.rcap);
-    hipLaunchKernelGGL((k_assemble<T, 1>), grid, dim3(kWave), lds, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta, X,
+    hipLaunchKernelGGL((k_assemble<T, 1>), grid, dim3(kWave), lds, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta, a.row_tab, X,
                        a.maxp, a.all_images, a.F, t, a.react, a.rcount, a.rlist, a.rcap, a.bin_atoms, a.pair_centres,
                        ncell, a.ntot, chunk);
     return hipGetLastError();
