@@ -10,6 +10,7 @@
 //     nbr_j    int32 [Ntot*maxp]    neighbour atom (index inside its structure)
 //     nbr_meta int32 [Ntot*maxp]    image << 8 | species << 1 | min-image flag
 //     nbr_r    double4[Ntot*maxp]   (r_i - r_j - T, |r|): points from neighbour to centre
+//   nbr_key    uint16[Ntot*maxp]    low 16 bits of nbr_j
 //   row_tab    uint16[Ntot][32]     index table of each row
 //   G          T[Ntot][ldg]          descriptors, dEdG same shape
 //   X          TX4[Ntot*maxp]       per-entry force term  -dE_i/dr_ij
@@ -54,10 +55,13 @@ __device__ __forceinline__ int xcd_slot(int n) {
 inline int xcd_grid(int n) { return kXcds * ((n + kXcds - 1) / kXcds); }
 
 // Index table of a neighbour row (rows ascend in the neighbour's index): entry q < kRowTab is the number of row
-// entries with an index below q row_tab_width(natoms), so the entries of one neighbour are found in a stretch of
-// P / 32 entries without a search.  Written with the rows, read by the force assembly.
+// entries with an index below q w, w = row_tab_width(natoms), the last one all of them, so the entries of one
+// neighbour are found between two table entries, a stretch of some P / 31, without a search.  Beside it the row's
+// keys: the low 16 bits of each entry's index, which tell the indices of a stretch apart up to w = 65536
+// (2 M atoms).  Written with the rows, read by the force assembly.
 constexpr int kRowTab = 32;
-__host__ __device__ __forceinline__ int row_tab_width(int natoms) { return (natoms + kRowTab - 1) / kRowTab; }
+constexpr int kKeyWidth = 65536;
+__host__ __device__ __forceinline__ int row_tab_width(int natoms) { return (natoms + kRowTab - 2) / (kRowTab - 1); }
 
 // Force assembly (k_assemble).  react points at two per-pass counters beside the neighbour
 // maximum: react[0] = reactions the gather from the neighbours' rows missed (mode 0; cleared by
@@ -78,6 +82,7 @@ struct AssembleArgs {
     const int* nbr_j;
     const int* meta;
     const unsigned short* row_tab;
+    const unsigned short* nbr_key;
     int maxp;
     int ntot;
     int all_images;

@@ -417,7 +417,7 @@ Engine::Engine(const Engine& o, int) : host(o.host), pb(o.pb), shape(o.shape) {
 size_t Engine::workspace_bytes() const {
     size_t b = 0;
     for (const DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
-                            &d_brank, &d_bpos, &d_rowtab, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount,
+                            &d_brank, &d_bpos, &d_rowtab, &d_key, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount,
                             &d_rlist, &d_out, &d_mom})
         b += m->cap;
     return b;
@@ -436,7 +436,7 @@ Engine::~Engine() {
         for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi, &d_powi})
             m->release();
     for (DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
-                      &d_brank, &d_bpos, &d_rowtab, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})
+                      &d_brank, &d_bpos, &d_rowtab, &d_key, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})
         m->release();
     h_up.release();
     h_down.release();
@@ -673,7 +673,10 @@ void Engine::bind_scratch(void* base, size_t bytes, const nnp_structure& s) {
     d_brank.bind((char*)d_X.p + N * sizeof(float4), N * 4);
     HIPCHK(hipMemsetAsync(d_bcount.p, 0, nb * 4, stream));
     take(d_rlist, N * fit * 4);
-    d_rowtab.bind(d_rlist.p, N * kRowTab * sizeof(unsigned short));  // receiver rows never read the table
+    // the rows' index tables (64 bytes) and keys (2 bytes a slot, of 32 slots at least) in the place of the receiver
+    // rows, whose mode reads neither
+    d_rowtab.bind(d_rlist.p, N * kRowTab * sizeof(unsigned short));
+    d_key.bind((char*)d_rlist.p + N * kRowTab * sizeof(unsigned short), N * fit * sizeof(unsigned short));
     HIPCHK(hipMemsetAsync(d_maxcnt.p, 0, 64, stream));  // counters the mode does not write read as zero
     maxp = 0;
     rcap = 0;
@@ -692,6 +695,7 @@ void Engine::build_neighbors(bool all_images) {
         d_meta.reserve(ent * 4);
         d_nbrr.reserve(ent * sizeof(double4));
         d_rowtab.reserve((size_t)ntot * kRowTab * sizeof(unsigned short));
+        d_key.reserve(ent * sizeof(unsigned short));
         if (!d_maxcnt.p) {  // counters the current mode does not write are read back as zero
             d_maxcnt.reserve(64);
             HIPCHK(hipMemsetAsync(d_maxcnt.p, 0, 64, stream));
@@ -890,6 +894,7 @@ void Engine::assemble(const EnergyTail* tail) {
     a.nbr_j = (const int*)d_nbrj.p;
     a.meta = (const int*)d_meta.p;
     a.row_tab = (const unsigned short*)d_rowtab.p;
+    a.nbr_key = (const unsigned short*)d_key.p;
     a.maxp = maxp;
     a.ntot = ntot;
     a.all_images = all_images_ ? 1 : 0;
@@ -1184,6 +1189,7 @@ NeighborArgs Engine::neighbor_args(bool all_images) const {
     a.nbr_meta = (int*)d_meta.p;
     a.nbr_r = (double4*)d_nbrr.p;
     a.row_tab = (unsigned short*)d_rowtab.p;
+    a.nbr_key = (unsigned short*)d_key.p;
     a.maxcnt = (int*)d_maxcnt.p;
     a.work = (int*)d_work.p;
     a.cell_centres = (const int*)d_centres.p;

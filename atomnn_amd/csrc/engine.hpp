@@ -83,6 +83,7 @@ struct NeighborArgs {
     int* nbr_meta;
     double4* nbr_r;
     unsigned short* row_tab;
+    unsigned short* nbr_key;
     int* maxcnt;
     int* work = nullptr;  // work counter of the fused persistent kernel (cleared with maxcnt)
     const int* cell_centres;
@@ -257,7 +258,7 @@ class Engine {
     DevMem d_up;
     HostPinned h_up, h_down;
     DevView d_pos, d_type, d_astruc, d_strucs, d_centres, d_spatoms;
-    DevMem d_cnt, d_nbrj, d_meta, d_nbrr, d_maxcnt, d_rowtab;
+    DevMem d_cnt, d_nbrj, d_meta, d_nbrr, d_maxcnt, d_rowtab, d_key;
     DevMem d_abin, d_bcount, d_bstart, d_brank, d_bpos;
     DevMem d_G, d_dEdG, d_X, d_eatom, d_F;
     // per-centre moment tables [S][NE][35] the moment-only descriptor kernel leaves for the

@@ -161,7 +161,8 @@ __global__ __launch_bounds__(kWave) void k_md_refresh(const DevStruc* __restrict
                                                      int built, double rc2, double half_skin2,
                                                      int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                      int* __restrict__ nbr_meta, double4* __restrict__ nbr_r, int maxp,
-                                                     unsigned short* __restrict__ row_tab, int* __restrict__ maxcnt, const int* __restrict__ list_maxcnt,
+                                                     unsigned short* __restrict__ row_tab,
+                                                     unsigned short* __restrict__ nbr_key, int* __restrict__ maxcnt, const int* __restrict__ list_maxcnt,
                                                      int* __restrict__ maxseen) {
     extern __shared__ __align__(8) unsigned char md_lds[];
     double* dk = (double*)md_lds;          // [maxp] kept distances
@@ -217,6 +218,7 @@ __global__ __launch_bounds__(kWave) void k_md_refresh(const DevStruc* __restrict
         if (keep && at < maxp) {
             const double d = sqrt(d2);
             nbr_j[row + at] = j;
+            nbr_key[row + at] = (unsigned short)j;
             nbr_r[row + at] = make_double4(rx, ry, rz, d);
             dk[at] = d;
             jk[at] = j;
@@ -310,7 +312,7 @@ struct Md {
                            (const int*)L.d_meta.p, (const double4*)L.d_nbrr.p, L.maxp, (double4*)d_T.p,
                            (double*)d_xb.p, built, E.host.rc * E.host.rc, half * half * (1.0 - 1e-9),
                            (int*)E.d_cnt.p, (int*)E.d_nbrj.p, (int*)E.d_meta.p, (double4*)E.d_nbrr.p, E.maxp,
-                           (unsigned short*)E.d_rowtab.p, (int*)E.d_maxcnt.p, (const int*)L.d_maxcnt.p, (int*)d_maxseen.p);
+                           (unsigned short*)E.d_rowtab.p, (unsigned short*)E.d_key.p, (int*)E.d_maxcnt.p, (const int*)L.d_maxcnt.p, (int*)d_maxseen.p);
         HIPCHK(hipGetLastError());
     }
 

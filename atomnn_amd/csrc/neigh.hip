@@ -89,21 +89,23 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int& total) {
     return x - v;
 }
 
-// Index table of row i from its ascending entries in LDS or registers' order: entry p with neighbour index j opens
-// every table slot after its predecessor's (index jp, -1 for the first entry) up to its own.
+// Index table of a row from its ascending entries: entry p with index j opens every table entry after its
+// predecessor's (index jp, -1 for the first entry) up to its own.
 __device__ __forceinline__ void row_tab_open(unsigned short* tab, int width, int jp, int j, int p) {
     const int q0 = jp < 0 ? 0 : jp / width + 1, q1 = j / width;
     for (int q = q0; q <= q1; ++q) tab[q] = (unsigned short)p;
 }
-// the slots after the last entry (index j, -1 in an empty row) of a row of P entries
+// the table entries after the last row entry (index j, -1 in an empty row) of a row of P entries
 __device__ __forceinline__ void row_tab_close(unsigned short* tab, int width, int j, int P, int lane) {
     const int q0 = j < 0 ? 0 : j / width + 1;
     if (lane >= q0 && lane < kRowTab) tab[lane] = (unsigned short)P;
 }
 
 __device__ __forceinline__ void put_entry(int64_t slot, int j, int img, int typ, bool mn, double x, double y, double z,
-                                          double d, int* nbr_j, int* nbr_meta, double4* nbr_r) {
+                                          double d, int* nbr_j, unsigned short* nbr_key, int* nbr_meta,
+                                          double4* nbr_r) {
     nbr_j[slot] = j;
+    nbr_key[slot] = (unsigned short)j;
     nbr_meta[slot] = (img << 8) | (typ << 1) | (mn ? 1 : 0);
     nbr_r[slot] = make_double4(x, y, z, d);
 }
@@ -158,7 +160,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
                                                           const int* __restrict__ centres, double rc2, int maxp,
                                                           int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                           int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                          unsigned short* __restrict__ row_tab, PassCounters pc) {
+                                                          unsigned short* __restrict__ row_tab, unsigned short* __restrict__ nbr_key, PassCounters pc) {
     clear_counters(pc);
     const int i = centres[blockIdx.x];
     const DevStruc& s = S[atom_struc[i]];
@@ -226,7 +228,8 @@ __global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __rest
                         const bool keep = (j != li) ? (d2 <= rc2) : (1e-6 < d2 && d2 <= rc2);
                         if (keep) {
                             if (at < maxp)
-                                put_entry(row + at, j, n, tj, n == minn, rx, ry, rz, sqrt(d2), nbr_j, nbr_meta, nbr_r);
+                                put_entry(row + at, j, n, tj, n == minn, rx, ry, rz, sqrt(d2), nbr_j, nbr_key, nbr_meta,
+                                          nbr_r);
                             ++at;
                         }
                     }
@@ -464,7 +467,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
                                                        const int* __restrict__ bin_atoms, double rc2, int maxp, int n2cap,
                                                        int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                        int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-                                                       unsigned short* __restrict__ row_tab, PassCounters pc) {
+                                                       unsigned short* __restrict__ row_tab, unsigned short* __restrict__ nbr_key, PassCounters pc) {
     extern __shared__ double lds_cells[];
     clear_counters(pc);
     const int cap = maxp;
@@ -557,7 +560,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
         const double d = sqrt(vals[4 * src + 3]);
         // one image per j: it is the minimum image when below ||R||_F (neighbor.cpp:132-140)
         put_entry(row + q, j, 0, type[s.atom0 + j], d < s.fro, vals[4 * src], vals[4 * src + 1], vals[4 * src + 2], d,
-                  nbr_j, nbr_meta, nbr_r);
+                  nbr_j, nbr_key, nbr_meta, nbr_r);
         row_tab_open(row_tab + (int64_t)i * kRowTab, row_tab_width(s.natoms), q > 0 ? skey[q - 1] : -1, j, q);
     }
     row_tab_close(row_tab + (int64_t)i * kRowTab, row_tab_width(s.natoms), P > 0 ? skey[P - 1] : -1, P, lane);
@@ -600,7 +603,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
     const int* __restrict__ type, int ncell, const int* __restrict__ atom_bin,
     const int* __restrict__ bin_start, const float4* __restrict__ bin_pos, int one_struc, double rc2, int maxp,
     int* __restrict__ cnt, int* __restrict__ nbr_j, int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
-    unsigned short* __restrict__ row_tab, int nwords_max, PassCounters pc) {
+    unsigned short* __restrict__ row_tab, unsigned short* __restrict__ nbr_key, int nwords_max, PassCounters pc) {
     extern __shared__ unsigned int lds_bits[];
     clear_counters(pc);
     unsigned short* pre = reinterpret_cast<unsigned short*>(lds_bits + nwords_max);
@@ -724,7 +727,8 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
             const int p = pre[w] + __popc(lds_bits[w] & ((1u << (e.j & 31)) - 1u));
             const double d = sqrt(e.d2);
             // one image per j: it is the minimum image when below ||R||_F (neighbor.cpp:132-140)
-            if (p < maxp) put_entry(row + p, e.j, 0, e.t, d < s.fro, e.x, e.y, e.z, d, nbr_j, nbr_meta, nbr_r);
+            if (p < maxp)
+                put_entry(row + p, e.j, 0, e.t, d < s.fro, e.x, e.y, e.z, d, nbr_j, nbr_key, nbr_meta, nbr_r);
         };
         const NeighEntry e0 = take(lane);
         NeighEntry e1{0.0, 0.0, 0.0, 0.0, -1, 0};
@@ -784,7 +788,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells_bits(
                 double rx, ry, rz;
                 cell_diff(s, xi - pos[3 * gj], yi - pos[3 * gj + 1], zi - pos[3 * gj + 2], rx, ry, rz);
                 const double d = sqrt(rx * rx + ry * ry + rz * rz);
-                put_entry(row + at, lj, 0, type[gj], d < s.fro, rx, ry, rz, d, nbr_j, nbr_meta, nbr_r);
+                put_entry(row + at, lj, 0, type[gj], d < s.fro, rx, ry, rz, d, nbr_j, nbr_key, nbr_meta, nbr_r);
             }
             ++at;
         }
@@ -842,20 +846,20 @@ hipError_t launch_neighbors(const NeighborArgs& a, hipStream_t st) {
             hipLaunchKernelGGL(k_neigh_cells_bits, dim3(xcd_grid(a.ncell)), dim3(kWave),
                                bits_lds + (bits_lds / 2 + 3) / 4 * 4, st, a.S, a.atom_struc, a.pos, a.type, a.ncell,
                                a.atom_bin, a.bin_start, a.bin_pos, a.nstruc == 1, a.rc2, a.maxp, a.cnt, a.nbr_j,
-                               a.nbr_meta, a.nbr_r, a.row_tab, (int)(bits_lds / 4), pc);
+                               a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, (int)(bits_lds / 4), pc);
         } else {  // very large structures: sort the kept candidates instead
             int n2cap = 1;
             while (n2cap < a.maxp) n2cap <<= 1;
             const size_t lds = (size_t)a.maxp * 32 + (size_t)a.maxp * 4 + (size_t)n2cap * 8;
             hipLaunchKernelGGL(k_neigh_cells, dim3(a.ncell), dim3(kWave), lds, st, a.S, a.atom_struc, a.pos, a.type,
                                a.cell_centres, a.atom_bin, a.bin_start, a.bin_atoms, a.rc2, a.maxp, n2cap, a.cnt,
-                               a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, pc);
+                               a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.npair > 0) {
         hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave), 0, st, a.S, a.atom_struc, a.pos, a.type,
-                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, pc);
+                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.ntot > 0 && a.count_max) return launch_count_max(a.cnt, a.ntot, a.maxcnt, st);

@@ -191,7 +191,7 @@ struct Segs {
 };
 
 // Stage the P entries of centre i into LDS, partitioned by neighbour species (stable).
-// su[4p..4p+3] = (ux, uy, uz, d); orig[p] = entry index in the reference order.
+// su[4p..4p+3] = (ux, uy, uz, d); orig[p] = 2 (entry index in the reference order) + min flag.
 template <typename T>
 __device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes, const int* __restrict__ nbr_meta,
                                               const double4* __restrict__ nbr_r, T* su, int* orig, Segs& sg, int lane) {
@@ -218,10 +218,11 @@ __device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     for (int p0 = 0; p0 < P; p0 += kWave) {
         const int p = p0 + lane;
-        int t = -1;
+        int t = -1, meta = 0;
         double4 r = make_double4(0, 0, 0, 1);
         if (p < P) {
-            t = (nbr_meta[row + p] >> 1) & 127;
+            meta = nbr_meta[row + p];
+            t = (meta >> 1) & 127;
             r = nbr_r[row + p];
         }
         int dst = -1;
@@ -239,7 +240,7 @@ __device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes
             su[4 * dst + 1] = T(r.y * inv);
             su[4 * dst + 2] = T(r.z * inv);
             su[4 * dst + 3] = T(r.w);
-            if (orig) orig[dst] = p;
+            if (orig) orig[dst] = (p << 1) | (meta & 1);
         }
     }
 }
@@ -306,16 +307,17 @@ __device__ __forceinline__ void ns_tables(const DevAngular& A, const T* su, int 
     }
 }
 
-// One entry's force term (x, y, z, 0) as a single 32-byte (FP64) or 16-byte (FP32) store.
+// The force term of the entry packed in orig (stage_entries), as (x, y, z, min flag) in a single 32-byte (FP64) or
+// 16-byte (FP32) store at its place in the row; the force assembly reads the flag with the term.
 template <typename T>
-__device__ __forceinline__ void store_x4(T* dst, T x, T y, T z);
+__device__ __forceinline__ void store_x4(T* row, int orig, T x, T y, T z);
 template <>
-__device__ __forceinline__ void store_x4<double>(double* dst, double x, double y, double z) {
-    *reinterpret_cast<double4*>(dst) = make_double4(x, y, z, 0.0);
+__device__ __forceinline__ void store_x4<double>(double* row, int orig, double x, double y, double z) {
+    *reinterpret_cast<double4*>(row + 4 * (orig >> 1)) = make_double4(x, y, z, (double)(orig & 1));
 }
 template <>
-__device__ __forceinline__ void store_x4<float>(float* dst, float x, float y, float z) {
-    *reinterpret_cast<float4*>(dst) = make_float4(x, y, z, 0.f);
+__device__ __forceinline__ void store_x4<float>(float* row, int orig, float x, float y, float z) {
+    *reinterpret_cast<float4*>(row + 4 * (orig >> 1)) = make_float4(x, y, z, (float)(orig & 1));
 }
 
 template <typename T>
@@ -327,7 +329,7 @@ __device__ __forceinline__ double4 load_x4<double>(const double* src) {
 template <>
 __device__ __forceinline__ double4 load_x4<float>(const float* src) {
     const float4 v = *reinterpret_cast<const float4*>(src);
-    return make_double4(v.x, v.y, v.z, 0.0);
+    return make_double4(v.x, v.y, v.z, v.w);
 }
 
 // ------------------------------------------------------------------ per-atom bodies
@@ -854,8 +856,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(NE * NC <
                               dEdG + (int64_t)i * ldg, sg, nsx, mom, lane);
     const int64_t row = (int64_t)i * maxp;
     for (int p = lane; p < P; p += kWave) {
-        const int o = orig[p];
-        store_x4<T>(Xout + 4 * (row + o), Xs[3 * p], Xs[3 * p + 1], Xs[3 * p + 2]);
+        store_x4<T>(Xout + 4 * row, orig[p], Xs[3 * p], Xs[3 * p + 1], Xs[3 * p + 2]);
     }
 }
 
@@ -916,7 +917,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 8))) v
         const double gx = gF[3 * (int64_t)i], gy = gF[3 * (int64_t)i + 1], gz = gF[3 * (int64_t)i + 2];
         const int64_t row = (int64_t)i * maxp;
         for (int p = lane; p < P; p += kWave) {
-            const int64_t e = row + orig[p];
+            const int64_t e = row + (orig[p] >> 1);
             double px = gx, py = gy, pz = gz;
             if ((nbr_meta[e] & 1) || all_images) {
                 const int64_t gj = st.atom0 + nbr_j[e];
@@ -1432,7 +1433,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
                 gx += __shfl_xor(gx, kWave / 2);
                 gy += __shfl_xor(gy, kWave / 2);
                 gz += __shfl_xor(gz, kWave / 2);
-                if (hf == 0 && p < P) store_x4<T>(Xout + 4 * (row + orig[p]), -gx, -gy, -gz);
+                if (hf == 0 && p < P) store_x4<T>(Xout + 4 * row, orig[p], -gx, -gy, -gz);
                 continue;
             }
         }
@@ -1455,7 +1456,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
                 gy += x[1];
                 gz += x[2];
             }
-            store_x4<T>(Xout + 4 * (row + orig[p]), -gx, -gy, -gz);
+            store_x4<T>(Xout + 4 * row, orig[p], -gx, -gy, -gz);
         }
         if (NW > 1) __syncthreads();
     }
@@ -1564,7 +1565,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(NE <= 2 &
         sr *= T(R.norm);
         T gx = sr * su[4 * p], gy = sr * su[4 * p + 1], gz = sr * su[4 * p + 2];
         force_powers_entry<T, NE>(ntypes, su, Rf, Rd, sg.start, wtab, p, s, gx, gy, gz);
-        store_x4<T>(Xout + 4 * (row + orig[p]), -gx, -gy, -gz);
+        store_x4<T>(Xout + 4 * row, orig[p], -gx, -gy, -gz);
     }
 }
 
@@ -1687,8 +1688,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(NE * NC <
                                        slot_row, dErow, dErow, sg, nsx, (use_mom & 2) ? mom : nullptr, lane);
             const int64_t row = (int64_t)i * maxp;
             for (int p = lane; p < P; p += kWave) {
-                const int o = orig[p];
-                store_x4<T>(Xout + 4 * (row + o), Xs[3 * p], Xs[3 * p + 1], Xs[3 * p + 2]);
+                store_x4<T>(Xout + 4 * row, orig[p], Xs[3 * p], Xs[3 * p + 1], Xs[3 * p + 2]);
             }
         }
         __syncthreads();
@@ -1793,7 +1793,9 @@ template hipError_t launch_fused<float>(int, int, int, const DevPlan*, const dou
 // Bound by its chain of dependent look-ups (a's row, the neighbour's table, the stretch of its row, the
 // term).  With a guess at the position and an 8-ary search where it missed (some lane of every wavefront did) the
 // launch took 13.9 us on 4096 atoms, 31 us on 11003 and 155 us on 16 x 4096 (FP32 terms); with the index table
-// 8.8, 25 and 130 us.
+// 8.8, 25 and 130 us.  There each scattered load of a wavefront costs the L1 a clock per lane, so their
+// number counts: 16-bit keys (one load of eight instead of three of four), both table entries in one load,
+// the min flag in the term's fourth word: 7.5, 19 and 96 us.
 //
 // Block order: workgroups are dealt to the 8 XCDs round-robin, each XCD with its own L2.  Block b
 // (after the tail blocks, padded to a multiple of 8) takes position (b mod 8) * chunk + b / 8 of the
@@ -1812,11 +1814,21 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
+// eight keys of a row, from an even place: 16 bytes at 4-byte alignment
+struct __attribute__((packed, aligned(4))) Key8 {
+    unsigned x, y, z, w;
+};
+// two neighbouring table entries in one load
+struct __attribute__((packed, aligned(2))) Pair16 {
+    unsigned v;
+};
+
 template <typename T, int MODE>
 __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                     const int* __restrict__ cnt, const int* __restrict__ nbr_j,
                                                     const int* __restrict__ nbr_meta,
-                                                    const unsigned short* __restrict__ row_tab, const T* __restrict__ X,
+                                                    const unsigned short* __restrict__ row_tab,
+                                                    const unsigned short* __restrict__ nbr_key, const T* __restrict__ X,
                                                     int maxp, int all_images, double* __restrict__ F, EnergyTail tail,
                                                     int* __restrict__ react, const int* __restrict__ rcount,
                                                     const int* __restrict__ rlist, int rcap,
@@ -1842,7 +1854,8 @@ __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__
     if (MODE == 0) {
         const DevStruc& st = S[atom_struc[a]];
         const int la = a - st.atom0;
-        const int slot = la / row_tab_width(st.natoms);  // the table slot of this atom in every row
+        const int width = row_tab_width(st.natoms), slot = la / width;  // the table slot of this atom in every row
+        const unsigned want = (unsigned)(la & 0xffff) * 0x10001u;
         int own = 0, used = 0;
         for (int s = lane; s < P; s += kWave) {
             const int64_t e = row + s;
@@ -1855,9 +1868,9 @@ __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__
             const int64_t rowj = (int64_t)gj * maxp;
             int q0 = 0, q1 = 0;
             if (first) {
-                const unsigned short* tab = row_tab + (int64_t)gj * kRowTab + slot;
-                q0 = tab[0];
-                q1 = slot + 1 < kRowTab ? tab[1] : min(cnt[gj], maxp);
+                const Pair16 tab = *reinterpret_cast<const Pair16*>(row_tab + (int64_t)gj * kRowTab + slot);
+                q0 = (int)(tab.v & 0xffff);
+                q1 = (int)(tab.v >> 16);
             }
             {
                 const double4 v = load_x4<T>(X + 4 * e);
@@ -1865,29 +1878,26 @@ __global__ __launch_bounds__(kWave) void k_assemble(const DevStruc* __restrict__
                 fy += v.y;
                 fz += v.z;
             }
-            // the stretch [q0, q1) of j's row, twelve entries at a time by aligned 16-byte loads
-            for (int w = min(q0 & ~3, maxp - 12); w < q1; w += 12) {
-                const int wc = min(w, maxp - 12);
-                const int4* kv = reinterpret_cast<const int4*>(nbr_j + rowj + wc);
+            // the stretch [q0, q1) of j's row, eight 16-bit keys to a load
+            for (int w = q0 & ~1; w < q1; w += 8) {
+                const int wc = min(w, maxp - 8);
+                const Key8 k4 = *reinterpret_cast<const Key8*>(nbr_key + rowj + wc);
+                const unsigned k[4] = {k4.x ^ want, k4.y ^ want, k4.z ^ want, k4.w ^ want};
                 unsigned m = 0;
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const int4 k4 = kv[k];
-                    m |= ((k4.x == la) | ((k4.y == la) << 1) | ((k4.z == la) << 2) | ((k4.w == la) << 3)) << (4 * k);
-                }
-                const int lo = max(q0, w) - wc, hi = min(q1 - wc, 12);
+                for (int q = 0; q < 4; ++q) m |= (((k[q] & 0xffff) == 0) | ((k[q] >> 16 == 0) << 1)) << (2 * q);
+                const int lo = max(q0, w) - wc, hi = min(q1 - wc, 8);
                 m &= (1u << hi) - (1u << lo);
                 while (m) {
                     const int64_t f = rowj + wc + __ffs(m) - 1;
                     m &= m - 1;
-                    const int meta = nbr_meta[f];
+                    if (width > kKeyWidth && nbr_j[f] != la) continue;  // keys repeat in a stretch this wide
                     const double4 v = load_x4<T>(X + 4 * f);
-                    if (all_images || (meta & 1)) {
-                        fx -= v.x;
-                        fy -= v.y;
-                        fz -= v.z;
-                        ++used;
-                    }
+                    const bool on = all_images || v.w != 0.0;  // selects: the term and its flag stay one load
+                    fx -= on ? v.x : 0.0;
+                    fy -= on ? v.y : 0.0;
+                    fz -= on ? v.z : 0.0;
+                    used += on ? 1 : 0;
                 }
             }
         }
@@ -2131,7 +2141,7 @@ hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* 
     const int ncell = a.bin_atoms ? a.ncell : 0;
     if (a.mode == 0) {
         hipLaunchKernelGGL((k_assemble<T, 0>), grid, dim3(kWave), 0, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta,
-                           a.row_tab, X, a.maxp, a.all_images, a.F, t, a.react, nullptr, nullptr, 0, a.bin_atoms, a.pair_centres,
+                           a.row_tab, a.nbr_key, X, a.maxp, a.all_images, a.F, t, a.react, nullptr, nullptr, 0, a.bin_atoms, a.pair_centres,
                            ncell, a.ntot, chunk);
         return hipGetLastError();
     }
@@ -2140,7 +2150,7 @@ hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* 
     hipLaunchKernelGGL(k_react_zero, dim3((a.ntot + 255) / 256), dim3(256), 0, st, a.rcount, a.ntot, a.react);
     hipLaunchKernelGGL(k_react_fill, dim3(a.ntot), dim3(kWave), 0, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta,
                        a.maxp, a.all_images, a.rcount, a.rlist, a.rcap);
-    hipLaunchKernelGGL((k_assemble<T, 1>), grid, dim3(kWave), lds, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta, a.row_tab, X,
+    hipLaunchKernelGGL((k_assemble<T, 1>), grid, dim3(kWave), lds, st, a.S, a.atom_struc, a.cnt, a.nbr_j, a.meta, a.row_tab, a.nbr_key, X,
                        a.maxp, a.all_images, a.F, t, a.react, a.rcount, a.rlist, a.rcap, a.bin_atoms, a.pair_centres,
                        ncell, a.ntot, chunk);
     return hipGetLastError();
