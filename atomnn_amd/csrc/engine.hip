@@ -286,6 +286,11 @@ Engine::Engine(HostModel&& hm) : host(std::move(hm)) {
     HIPCHK(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev));
     build_adjoint_table();
     build_power_index();
+    if (!pb.net_bf.empty()) {
+        d_netbf.reserve(pb.net_bf.size() * 2);
+        HIPCHK(hipMemcpy(d_netbf.p, pb.net_bf.data(), pb.net_bf.size() * 2, hipMemcpyHostToDevice));
+        pb.plan.net_bf = (const uint16_t*)d_netbf.p;
+    }
     d_plan.reserve(sizeof(DevPlan));
     HIPCHK(hipMemcpy(d_plan.p, &pb.plan, sizeof(DevPlan), hipMemcpyHostToDevice));
     d_rfe.reserve(pb.rfun_eta.size() * 8);
@@ -433,7 +438,7 @@ Engine::~Engine() {
     d_sstart.release();
     d_work.release();
     if (owns_model)
-        for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi, &d_powi})
+        for (DevMem* m : {&d_plan, &d_rfe, &d_rfr, &d_w64, &d_w32, &d_adjc, &d_adji, &d_angc, &d_angi, &d_powi, &d_netbf})
             m->release();
     for (DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
                       &d_brank, &d_bpos, &d_rowtab, &d_key, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_rcount, &d_rlist, &d_mom})

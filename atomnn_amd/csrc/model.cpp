@@ -272,6 +272,38 @@ HostModel parse_ann(const char* path) {
 
 static int pad_to(int v, int q) { return (v + q - 1) / q * q; }
 
+// float to BF16, to nearest even (finite values), and back
+static uint16_t bf16_bits(float x) {
+    uint32_t u;
+    std::memcpy(&u, &x, 4);
+    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+static float bf16_value(uint16_t h) {
+    const uint32_t u = (uint32_t)h << 16;
+    float x;
+    std::memcpy(&x, &u, 4);
+    return x;
+}
+
+// A layer's FP32 weights as the B operand of v_mfma_f32_16x16x32_bf16, split x = hi + lo: for column tile jt and
+// step s of 32 in K, 64 lanes x 8 values of hi, then of lo, where lane l holds B[32 s + 8 (l / 16) + q][16 jt + l % 16]
+// (zero past the layer), so a wavefront loads each operand as one 16-byte load per lane over 1 KB.
+template <class B>
+static int pack_net_bf(std::vector<uint16_t>& out, int ncol, int K, B value) {
+    const int at = (int)(out.size() / 8);
+    for (int jt = 0; jt < ncol / 16; ++jt)
+        for (int s = 0; s < (K + 31) / 32; ++s)
+            for (int part = 0; part < 2; ++part)
+                for (int l = 0; l < 64; ++l)
+                    for (int q = 0; q < 8; ++q) {
+                        const int k = 32 * s + 8 * (l / 16) + q;
+                        const float x = k < K ? (float)value(k, 16 * jt + l % 16) : 0.f;
+                        const uint16_t hi = bf16_bits(x);
+                        out.push_back(part == 0 ? hi : bf16_bits(x - bf16_value(hi)));
+                    }
+    return at;
+}
+
 PlanBuffers build_plan(const HostModel& m) {
     PlanBuffers pb;
     DevPlan& P = pb.plan;
@@ -456,6 +488,16 @@ PlanBuffers build_plan(const HostModel& m) {
         pb.rfun_eta.push_back(0.0);
         pb.rfun_rs.push_back(0.0);
     }
+    if (net_bf_hidden(P))
+        for (int t = 0; t < m.T; ++t) {
+            DevNet& n = P.net[t];
+            for (int l = 0; l < n.L - 1; ++l) {
+                const int in = l == 0 ? n.nin_pad : n.wpad[l - 1], out = n.wpad[l];
+                const double* W = &pb.weights[n.woff[l]];  // out x in, row-major
+                n.bf_fwd[l] = pack_net_bf(pb.net_bf, out, in, [&](int k, int j) { return W[(size_t)j * in + k]; });
+                n.bf_bwd[l] = pack_net_bf(pb.net_bf, in, out, [&](int k, int j) { return W[(size_t)k * in + j]; });
+            }
+        }
     if (pow_ok && !all_mom && P.ne_max <= 4) P.pow_ne = P.ne_max <= 2 ? 2 : 4;
     return pb;
 }

@@ -135,6 +135,9 @@ struct DevNet {
     int pb_off[kMaxLayers];
     int act;                   // NeuronKind of the hidden layers
     int pad_;
+    // weights as split-BF16 MFMA operands (PlanBuffers::net_bf, in 16-byte units): of hidden layer l the forward
+    // operand, and the backward one onto its inputs; see pack_net_bf
+    int bf_fwd[kMaxLayers], bf_bwd[kMaxLayers];
     double outw, outb, evac;
 };
 
@@ -168,6 +171,7 @@ struct DevPlan {
     // G = sum_p coefficient_p X_p over the powers p of the block's moment products
     const double* ang_coef;
     const int* ang_index;
+    const uint16_t* net_bf;  // split-BF16 network weights (device array, set by the engine), or null
     // models in the domain of powers.hpp (pow_ne = 2 or 4 exponents per block, 0 for the others): for centre
     // species t and item (block, exponent e < pow_ne, level) the function's index within the block, or -1
     // (device array, set by the engine)
@@ -175,8 +179,23 @@ struct DevPlan {
     const int* pow_index;
 };
 
+// Hidden layers (1 to 3, the same for every species, tanh, at most 64 units each) that the 32-atom mixed network
+// kernel takes; 0: the model is outside it.
+constexpr int kNetBfUnits = 64, kNetBfLayers = 3;
+inline int net_bf_hidden(const DevPlan& p) {
+    const int h = p.net[0].L - 1;
+    if (h < 1 || h > kNetBfLayers) return 0;
+    for (int t = 0; t < p.T; ++t) {
+        if (p.net[t].L - 1 != h || p.net[t].act != NEU_TANH) return 0;
+        for (int l = 0; l < h; ++l)
+            if (p.net[t].wpad[l] > kNetBfUnits) return 0;
+    }
+    return h;
+}
+
 struct PlanBuffers {
     DevPlan plan;
+    std::vector<uint16_t> net_bf;           // network weights as split-BF16 MFMA operands
     std::vector<double> rfun_eta, rfun_rs;  // radial functions, all blocks
     std::vector<double> weights;            // network weights/biases/scalings (padded)
 };

@@ -493,8 +493,194 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mixed(const DevPlan* 
     }
 }
 
-// One launch covers the 16-atom tiles of every species; the LDS size is the largest species'.
-static NetTiles make_tiles(const int* sp_off, int ntypes, int& ntiles) {
+// ------------------------------------------------------------------ mixed, 32-atom tiles
+// The mixed form for networks of H = 1 to 3 tanh layers of at most 64 units (net_bf_hidden): a block of four
+// wavefronts takes 32 atoms of a species as two 16-row MFMA tiles, and each wavefront one 16-column tile of every
+// hidden layer, so a layer's activations, derivatives and deltas of its tile stay in the wavefront's registers
+// and only the split operands of the next product go through LDS.  The same split products in the same order as
+// k_net_mixed (the energy's row dot products are summed in another order).
+// k_net_mixed converts and splits its operands at every use (each weight once per 16 atoms, each activation once
+// per column tile), 1984 VALU instructions per wavefront and 16 atoms, and reads the weights of the
+// backward products a 4-byte column element at a time.  Here the weights are split once per model and laid out
+// as operands (16 bytes per lane, 1 KB per wavefront), and an activation is split once, where it is computed.
+// 65536 atoms, 84-64-64-1: 130 -> 46 us; 11003 atoms 31 -> 18 us.
+constexpr int kBfRows = 32;
+__host__ __device__ constexpr int bf_lda(int k) { return (k + 31) / 32 * 32 + 8; }  // rows start in different banks
+static size_t net_bf_lds_bytes(const DevNet& n) {
+    return (size_t)kBfRows * 2 * 2 * (size_t)(bf_lda(std::max(n.nin_pad, kNetBfUnits)) + bf_lda(kNetBfUnits)) + 4 * kBfRows * 4 + kBfRows * 4;
+}
+
+// D(32 x 16, column tile jt) over K: A from LDS (hi plane, then lo plane of kBfRows x lda), B from the packed weights.
+template <int TERMS>
+__device__ __forceinline__ void bf_mm(const __bf16* A, int lda, const uint4* __restrict__ B, int K, int jt, int lane,
+                                      f4_t (&acc)[2]) {
+    const int li = lane & 15, lk = lane >> 4;
+    const int ns = (K + 31) / 32;
+    acc[0] = acc[1] = f4_t{0.f, 0.f, 0.f, 0.f};
+    const uint4* b = B + (size_t)jt * ns * 128 + lane;
+    const __bf16* a = A + li * lda + 8 * lk;
+    for (int s = 0; s < ns; ++s) {
+        const bf8_t bh = __builtin_bit_cast(bf8_t, b[s * 128]);
+        bf8_t bl{};
+        if constexpr (TERMS == 3) bl = __builtin_bit_cast(bf8_t, b[s * 128 + 64]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const bf8_t ah = *reinterpret_cast<const bf8_t*>(a + t * 16 * lda + 32 * s);
+            if constexpr (TERMS == 3) {
+                const bf8_t al = *reinterpret_cast<const bf8_t*>(a + (kBfRows + t * 16) * lda + 32 * s);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc[t], 0, 0, 0);
+            }
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc[t], 0, 0, 0);
+        }
+    }
+}
+
+__device__ __forceinline__ void bf_put(__bf16* A, int lda, int row, int col, float x) {
+    const __bf16 h = to_bf16(x);
+    A[row * lda + col] = h;
+    A[(kBfRows + row) * lda + col] = to_bf16(x - (float)h);
+}
+
+template <int TERMS, int H>
+__global__ __launch_bounds__(kNetThreads) void k_net_mixed32(const DevPlan* __restrict__ plan,
+                                                             const float* __restrict__ Wf, NetTiles nt,
+                                                             const int* __restrict__ spatoms,
+                                                             const float* __restrict__ G, int ldg, int vac,
+                                                             double* __restrict__ eatom, float* __restrict__ dEdG) {
+    extern __shared__ __align__(16) unsigned char bf_lds[];
+    const int s = tile_species(nt, plan->T, blockIdx.x);
+    const DevNet& N = plan->net[s];
+    const uint4* bf = reinterpret_cast<const uint4*>(plan->net_bf);
+    const int* atoms = spatoms + nt.atom_start[s];
+    const int M = nt.atom_start[s + 1] - nt.atom_start[s];
+    const int tid = threadIdx.x, wv = tid / kWave, lane = tid % kWave, li = lane & 15, lk = lane >> 4;
+    const int r0 = (blockIdx.x - nt.tile_start[s]) * kBfRows;
+    const int ldi = bf_lda(max(N.nin_pad, kNetBfUnits)), ldh = bf_lda(kNetBfUnits);
+    __bf16* bin = reinterpret_cast<__bf16*>(bf_lds);  // the descriptors' operand (hi, lo); then every other layer's
+    __bf16* bhid = bin + 2 * kBfRows * ldi;
+    float* esum = reinterpret_cast<float*>(bhid + 2 * kBfRows * ldh);  // [4][32] energy parts of the wavefronts
+    int* sat = reinterpret_cast<int*>(esum + 4 * kBfRows);             // atom of each row, -1 past M
+    // scaled inputs inpw .* (G + inpb), zero past nin and on rows past M: eight threads a row, two columns each
+    {
+        const int r = tid >> 3, q = 2 * (tid & 7);
+        const int at = r0 + r < M ? atoms[r0 + r] : -1;
+        if (q == 0) sat[r] = at;
+        const float* g = G + (int64_t)(at >= 0 ? at : 0) * ldg;
+        const int kend = (N.nin_pad + 31) / 32 * 32;
+#pragma unroll 3
+        for (int k = q; k < kend; k += 16) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int kc = min(k + c, N.nin - 1);
+                const float v = Wf[N.inpw_off + kc] * (g[kc] + Wf[N.inpb_off + kc]);
+                bf_put(bin, ldi, r, k + c, at >= 0 && k + c < N.nin ? v : 0.f);
+            }
+        }
+    }
+    // the hidden operand's columns between a layer's width and the next multiple of 32 are read as zeros
+    for (int idx = tid; idx < 2 * kBfRows * ldh / 2; idx += kNetThreads) reinterpret_cast<unsigned*>(bhid)[idx] = 0u;
+    __syncthreads();
+    const int col = wv * 16 + li;
+    float der[H][2][4];  // derivatives of this wavefront's tile, row 16 t + 4 lk + v
+    f4_t acc[2];
+#pragma unroll
+    for (int l = 0; l < H; ++l) {
+        const bool mine = wv * 16 < N.wpad[l];
+        // layer l reads bin (l even) or bhid (l odd) and writes the other
+        const __bf16* A = (l & 1) ? bhid : bin;
+        __bf16* O = (l & 1) ? bin : bhid;
+        const int lda = (l & 1) ? ldh : ldi, ldo = (l & 1) ? ldi : ldh;
+        float part[2][4];
+        if (mine) {
+            bf_mm<TERMS>(A, lda, bf + N.bf_fwd[l], l == 0 ? N.nin_pad : N.wpad[l - 1], wv, lane, acc);
+            const float bc = Wf[N.boff[l] + col];
+            const float wo = l == H - 1 ? Wf[N.woff[H] + col] : 0.f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                float z[4], a[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) z[v] = acc[t][v] + bc;
+                net_act4<false>(NEU_TANH, z, a, der[l][t]);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int row = 16 * t + 4 * lk + v;
+                    if (l < H - 1) {
+                        bf_put(O, ldo, row, col, a[v]);
+                    } else {
+                        // output layer (linear, one unit): energy terms, and the first backward step
+                        part[t][v] = wo * a[v];
+                        bf_put(O, ldo, row, col, (float)N.outw * wo * der[l][t][v]);
+                    }
+                }
+            }
+        } else if (l == H - 1) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) part[t][v] = 0.f;
+        }
+        // what an earlier operand left past this layer's width must read as zero
+        if (l > 0 && N.wpad[l] % 32 != 0)
+            for (int idx = tid; idx < 2 * kBfRows * 16; idx += kNetThreads)
+                O[(idx >> 4) * ldo + N.wpad[l] + (idx & 15)] = (__bf16)0.f;
+        if (l == H - 1) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float e = part[t][v];
+#pragma unroll
+                    for (int o = 8; o > 0; o >>= 1) e += __shfl_xor(e, o, 16);
+                    if (li == 0) esum[wv * kBfRows + 16 * t + 4 * lk + v] = e;
+                }
+        }
+        __syncthreads();
+    }
+    if (tid < kBfRows && sat[tid] >= 0) {
+        const float e = (esum[tid] + esum[kBfRows + tid]) + (esum[2 * kBfRows + tid] + esum[3 * kBfRows + tid]);
+        eatom[sat[tid]] = (double)N.outb + (double)(Wf[N.boff[H]] + e) * N.outw + (vac ? N.evac : 0.0);
+    }
+    // backward through the hidden layers: delta_{l-1} = (delta_l W_l) .* d_{l-1}.  The last hidden layer wrote its
+    // deltas to bhid (H odd) or bin (H even).
+#pragma unroll
+    for (int l = H - 1; l >= 1; --l) {
+        const bool from_bin = (l & 1) != 0;  // layer l's deltas: where the forward step of layer l wrote
+        const __bf16* A = from_bin ? bin : bhid;
+        __bf16* O = from_bin ? bhid : bin;
+        const int lda = from_bin ? ldi : ldh, ldo = from_bin ? ldh : ldi;
+        const bool mine = wv * 16 < N.wpad[l - 1];
+        if (mine) {
+            bf_mm<TERMS>(A, lda, bf + N.bf_bwd[l], N.wpad[l], wv, lane, acc);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) bf_put(O, ldo, 16 * t + 4 * lk + v, col, acc[t][v] * der[l - 1][t][v]);
+        }
+        if (N.wpad[l - 1] % 32 != 0)
+            for (int idx = tid; idx < 2 * kBfRows * 16; idx += kNetThreads)
+                O[(idx >> 4) * ldo + N.wpad[l - 1] + (idx & 15)] = (__bf16)0.f;
+        __syncthreads();
+    }
+    // dE/dG = (delta_0 W_0) .* inpw; layer 0's deltas are in bhid
+    for (int jt = wv; jt < N.nin_pad / 16; jt += kNetWaves) {
+        bf_mm<TERMS>(bhid, ldh, bf + N.bf_bwd[0], N.wpad[0], jt, lane, acc);
+        const int j = jt * 16 + li;
+        if (j < N.nin) {
+            const float w = Wf[N.inpw_off + j];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int at = sat[16 * t + 4 * lk + v];
+                    if (at >= 0) dEdG[(int64_t)at * ldg + j] = acc[t][v] * w;
+                }
+        }
+    }
+}
+
+// One launch covers the tiles (of `rows` atoms) of every species; the LDS size is the largest species'.
+static NetTiles make_tiles(const int* sp_off, int ntypes, int& ntiles, int rows = 16) {
     NetTiles nt;
     ntiles = 0;
     for (int s = 0; s <= kMaxSpecies; ++s) {
@@ -504,7 +690,7 @@ static NetTiles make_tiles(const int* sp_off, int ntypes, int& ntiles) {
     for (int s = 0; s < ntypes; ++s) {
         nt.tile_start[s] = ntiles;
         nt.atom_start[s] = sp_off[s];
-        ntiles += (sp_off[s + 1] - sp_off[s] + 15) / 16;
+        ntiles += (sp_off[s + 1] - sp_off[s] + rows - 1) / rows;
     }
     for (int s = ntypes; s <= kMaxSpecies; ++s) {
         nt.tile_start[s] = ntiles;
@@ -555,6 +741,21 @@ hipError_t launch_net(bool fp64, const DevPlan* plan, const DevPlan& hplan, cons
         const hipError_t e = hipLaunchKernel(f, dim3(grid), dim3(kNetThreads), args, bytes, st);
         if (e != hipSuccess) return e;
         return hipGetLastError();
+    }
+    if (hplan.net_bf) {
+        size_t bfl = 0;
+        for (int s = 0; s < hplan.T; ++s) bfl = std::max(bfl, net_bf_lds_bytes(hplan.net[s]));
+        if (bfl <= 65536) {
+            NetTiles n32 = make_tiles(sp_off, hplan.T, ntiles, kBfRows);
+            const int h = net_bf_hidden(hplan), k = (bf16_terms == 1 ? 0 : 3) + h - 1;
+            const void* fs[] = {kern(k_net_mixed32<1, 1>), kern(k_net_mixed32<1, 2>), kern(k_net_mixed32<1, 3>),
+                                kern(k_net_mixed32<3, 1>), kern(k_net_mixed32<3, 2>), kern(k_net_mixed32<3, 3>)};
+            void* args[] = {(void*)&plan, (void*)&W, (void*)&n32, (void*)&spatoms, (void*)&G, (void*)&ldg, (void*)&vac,
+                            (void*)&eatom, (void*)&dEdG};
+            const hipError_t e = hipLaunchKernel(fs[k], dim3(ntiles), dim3(kNetThreads), args, bfl, st);
+            if (e != hipSuccess) return e;
+            return hipGetLastError();
+        }
     }
     const void* f = bf16_terms == 1 ? (gen ? kern(k_net_mixed<1, true>) : kern(k_net_mixed<1, false>))
                                     : (gen ? kern(k_net_mixed<3, true>) : kern(k_net_mixed<3, false>));
