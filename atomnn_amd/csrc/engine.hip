@@ -34,6 +34,13 @@ int shape_ne(int shape);  // exponents per centre of a grid shape
 constexpr int kMomK = 35;  // monomials of degree <= 4: the moment table's row length
 constexpr int kMomZ = 4;   // their highest degree
 constexpr int kPowL = 10;  // levels of powers.hpp (lambda = +-1, zeta = 1, 2, 4, 8, 16)
+int symm_mom_shape(const DevPlan& p, int ne);
+template <typename T>
+size_t symm_mom_lds(int shape, int lmaxp, int ldg, int ntypes);
+template <typename T>
+hipError_t launch_symm_mom(int shape, int rt, const DevPlan* plan, const double* rfe, const double* rfr,
+                           const int* atom_type, const int* centres, int ncentres, const int* cnt, const int* meta,
+                           const double4* r, int maxp, int lmaxp, T* G, int ldg, int ntypes, hipStream_t st, T* mom_out);
 size_t symm_pow_lds(int ne, bool fp64, int lmaxp, int ldg);
 size_t force_pow_lds(int ne, bool fp64, int lmaxp, int ldg, int ntypes);
 template <typename T>
@@ -60,7 +67,7 @@ template <typename T>
 hipError_t launch_force_mom(int shape, int waves, const DevPlan* plan, const double* rfe, const double* rfr,
                             const int* atom_type, const int* centres, int ncentres, const int* cnt, const int* meta,
                             const double4* r, int maxp, int lmaxp, const T* dEdG, int ldg, T* X, int ntypes,
-                            hipStream_t st, const T* mom_in);
+                            hipStream_t st, const T* mom_in, int mfma);
 template <typename T>
 hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* tail, hipStream_t st);
 hipError_t launch_net(bool fp64, const DevPlan* plan, const DevPlan& hplan, const void* W, const int* sp_off,
@@ -785,7 +792,14 @@ void Engine::descriptors() {
     const bool keep = mom == 2 && !bound && !pb.plan.generic && (moments & 2);
     mom_fresh = 0;
     if (keep) d_mom.reserve((size_t)ntot * pb.plan.T * shape_ne(shape) * kMomK * sizeof(T));
-    HIPCHK(launch_symm<T>(shape, pb.plan.generic, (const DevPlan*)d_plan.p, (const double*)d_rfe.p, (const double*)d_rfr.p,
+    const int rt = mom == 2 ? symm_mom_shape(pb.plan, shape_ne(shape)) : 0;
+    if (rt && symm_mom_lds<T>(shape, lmaxp, pb.plan.ldg, pb.plan.T) <= 65536)
+        HIPCHK(launch_symm_mom<T>(shape, rt, (const DevPlan*)d_plan.p, (const double*)d_rfe.p, (const double*)d_rfr.p,
+                                  (const int*)d_type.p, (const int*)d_centres.p, ntot, (const int*)d_cnt.p,
+                                  (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp, (T*)d_G.p, pb.plan.ldg,
+                                  pb.plan.T, stream, keep ? (T*)d_mom.p : nullptr));
+    else
+        HIPCHK(launch_symm<T>(shape, pb.plan.generic, (const DevPlan*)d_plan.p, (const double*)d_rfe.p, (const double*)d_rfr.p,
                           (const int*)d_type.p, (const int*)d_centres.p, ntot, (const int*)d_cnt.p,
                           (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp, (T*)d_G.p, pb.plan.ldg, mom,
                           pb.plan.T, stream, keep ? (T*)d_mom.p : nullptr));
@@ -870,7 +884,8 @@ void Engine::force_terms() {
                                    (const int*)d_type.p, (const int*)d_centres.p, ntot, (const int*)d_cnt.p,
                                    (const int*)d_meta.p, (const double4*)d_nbrr.p, maxp, lmaxp, (const T*)d_dEdG.p,
                                    pb.plan.ldg, (T*)d_X.p, pb.plan.T, stream,
-                                   mom_fresh == (int)sizeof(T) ? (const T*)d_mom.p : nullptr));
+                                   mom_fresh == (int)sizeof(T) ? (const T*)d_mom.p : nullptr,
+                                   symm_mom_shape(pb.plan, shape_ne(shape)) > 0));
         return;
     }
     if (pb.plan.pow_ne && force_pow_lds(pb.plan.pow_ne, fp64, lmaxp, pb.plan.ldg, pb.plan.T) <= 65536) {

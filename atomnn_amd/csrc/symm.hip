@@ -1230,6 +1230,133 @@ __device__ __forceinline__ double net_body(const DevNet& N, const T* __restrict_
     return E;
 }
 
+// ------------------------------------------------------------------ sums over the entries on the matrix cores
+// Everything summed over a centre's entries is one matrix product, A (32 + 16 RT rows x P) times B (P x 16), in
+// K-steps of four entries of one species:
+//   A rows 0-31    the directly summed monomials u_p^q (moments.hpp)
+//   A rows 32-     the radial functions phi_f(d_p) of the entry's species, 16 to a tile (RT tiles)
+//   B columns      (species s, c): R_e(p) for c = e < NE, fc(p) for c = NE, zero for entries of other species
+// so D holds the moments M[s][e][q] and the radial sums of every function (the other products are unused: a
+// 16 x 16 tile costs the same).  v_mfma_f64_16x16x4 / v_mfma_f32_16x16x4: operands of one value per lane,
+// lane l holding A[l % 16][l / 16] and B[l / 16][l % 16], so the exponentials of the radial functions spread over
+// (function, entry) pairs and no sum crosses lanes on the vector unit.
+template <typename T>
+struct Mfma16x4;
+template <>
+struct Mfma16x4<double> {
+    typedef double Acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ Acc mul(double a, double b, Acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int v, int lk) { return 4 * v + lk; }
+};
+template <>
+struct Mfma16x4<float> {
+    typedef float Acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ Acc mul(float a, float b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int v, int lk) { return 4 * lk + v; }
+};
+
+
+constexpr int kSumCh = 16;  // entries per power-table chunk
+template <typename T, int NE, int RT>
+struct EntrySums {
+    typename Mfma16x4<T>::Acc acc[2 + RT];
+    T diag;  // sum of R_e^2 of this lane's column over its quarter of the entries
+};
+
+// tab: the entries' R_e and (RT > 0) fc, `stride` values per entry.  pw: kSumCh power rows.  Starts and ends with
+// other lanes' LDS reads in flight: barriers around it are the caller's.
+template <typename T, int NE, int RT>
+__device__ __forceinline__ void entry_sums(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
+                                           const double* __restrict__ rfun_rs, int ti, int ntypes, const T* su,
+                                           const T* tab, int stride, const int* seg, T* pw, int lane,
+                                           EntrySums<T, NE, RT>& out) {
+    using M = Mfma16x4<T>;
+    const int li = lane & 15, lk = lane >> 4;
+    // this lane's column (species cs, value cc) and its monomials' places in a power row
+    const int cs = li / (NE + 1), cc = min(li - cs * (NE + 1), stride - 1);
+    int off[2][3];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        int ax, ay, az;
+        mom_exps(16 * t + li, ax, ay, az);
+        off[t][0] = ax;
+        off[t][1] = 5 + ay;
+        off[t][2] = 10 + az;
+    }
+#pragma unroll
+    for (int t = 0; t < 2 + RT; ++t) out.acc[t] = typename M::Acc{T(0), T(0), T(0), T(0)};
+    out.diag = T(0);
+    for (int s = 0; s < ntypes; ++s) {
+        const int p0 = seg[s], p1 = seg[s + 1];
+        if (p0 >= p1) continue;
+        T eta[RT > 0 ? RT : 1], rs[RT > 0 ? RT : 1];
+        if constexpr (RT > 0) {
+            const DevRadial& R = plan->rad[ti][s];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const int f = min(16 * t + li, R.n - 1);  // rows past the functions repeat the last: unused
+                eta[t] = R.n > 0 ? T(rfun_eta[R.fbase + f]) : T(0);
+                rs[t] = R.n > 0 ? T(rfun_rs[R.fbase + f]) : T(0);
+            }
+        }
+        const bool col = cs == s;
+        for (int c0 = p0; c0 < p1; c0 += kSumCh) {
+            __syncthreads();  // the entries and their values are written; the last chunk's readers are done
+            if (lane < 3 * kSumCh) {  // lane (axis, entry)
+                const int c = lane / kSumCh, q = lane - c * kSumCh, p = min(c0 + q, p1 - 1);
+                const T x = su[4 * p + c], x2 = x * x;
+                T* row = pw + q * kMomPw + 5 * c;
+                row[0] = T(1);
+                row[1] = x;
+                row[2] = x2;
+                row[3] = x2 * x;
+                row[4] = x2 * x2;
+            }
+            __syncthreads();
+            for (int k0 = c0; k0 < min(p1, c0 + kSumCh); k0 += 4) {
+                const int p = k0 + lk, pc = min(p, p1 - 1);
+                const T tv = tab[pc * stride + cc];
+                const T b = col && p < p1 ? tv : T(0);
+                out.diag += b * b;
+                const T* row = pw + (k0 - c0 + lk) * kMomPw;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    out.acc[t] = M::mul(row[off[t][0]] * row[off[t][1]] * row[off[t][2]], b, out.acc[t]);
+                if constexpr (RT > 0) {
+                    const T d = su[4 * pc + 3];
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) {
+                        const T x = d - rs[t];
+                        out.acc[2 + t] = M::mul(kexp(-eta[t] * x * x), b, out.acc[2 + t]);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The directly summed moments into Mom[s][e][35], and the diagonals D[s][e] = sum R_e^2 when D is given (the caller's
+// barrier, then mom_derive).
+template <typename T, int NE, int RT>
+__device__ __forceinline__ void put_moments(const EntrySums<T, NE, RT>& sums, int ntypes, T* Mom, T* D, int lane) {
+    const int li = lane & 15, lk = lane >> 4, cs = li / (NE + 1), cc = li - cs * (NE + 1);
+    T diag = sums.diag;
+    diag += __shfl_xor(diag, 16);
+    diag += __shfl_xor(diag, 32);
+    if (cs < ntypes && cc < NE) {
+        T* m = Mom + (cs * NE + cc) * kMomK;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) m[16 * t + Mfma16x4<T>::row(v, lk)] = sums.acc[t][v];
+        if (D && lk == 0) D[cs * NE + cc] = diag;
+    }
+}
+
 // ------------------------------------------------------------------ force terms, NW waves per centre
 // Moment-path force terms when every species takes the moments (fast-path models).  NW
 // wavefronts share one centre: wave w owns the exponents e = w NE/NW ... (w + 1) NE/NW - 1 and the radial
@@ -1319,7 +1446,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
     const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta, const double* __restrict__ rfun_rs,
     const int* __restrict__ atom_type, const int* __restrict__ centres, int ncentres, const int* __restrict__ cnt,
     const int* __restrict__ nbr_meta, const double4* __restrict__ nbr_r, int maxp, int lmaxp,
-    const T* __restrict__ dEdG, int ldg, T* __restrict__ Xout, const T* __restrict__ Min) {
+    const T* __restrict__ dEdG, int ldg, T* __restrict__ Xout, const T* __restrict__ Min, int mfma) {
     constexpr int NK = NE / NW;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int ntypes = plan->T;
@@ -1369,6 +1496,14 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
     }
     __syncthreads();
 
+    if (NW == 1 && mfma) {  // as the descriptor kernel sums them (the same bits)
+        EntrySums<T, NE, 0> sums;
+        entry_sums<T, NE, 0>(plan, rfun_eta, rfun_rs, ti, ntypes, su, Rf, NE, sg.start, U, lane, sums);
+        put_moments<T, NE, 0>(sums, ntypes, Mp, (T*)nullptr, lane);
+        __syncthreads();
+        for (int it = lane; it < ntypes * NE; it += kWave) mom_derive<T>(Mp + it * kMomK);
+        __syncthreads();
+    } else
     // partial moments of this wave's entries [lo, hi) (32 monomials summed over the two half-waves,
     // the last three derived from |u| = 1)
     {
@@ -1466,13 +1601,153 @@ template <typename T, int NE, int NW>
 static hipError_t launch_force_mom_t(const DevPlan* plan, const double* rfe, const double* rfr, const int* atom_type,
                                      const int* centres, int ncentres, const int* cnt, const int* meta,
                                      const double4* r, int maxp, int lmaxp, const T* dEdG, int ldg, T* X, int ntypes,
-                                     hipStream_t st, const T* Min) {
+                                     hipStream_t st, const T* Min, int mfma) {
     const size_t lds = force_mom_lds_bytes<T, NE, NW>(lmaxp, ldg, ntypes);
     if (lds > 65536) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((k_force_mom<T, NE, NW>), dim3(xcd_grid(ncentres)), dim3(kWave * NW), lds, st, plan, rfe,
-                       rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, dEdG, ldg, X, Min);
+                       rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, dEdG, ldg, X, Min, mfma);
     return hipGetLastError();
 }
+
+// ------------------------------------------------------------------ descriptors from moments, on the matrix cores
+// Descriptors of models whose every species takes the moment expansion, with one cutoff per centre species and at
+// most 16 columns (symm_mom_shape); one wavefront per centre, its sums by entry_sums.  Bound by VALU issue.  With
+// the sums on the vector unit (k_symm: per-lane monomials over half-waves, functions over lanes, the cutoff once per
+// species and once more for the angular factors) FP64 took 2203 VALU instructions per centre at P = 45 (2
+// species, NE = 4, 16 radial functions) and FP32 2048 at P = 69 (3 species, NE = 2, 12): 29.2 us on 4096 atoms, 240 us
+// on 16 x 4096; here 1663 and 1463 instructions, 26.1 us and 207 us, and at row head room (molecular dynamics) 34.7 ->
+// 27 us: the moments take the entries' LDS after the sums, 7.2 instead of 9.9 KB a centre.
+// LDS in elements of T: the entries (u, d), their B values and a chunk of power rows, then, in their place, the
+// moments, diagonals and products; the descriptor row
+template <int NE>
+__host__ __device__ constexpr int symm_mom_elems(int lmaxp, int ldg, int ntypes) {
+    return (4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kMomPw > mom_symm_elems<NE>(ntypes)
+                ? 4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kMomPw
+                : mom_symm_elems<NE>(ntypes)) +
+           ((ldg + 1) & ~1);
+}
+
+template <typename T, int NE, int RT>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_symm_mom(
+    const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta, const double* __restrict__ rfun_rs,
+    const int* __restrict__ atom_type, const int* __restrict__ centres, int ncentres, const int* __restrict__ cnt,
+    const int* __restrict__ nbr_meta, const double4* __restrict__ nbr_r, int maxp, int lmaxp, T* __restrict__ G,
+    int ldg, T* __restrict__ Mout) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int ntypes = plan->T;
+    T* Grow = (T*)lds_raw;
+    T* su = Grow + ((ldg + 1) & ~1);
+    T* tab = su + 4 * lmaxp;              // [lmaxp][NE + 1]: R_e, fc
+    T* pw = tab + (NE + 1) * lmaxp;       // [kSumCh][15]
+    T* Mom = su;                          // after the sums
+    T* Dg = Mom + ntypes * NE * kMomK;
+    T* S = Dg + ntypes * NE;
+    __shared__ int seg_lds[kMaxSpecies + 1];
+    Segs sg{seg_lds};
+    const int slot = xcd_slot(ncentres);  // the XCD-local order of the neighbour kernel
+    if (slot < 0) return;
+    const int i = centres[slot];
+    const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+    const int ti = atom_type[i];
+    const int P = min(cnt[i], lmaxp);
+    stage_entries<T>(i, P, maxp, ntypes, nbr_meta, nbr_r, su, nullptr, sg, lane);
+    for (int k = lane; k < ldg; k += kWave) Grow[k] = T(0);
+    __syncthreads();
+    // per entry: the cutoff (one for every block) and the angular factors
+    {
+        const DevAngular& A = plan->ang[ti][0];
+        const T rc = T(A.rc), rci = T(A.rci), pirci = T(A.pirci);
+        for (int p = lane; p < P; p += kWave) {
+            const T d = su[4 * p + 3];
+            T fc, gc;
+            cutoff_fg<T>(A.cut, d, rc, rci, pirci, fc, gc);
+            T* row = tab + p * (NE + 1);
+            ang_sep_entry<T, NE, false>(A, d, fc, gc, row, nullptr);
+            row[NE] = fc;
+        }
+    }
+    EntrySums<T, NE, RT> sums;
+    entry_sums<T, NE, RT>(plan, rfun_eta, rfun_rs, ti, ntypes, su, tab, NE + 1, sg.start, pw, lane, sums);
+    __syncthreads();  // the entries are read; the moments take their place
+    put_moments<T, NE, RT>(sums, ntypes, Mom, Dg, lane);
+    const int cs = li / (NE + 1);
+    if (li - cs * (NE + 1) == NE && cs < ntypes) {  // the fc column of species cs: its radial functions
+        const DevRadial& R = plan->rad[ti][cs];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int f = 16 * t + Mfma16x4<T>::row(v, lk);
+                if (f < R.n) Grow[R.goff + f] = sums.acc[2 + t][v] * T(R.norm);
+            }
+    }
+    __syncthreads();
+    for (int it = lane; it < ntypes * NE; it += kWave) mom_derive<T>(Mom + it * kMomK);
+    __syncthreads();
+    if (Mout) {  // the centre's moment table for the force-term kernel of the same pass
+        T* out = Mout + (int64_t)i * (ntypes * NE * kMomK);
+        for (int it = lane; it < ntypes * NE * kMomK; it += kWave) out[it] = Mom[it];
+    }
+    symm_angular_moments<T, NE>(plan, ti, ntypes, Mom, Dg, S, Grow, lane);
+    __syncthreads();
+    for (int k = lane; k < ldg; k += kWave) G[(int64_t)i * ldg + k] = Grow[k];
+}
+
+// Radial tiles (1 or 2) of k_symm_mom for a model, 0 where it does not apply.
+int symm_mom_shape(const DevPlan& p, int ne) {
+    if (p.generic || p.T * (ne + 1) > 16) return 0;
+    int nr = 0;
+    for (int t = 0; t < p.T; ++t) {
+        const DevAngular& A = p.ang[t][0];
+        if (!p.mom_ok[t]) return 0;  // which also gives every angular block of the species one cutoff
+        for (int b = 0; b < p.T; ++b) {
+            const DevRadial& R = p.rad[t][b];
+            if (R.n > 0 && (R.cut != A.cut || R.rc != A.rc)) return 0;
+            nr = max(nr, R.n);
+        }
+    }
+    return nr <= 16 ? 1 : (nr <= 32 ? 2 : 0);
+}
+template <typename T>
+size_t symm_mom_lds(int shape, int lmaxp, int ldg, int ntypes) {
+    return sizeof(T) * (size_t)(shape == 0 ? symm_mom_elems<2>(lmaxp, ldg, ntypes)
+                                           : shape == 1 ? symm_mom_elems<4>(lmaxp, ldg, ntypes)
+                                                        : symm_mom_elems<8>(lmaxp, ldg, ntypes));
+}
+template <typename T, int NE>
+static void launch_symm_mom_t(int rt, dim3 grid, size_t lds, hipStream_t st, const DevPlan* plan, const double* rfe,
+                              const double* rfr, const int* atom_type, const int* centres, int ncentres, const int* cnt,
+                              const int* meta, const double4* r, int maxp, int lmaxp, T* G, int ldg, T* Mout) {
+    if (rt == 1)
+        hipLaunchKernelGGL((k_symm_mom<T, NE, 1>), grid, dim3(kWave), lds, st, plan, rfe, rfr, atom_type, centres, ncentres,
+                           cnt, meta, r, maxp, lmaxp, G, ldg, Mout);
+    else
+        hipLaunchKernelGGL((k_symm_mom<T, NE, 2>), grid, dim3(kWave), lds, st, plan, rfe, rfr, atom_type, centres, ncentres,
+                           cnt, meta, r, maxp, lmaxp, G, ldg, Mout);
+}
+// rt: symm_mom_shape
+template <typename T>
+hipError_t launch_symm_mom(int shape, int rt, const DevPlan* plan, const double* rfe, const double* rfr,
+                           const int* atom_type, const int* centres, int ncentres, const int* cnt, const int* meta,
+                           const double4* r, int maxp, int lmaxp, T* G, int ldg, int ntypes, hipStream_t st, T* Mout) {
+    const size_t lds = symm_mom_lds<T>(shape, lmaxp, ldg, ntypes);
+    if (lds > 65536) return hipErrorInvalidConfiguration;
+    const dim3 grid(xcd_grid(ncentres));
+#define SYMM_MOM_ARGS rt, grid, lds, st, plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, G, ldg, Mout
+    if (shape == 0) launch_symm_mom_t<T, 2>(SYMM_MOM_ARGS);
+    else if (shape == 1) launch_symm_mom_t<T, 4>(SYMM_MOM_ARGS);
+    else launch_symm_mom_t<T, 8>(SYMM_MOM_ARGS);
+#undef SYMM_MOM_ARGS
+    return hipGetLastError();
+}
+template size_t symm_mom_lds<double>(int, int, int, int);
+template size_t symm_mom_lds<float>(int, int, int, int);
+template hipError_t launch_symm_mom<double>(int, int, const DevPlan*, const double*, const double*, const int*, const int*,
+                                            int, const int*, const int*, const double4*, int, int, double*, int, int,
+                                            hipStream_t, double*);
+template hipError_t launch_symm_mom<float>(int, int, const DevPlan*, const double*, const double*, const int*, const int*,
+                                           int, const int*, const int*, const double4*, int, int, float*, int, int,
+                                           hipStream_t, float*);
 
 // ------------------------------------------------------------------ models with zeta up to 16
 // Descriptor and force kernels of the models whose every angular block is in the domain of powers.hpp (and not
@@ -2102,34 +2377,34 @@ template <typename T, int NW>
 static hipError_t launch_force_mom_w(int shape, const DevPlan* plan, const double* rfe, const double* rfr,
                                      const int* atom_type, const int* centres, int ncentres, const int* cnt,
                                      const int* meta, const double4* r, int maxp, int lmaxp, const T* dEdG, int ldg,
-                                     T* X, int ntypes, hipStream_t st, const T* Min) {
+                                     T* X, int ntypes, hipStream_t st, const T* Min, int mfma) {
     if (shape == 0)
         return launch_force_mom_t<T, 2, NW>(plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp,
-                                            dEdG, ldg, X, ntypes, st, Min);
+                                            dEdG, ldg, X, ntypes, st, Min, mfma);
     if (shape == 1)
         return launch_force_mom_t<T, 4, NW>(plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp,
-                                            dEdG, ldg, X, ntypes, st, Min);
+                                            dEdG, ldg, X, ntypes, st, Min, mfma);
     return launch_force_mom_t<T, 8, NW>(plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, dEdG,
-                                        ldg, X, ntypes, st, Min);
+                                        ldg, X, ntypes, st, Min, mfma);
 }
 
 template <typename T>
 hipError_t launch_force_mom(int shape, int waves, const DevPlan* plan, const double* rfe, const double* rfr,
                             const int* atom_type, const int* centres, int ncentres, const int* cnt, const int* meta,
                             const double4* r, int maxp, int lmaxp, const T* dEdG, int ldg, T* X, int ntypes,
-                            hipStream_t st, const T* Min) {
+                            hipStream_t st, const T* Min, int mfma) {
     if (waves == 1)
         return launch_force_mom_w<T, 1>(shape, plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp,
-                                        dEdG, ldg, X, ntypes, st, Min);
+                                        dEdG, ldg, X, ntypes, st, Min, mfma);
     return launch_force_mom_w<T, 2>(shape, plan, rfe, rfr, atom_type, centres, ncentres, cnt, meta, r, maxp, lmaxp, dEdG,
-                                    ldg, X, ntypes, st, Min);
+                                    ldg, X, ntypes, st, Min, mfma);
 }
 template hipError_t launch_force_mom<double>(int, int, const DevPlan*, const double*, const double*, const int*,
                                              const int*, int, const int*, const int*, const double4*, int, int,
-                                             const double*, int, double*, int, hipStream_t, const double*);
+                                             const double*, int, double*, int, hipStream_t, const double*, int);
 template hipError_t launch_force_mom<float>(int, int, const DevPlan*, const double*, const double*, const int*,
                                             const int*, int, const int*, const int*, const double4*, int, int,
-                                            const float*, int, float*, int, hipStream_t, const float*);
+                                            const float*, int, float*, int, hipStream_t, const float*, int);
 
 template <typename T>
 hipError_t launch_assemble(const AssembleArgs& a, const T* X, const EnergyTail* tail, hipStream_t st) {
