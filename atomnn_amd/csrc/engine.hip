@@ -314,14 +314,15 @@ Engine::Engine(HostModel&& hm) : host(std::move(hm)) {
 // The w table of the moment path's adjoint (moments.hpp adjoint_moments) as a linear map of the
 // dE/dG row: w[blk][e][p] = norm (1/2 for a same-species block) sum_c dE/dG[f(e, c)] C(zeta_c, p)
 // lambda_c^p 2^-zeta_c over the block's angular terms c with f(e, c) defined and p <= zeta_c.
-// Stored per item as kMaxC (index, coefficient) pairs, so the kernel reads one row of constants
+// Stored per item as nc_max (index, coefficient) pairs, so the kernel reads one row of constants
 // instead of walking the block's description.
 void Engine::build_adjoint_table() {
     const DevPlan& P = pb.plan;
     const int ne = shape_ne(shape), T = P.T, nblk = T * (T + 1) / 2;
     const size_t items = (size_t)T * nblk * ne * (kMomZ + 1);
-    std::vector<double> coef(items * kMaxC, 0.0);
-    std::vector<int> index(items * kMaxC, 0);
+    const int nc = P.nc_max;  // terms per item
+    std::vector<double> coef(items * nc, 0.0);
+    std::vector<int> index(items * nc, 0);
     auto binom = [](int z, int p) { int r = 1; for (int k = 0; k < p; ++k) r = r * (z - k) / (k + 1); return r; };
     for (int t = 0; t < T; ++t) {
         if (!P.mom_ok[t]) continue;
@@ -332,7 +333,7 @@ void Engine::build_adjoint_table() {
             const DevAngular& A = P.ang[t][blk];
             for (int e = 0; e < ne && e < A.ne; ++e)
                 for (int p = 0; p <= kMomZ; ++p) {
-                    const size_t base = ((((size_t)t * nblk + blk) * ne + e) * (kMomZ + 1) + p) * kMaxC;
+                    const size_t base = ((((size_t)t * nblk + blk) * ne + e) * (kMomZ + 1) + p) * nc;
                     int k = 0;
                     for (int c = 0; c < A.nc; ++c) {
                         const int f = A.fmap[e * kMaxC + c], z = A.zint[c];
@@ -355,7 +356,7 @@ void Engine::build_adjoint_table() {
     pb.plan.adj_ne = ne;
     // the angular descriptors from the moment products: G_f = norm 2^-zeta sum_p C(zeta, p)
     // lambda^p X_p for the function f of each (block, exponent, term)
-    const size_t gitems = (size_t)T * nblk * ne * kMaxC;
+    const size_t gitems = (size_t)T * nblk * ne * nc;
     std::vector<double> gcoef(gitems * (kMomZ + 1), 0.0);
     std::vector<int> gindex(gitems, -1);
     for (int t = 0; t < T; ++t) {
@@ -366,7 +367,7 @@ void Engine::build_adjoint_table() {
                 for (int c = 0; c < A.nc; ++c) {
                     const int f = A.fmap[e * kMaxC + c], z = A.zint[c];
                     if (f < 0) continue;
-                    const size_t it = (((size_t)t * nblk + blk) * ne + e) * kMaxC + c;
+                    const size_t it = (((size_t)t * nblk + blk) * ne + e) * nc + c;
                     gindex[it] = A.goff + f;
                     double lp = 1.0;
                     for (int p = 0; p <= z && p <= kMomZ; ++p) {

@@ -161,13 +161,13 @@ struct DevPlan {
     DevAngular ang[kMaxSpecies][kMaxSpecies * (kMaxSpecies + 1) / 2];
     DevNet net[kMaxSpecies];
     // adjoint coefficients of the moment path (device arrays, set by the engine): for centre
-    // species t and item (block, exponent e < adj_ne, power p) of the w table, kMaxC pairs
+    // species t and item (block, exponent e < adj_ne, power p) of the w table, nc_max pairs
     // (dE/dG index, coefficient) with w = sum_c dE/dG[index] coefficient (unused pairs: 0, 0.0)
     const double* adj_coef;
     const int* adj_index;
     int adj_ne;
     // angular descriptors from the moment sums: for centre species t and item (block, exponent
-    // e < adj_ne, term c < kMaxC), the descriptor index (-1: none) and five coefficients with
+    // e < adj_ne, term c < nc_max), the descriptor index (-1: none) and five coefficients with
     // G = sum_p coefficient_p X_p over the powers p of the block's moment products
     const double* ang_coef;
     const int* ang_index;

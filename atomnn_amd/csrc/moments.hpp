@@ -271,36 +271,34 @@ template <typename T, int NE>
 __device__ __forceinline__ void symm_angular_moments(const DevPlan* __restrict__ plan, int ti, int ntypes,
                                                      const T* Mom, const T* D, T* S, T* Grow, int lane) {
     const int nblk = ntypes * (ntypes + 1) / 2;
-    // S[blk][e][p] = sum_{|a| = p} (p!/a!) M_a[e][a] M_b[e][a]
-    for (int it = lane; it < nblk * NE * (kMomZ + 1); it += kWave) {
-        const int pd = it % (kMomZ + 1), e = (it / (kMomZ + 1)) % NE, blk = it / ((kMomZ + 1) * NE);
+    // S[blk][e][p] = X_p = sum_{|a| = p} (p!/a!) M_a[e][a] M_b[e][a] (with the diagonal taken out in a species), one lane
+    // per (blk, e): the monomials, and with them the multiplicities, are the same for every lane
+    for (int it = lane; it < nblk * NE; it += kWave) {
+        const int e = it % NE, blk = it / NE;
         int a, bb;
         blk_species(blk, a, bb);
-        const T* Ma = Mom + (a * NE + e) * kMomK;
-        const T* Mb = Mom + (bb * NE + e) * kMomK;
-        T acc = T(0);
-        const int q0 = pd * (pd + 1) * (pd + 2) / 6, q1 = (pd + 1) * (pd + 2) * (pd + 3) / 6;
-        for (int q = q0; q < q1; ++q) acc += T(mom_mult(q)) * Ma[q] * Mb[q];
-        S[it] = acc;
+        const T *Ma = Mom + (a * NE + e) * kMomK, *Mb = Mom + (bb * NE + e) * kMomK;
+        const T diag = D[a * NE + e];
+        int q = 0;
+        for (int p = 0; p <= kMomZ; ++p) {
+            T x = T(0);
+            for (const int q1 = (p + 1) * (p + 2) * (p + 3) / 6; q < q1; ++q) x += T(mom_mult(q)) * Ma[q] * Mb[q];
+            S[it * (kMomZ + 1) + p] = a == bb ? T(0.5) * (x - diag) : x;
+        }
     }
     __syncthreads();
     // G_f = norm 2^-zeta sum_p C(zeta,p) lambda^p X_p, X_p = S_ab or (S_aa - D_a)/2
     if (plan->ang_coef && plan->adj_ne == NE) {  // the engine's rows: index and five coefficients
-        const size_t r0 = (size_t)ti * nblk * NE * kMaxC;
-        for (int it = lane; it < nblk * NE * kMaxC; it += kWave) {
+        const int nc = plan->nc_max;
+        const size_t r0 = (size_t)ti * nblk * NE * nc;
+        for (int it = lane; it < nblk * NE * nc; it += kWave) {
             const int gi = plan->ang_index[r0 + it];
             if (gi < 0) continue;
-            const int e = (it / kMaxC) % NE, blk = it / (kMaxC * NE);
-            int a, bb;
-            blk_species(blk, a, bb);
             const double* cf = plan->ang_coef + (r0 + it) * (kMomZ + 1);
+            const T* x = S + it / nc * (kMomZ + 1);
             T acc = T(0);
 #pragma unroll
-            for (int p = 0; p <= kMomZ; ++p) {
-                T x = S[(blk * NE + e) * (kMomZ + 1) + p];
-                if (a == bb) x = T(0.5) * (x - D[a * NE + e]);
-                acc += T(cf[p]) * x;
-            }
+            for (int p = 0; p <= kMomZ; ++p) acc += T(cf[p]) * x[p];
             Grow[gi] = acc;
         }
         return;
@@ -311,15 +309,11 @@ __device__ __forceinline__ void symm_angular_moments(const DevPlan* __restrict__
         if (e >= A.ne || c >= A.nc) continue;
         const int f = A.fmap[e * kMaxC + c];
         if (f < 0) continue;
-        int a, bb;
-        blk_species(blk, a, bb);
         const int z = A.zint[c];
         const T lam = T(A.lambda[c]);
         T acc = T(0), lp = T(1);
         for (int p = 0; p <= z; ++p) {
-            T x = S[(blk * NE + e) * (kMomZ + 1) + p];
-            if (a == bb) x = T(0.5) * (x - D[a * NE + e]);
-            acc += T(binom4(z, p)) * lp * x;
+            acc += T(binom4(z, p)) * lp * S[(blk * NE + e) * (kMomZ + 1) + p];
             lp *= lam;
         }
         Grow[A.goff + f] = acc * T(A.norm) * T(1.0 / (double)(1 << z));
@@ -456,11 +450,12 @@ __device__ __forceinline__ void adjoint_moments(const DevPlan* __restrict__ plan
         // the w table from the engine's coefficient rows: one row of constants per item
         const size_t b0 = (size_t)ti * nblk * NE * (kMomZ + 1);
         for (int it = tid; it < nblk * NE * (kMomZ + 1); it += nthreads) {
-            const double* cf = plan->adj_coef + (b0 + it) * kMaxC;
-            const int* ix = plan->adj_index + (b0 + it) * kMaxC;
+            const int nc = plan->nc_max;
+            const double* cf = plan->adj_coef + (b0 + it) * nc;
+            const int* ix = plan->adj_index + (b0 + it) * nc;
             T acc = T(0);
-#pragma unroll
-            for (int c = 0; c < kMaxC; ++c) acc += W[ix[c]] * T(cf[c]);
+#pragma unroll 4
+            for (int c = 0; c < nc; ++c) acc += W[ix[c]] * T(cf[c]);
             wtab[it] = acc;
         }
     } else
@@ -485,19 +480,33 @@ __device__ __forceinline__ void adjoint_moments(const DevPlan* __restrict__ plan
         wtab[it] = acc;
     }
     __syncthreads();
-    for (int it = tid; it < ntypes * kMomK * NE; it += nthreads) {
-        const int e = it % NE, q = (it / NE) % kMomK, s = it / (NE * kMomK);
-        const int pd = mom_deg(q);
-        T acc = T(0);
-        for (int b = 0; b < ntypes; ++b) {
-            const int blk = b >= s ? b * (b + 1) / 2 + s : s * (s + 1) / 2 + b;
-            const T wv = wtab[(blk * NE + e) * (kMomZ + 1) + pd];
-            const int mi = (b * NE + e) * kMomK + q;
-            T mb = Mom[mi];
-            for (int k = 1; k < nparts; ++k) mb += Mom[k * pstride + mi];
-            acc += (b == s ? T(2) : T(1)) * wv * mb;
+    // L[s][q][e]: lane q of a wavefront, the species in turn (wavefronts share them), the exponents unrolled; the
+    // multiplicity and degree of a lane's monomial are found once
+    {
+        const int q = tid & (kWave - 1);
+        if (q < kMomK) {
+            const int pd = mom_deg(q);
+            const T mult = T(mom_mult(q));
+            for (int s = tid / kWave; s < ntypes; s += nthreads / kWave) {
+                T acc[NE];
+#pragma unroll
+                for (int e = 0; e < NE; ++e) acc[e] = T(0);
+                for (int b = 0; b < ntypes; ++b) {
+                    const int blk = b >= s ? b * (b + 1) / 2 + s : s * (s + 1) / 2 + b;
+                    const T* wv = wtab + blk * NE * (kMomZ + 1) + pd;
+                    const T* M = Mom + b * NE * kMomK + q;
+                    const T f = b == s ? T(2) * mult : mult;
+#pragma unroll
+                    for (int e = 0; e < NE; ++e) {
+                        T mb = M[e * kMomK];
+                        for (int k = 1; k < nparts; ++k) mb += M[k * pstride + e * kMomK];
+                        acc[e] += f * wv[e * (kMomZ + 1)] * mb;
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < NE; ++e) L[(s * kMomK + q) * NE + e] = acc[e];
+            }
         }
-        L[it] = T(mom_mult(q)) * acc;  // [s][q][e]
     }
     for (int it = tid; it < ntypes * NE; it += nthreads) {
         const int e = it % NE, s = it / NE;

@@ -33,15 +33,16 @@
 #include "basis.hpp"
 #include "moments.hpp"
 #include "powers.hpp"
+#include "fastmath.hpp"
 
 namespace atomnn {
 
-// sin(pi x), cos(pi x): the reduction by pi is exact, so no large-argument path is needed
+// sin(pi x), cos(pi x) for 0 <= x <= 1
 template <typename T>
 __device__ __forceinline__ void sincos_pi(T x, T& s, T& c);
 template <>
 __device__ __forceinline__ void sincos_pi<double>(double x, double& s, double& c) {
-    sincospi(x, &s, &c);
+    sincospi_f64(x, s, c);
 }
 template <>
 __device__ __forceinline__ void sincos_pi<float>(float x, float& s, float& c) {
@@ -70,7 +71,7 @@ __device__ __forceinline__ void cutoff_fg(int kind, T d, T rc, T rci, T pirci, T
     }
 }
 
-// e^x in the per-entry loops.  FP64: the library exp.  FP32 (the mixed form): the hardware 2^x
+// e^x in the per-entry loops.  FP64: exp_f64 (fastmath.hpp).  FP32 (the mixed form): the hardware 2^x
 // (v_exp_f32) of x log2(e), two instructions instead of about ten: the rounding of x log2(e)
 // adds a relative error of |x| 2^-24 at most (3e-6 at x = -50, where e^x is 2e-22), inside what
 // the mixed form's 1 meV/atom gate allows by orders of magnitude.
@@ -78,7 +79,7 @@ template <typename T>
 __device__ __forceinline__ T kexp(T x);
 template <>
 __device__ __forceinline__ double kexp<double>(double x) {
-    return exp(x);
+    return exp_f64(x);
 }
 template <>
 __device__ __forceinline__ float kexp<float>(float x) {
@@ -193,7 +194,7 @@ struct Segs {
 // Stage the P entries of centre i into LDS, partitioned by neighbour species (stable).
 // su[4p..4p+3] = (ux, uy, uz, d); orig[p] = 2 (entry index in the reference order) + min flag.
 template <typename T>
-__device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes, const int* __restrict__ nbr_meta,
+__device__ __forceinline__ void stage_entries_many(int i, int P, int maxp, int ntypes, const int* __restrict__ nbr_meta,
                                               const double4* __restrict__ nbr_r, T* su, int* orig, Segs& sg, int lane) {
     int count[kMaxSpecies];
 #pragma unroll
@@ -243,6 +244,61 @@ __device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes
             if (orig) orig[dst] = (p << 1) | (meta & 1);
         }
     }
+}
+
+// Up to 128 entries stay in registers, two per lane, so all their loads go out together and each species takes one
+// ballot per register; more go through stage_entries_many, which reads the metadata twice.
+template <typename T>
+__device__ __forceinline__ void put_staged(T* su, int* orig, int dst, int p, int meta, const double4& r) {
+    const double inv = 1.0 / r.w;
+    su[4 * dst + 0] = T(r.x * inv);
+    su[4 * dst + 1] = T(r.y * inv);
+    su[4 * dst + 2] = T(r.z * inv);
+    su[4 * dst + 3] = T(r.w);
+    if (orig) orig[dst] = (p << 1) | (meta & 1);
+}
+
+template <typename T>
+__device__ __forceinline__ void stage_entries(int i, int P, int maxp, int ntypes, const int* __restrict__ nbr_meta,
+                                              const double4* __restrict__ nbr_r, T* su, int* orig, Segs& sg, int lane) {
+    if (P > 2 * kWave) {
+        stage_entries_many<T>(i, P, maxp, ntypes, nbr_meta, nbr_r, su, orig, sg, lane);
+        return;
+    }
+    const int64_t row = (int64_t)i * maxp;
+    const int q = kWave + lane;
+    int m0 = 0, m1 = 0, t0 = -1, t1 = -1, d0 = 0, d1 = 0;
+    double4 r0 = make_double4(0, 0, 0, 1), r1 = r0;
+    if (lane < P) {
+        m0 = nbr_meta[row + lane];
+        r0 = nbr_r[row + lane];
+        t0 = (m0 >> 1) & 127;
+    }
+    if (P > kWave) {
+        if (q < P) {
+            m1 = nbr_meta[row + q];
+            r1 = nbr_r[row + q];
+            t1 = (m1 >> 1) & 127;
+        }
+    }
+    auto below = [](unsigned long long m) {
+        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    };
+    int run = 0;
+    for (int s = 0; s < ntypes; ++s) {
+        const unsigned long long b0 = __ballot(t0 == s);
+        if (lane == 0) sg.start[s] = run;
+        d0 = t0 == s ? run + below(b0) : d0;
+        run += __popcll(b0);
+        if (P > kWave) {
+            const unsigned long long b1 = __ballot(t1 == s);
+            d1 = t1 == s ? run + below(b1) : d1;
+            run += __popcll(b1);
+        }
+    }
+    if (lane >= ntypes && lane <= kMaxSpecies) sg.start[lane] = run;
+    if (lane < P) put_staged<T>(su, orig, d0, lane, m0, r0);
+    if (q < P) put_staged<T>(su, orig, d1, q, m1, r1);
 }
 
 // Radial exponent factors of one entry at distance d for an angular block with a separable
@@ -1261,13 +1317,16 @@ struct Mfma16x4<float> {
 
 
 constexpr int kSumCh = 16;  // entries per power-table chunk
+// power row: 1 | x .. x^4 | y .. y^4 | z .. z^4 | d, and one word so that the rows of a K-step start in different banks
+constexpr int kSumRow = 15;
 template <typename T, int NE, int RT>
 struct EntrySums {
-    typename Mfma16x4<T>::Acc acc[2 + RT];
+    typename Mfma16x4<T>::Acc acc[2 + RT], acc2[2 + RT];  // even and odd K-steps: shorter chains of additions
     T diag;  // sum of R_e^2 of this lane's column over its quarter of the entries
 };
 
-// tab: the entries' R_e and (RT > 0) fc, `stride` values per entry.  pw: kSumCh power rows.  Starts and ends with
+// tab: the entries' R_e and (RT > 0) fc, `stride` values per entry; up to 15 entries past the last are read (inside the
+// kernel's LDS: the power rows follow).  pw: kSumCh power rows.  Starts and ends with
 // other lanes' LDS reads in flight: barriers around it are the caller's.
 template <typename T, int NE, int RT>
 __device__ __forceinline__ void entry_sums(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
@@ -1284,11 +1343,11 @@ __device__ __forceinline__ void entry_sums(const DevPlan* __restrict__ plan, con
         int ax, ay, az;
         mom_exps(16 * t + li, ax, ay, az);
         off[t][0] = ax;
-        off[t][1] = 5 + ay;
-        off[t][2] = 10 + az;
+        off[t][1] = ay > 0 ? 4 + ay : 0;
+        off[t][2] = az > 0 ? 8 + az : 0;
     }
 #pragma unroll
-    for (int t = 0; t < 2 + RT; ++t) out.acc[t] = typename M::Acc{T(0), T(0), T(0), T(0)};
+    for (int t = 0; t < 2 + RT; ++t) out.acc[t] = out.acc2[t] = typename M::Acc{T(0), T(0), T(0), T(0)};
     out.diag = T(0);
     for (int s = 0; s < ntypes; ++s) {
         const int p0 = seg[s], p1 = seg[s + 1];
@@ -1306,37 +1365,52 @@ __device__ __forceinline__ void entry_sums(const DevPlan* __restrict__ plan, con
         const bool col = cs == s;
         for (int c0 = p0; c0 < p1; c0 += kSumCh) {
             __syncthreads();  // the entries and their values are written; the last chunk's readers are done
-            if (lane < 3 * kSumCh) {  // lane (axis, entry)
-                const int c = lane / kSumCh, q = lane - c * kSumCh, p = min(c0 + q, p1 - 1);
+            {  // lane (entry, quarter): an axis each, and the distance
+                const int c = lk, p = min(c0 + li, p1 - 1);
                 const T x = su[4 * p + c], x2 = x * x;
-                T* row = pw + q * kMomPw + 5 * c;
-                row[0] = T(1);
+                T* row = pw + li * kSumRow + 4 * c;
                 row[1] = x;
-                row[2] = x2;
-                row[3] = x2 * x;
-                row[4] = x2 * x2;
+                if (c < 3) {
+                    row[2] = x2;
+                    row[3] = x2 * x;
+                    row[4] = x2 * x2;
+                } else {
+                    row[-12] = T(1);
+                }
             }
             __syncthreads();
-            for (int k0 = c0; k0 < min(p1, c0 + kSumCh); k0 += 4) {
-                const int p = k0 + lk, pc = min(p, p1 - 1);
-                const T tv = tab[pc * stride + cc];
-                const T b = col && p < p1 ? tv : T(0);
+            const T* tb = tab + (c0 + lk) * stride + cc;
+            const T* row = pw + lk * kSumRow;
+            const int left = p1 - c0;
+            auto step = [&](auto Q) {
+                constexpr int q = 4 * decltype(Q)::value;
+                auto& ac = decltype(Q)::value % 2 ? out.acc2 : out.acc;
+                if (q >= left) return;
+                const T tv = tb[q * stride];  // past the segment: some other word of the LDS, not used
+                const T b = col && q + lk < left ? tv : T(0);
                 out.diag += b * b;
-                const T* row = pw + (k0 - c0 + lk) * kMomPw;
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
-                    out.acc[t] = M::mul(row[off[t][0]] * row[off[t][1]] * row[off[t][2]], b, out.acc[t]);
+                    ac[t] = M::mul(row[q * kSumRow + off[t][0]] * row[q * kSumRow + off[t][1]] *
+                                       row[q * kSumRow + off[t][2]],
+                                   b, ac[t]);
                 if constexpr (RT > 0) {
-                    const T d = su[4 * pc + 3];
+                    const T d = row[q * kSumRow + 13];
 #pragma unroll
                     for (int t = 0; t < RT; ++t) {
                         const T x = d - rs[t];
-                        out.acc[2 + t] = M::mul(kexp(-eta[t] * x * x), b, out.acc[2 + t]);
+                        ac[2 + t] = M::mul(kexp(-eta[t] * x * x), b, ac[2 + t]);
                     }
                 }
-            }
+            };
+            step(std::integral_constant<int, 0>{});
+            step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{});
+            step(std::integral_constant<int, 3>{});
         }
     }
+#pragma unroll
+    for (int t = 0; t < 2 + RT; ++t) out.acc[t] += out.acc2[t];
 }
 
 // The directly summed moments into Mom[s][e][35], and the diagonals D[s][e] = sum R_e^2 when D is given (the caller's
@@ -1395,8 +1469,8 @@ __host__ __device__ constexpr size_t force_mom_lds_bytes(int lmaxp, int ldg, int
 template <typename T, int NE, int NK>
 __device__ __forceinline__ void force_mom_entry(const DevPlan* __restrict__ plan, const double* __restrict__ rfun_eta,
                                                 const double* __restrict__ rfun_rs, int ti, int ntypes, const Segs& sg,
-                                                const T* su, const T* Cut, const T* W, const T* U, const T* Delta,
-                                                int p, int f0, int fstep, int e0, T& gx, T& gy, T& gz) {
+                                                const T* su, const T* Cut, const T* Ex, const T* W, const T* U,
+                                                const T* Delta, int p, int f0, int fstep, int e0, T& gx, T& gy, T& gz) {
     const DevAngular& A0 = plan->ang[ti][0];
     int s = 0;
     while (s + 1 < ntypes && p >= sg.start[s + 1]) ++s;
@@ -1429,7 +1503,7 @@ __device__ __forceinline__ void force_mom_entry(const DevPlan* __restrict__ plan
     for (int k = 0; k < NK; ++k) {
         const int e = e0 + k;
         const T ie = T(A0.ietap[e]);
-        const T ex = kexp(-ie * dp);
+        const T ex = Ex[p * NE + e];
         const T r = fa * ex, rd = (ga - ie * ddp * fa) * ex;
         const T gu = u[0] * h[0][k] + u[1] * h[1][k] + u[2] * h[2][k];
         const T dEdR = g0[k] - T(2) * Delta[s * NE + e] * r;
@@ -1530,8 +1604,8 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
                                  kWave * NW);
 
     // cutoff value and derivative of every entry, radial then angular, in the partial moments'
-    // place.  Computed ahead of the entry loop: inside it, the polynomial constants of the cosine
-    // are loop invariants that the compiler keeps in registers across the loop, beyond its budget.
+    // place, and its angular exponentials.  Computed ahead of the entry loop, whose adjoint polynomial
+    // takes the registers.
     T* Xx = Mp;
     T* Cut = Mp + (NW - 1) * kWave * 3;
     for (int p = tid; p < P; p += kWave * NW) {
@@ -1547,6 +1621,9 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
         Cut[4 * p + 1] = gc;
         Cut[4 * p + 2] = fa;
         Cut[4 * p + 3] = ga;
+        const T dp = ipow(d, A0.alpha);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) Rf[p * NE + e] = kexp(-T(A0.ietap[e]) * dp);
     }
     __syncthreads();
 
@@ -1563,7 +1640,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
                 const int hf = lane >> 5, p = j0 + (lane & 31);
                 T gx = T(0), gy = T(0), gz = T(0);
                 if (p < P)
-                    force_mom_entry<T, NE, NK / 2>(plan, rfun_eta, rfun_rs, ti, ntypes, sg, su, Cut, W, U, Delta, p, hf,
+                    force_mom_entry<T, NE, NK / 2>(plan, rfun_eta, rfun_rs, ti, ntypes, sg, su, Cut, Rf, W, U, Delta, p, hf,
                                                    2, hf * (NK / 2), gx, gy, gz);
                 gx += __shfl_xor(gx, kWave / 2);
                 gy += __shfl_xor(gy, kWave / 2);
@@ -1575,7 +1652,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(size
         const int p = j0 + lane;
         T gx = T(0), gy = T(0), gz = T(0);
         if (p < P)
-            force_mom_entry<T, NE, NK>(plan, rfun_eta, rfun_rs, ti, ntypes, sg, su, Cut, W, U, Delta, p, w, NW, w * NK,
+            force_mom_entry<T, NE, NK>(plan, rfun_eta, rfun_rs, ti, ntypes, sg, su, Cut, Rf, W, U, Delta, p, w, NW, w * NK,
                                        gx, gy, gz);
         if (w > 0) {
             T* x = Xx + ((w - 1) * kWave + lane) * 3;
@@ -1615,14 +1692,16 @@ static hipError_t launch_force_mom_t(const DevPlan* plan, const double* rfe, con
 // the sums on the vector unit (k_symm: per-lane monomials over half-waves, functions over lanes, the cutoff once per
 // species and once more for the angular factors) FP64 took 2203 VALU instructions per centre at P = 45 (2
 // species, NE = 4, 16 radial functions) and FP32 2048 at P = 69 (3 species, NE = 2, 12): 29.2 us on 4096 atoms, 240 us
-// on 16 x 4096; here 1663 and 1463 instructions, 26.1 us and 207 us, and at row head room (molecular dynamics) 34.7 ->
-// 27 us: the moments take the entries' LDS after the sums, 7.2 instead of 9.9 KB a centre.
+// on 16 x 4096.  Here 1018 and 973 instructions, 21.5 us and 163 us (of which exp_f64, sincospi_f64, entries staged in
+// registers, K-steps unrolled over a chunk and products with uniform trip counts: 1663 -> 1018, 26.1 -> 21.5 us), and at
+// row head room (molecular dynamics) 34.7 -> 22 us: the moments take the entries' LDS after the sums, 7.2 instead of 9.9 KB
+// a centre.
 // LDS in elements of T: the entries (u, d), their B values and a chunk of power rows, then, in their place, the
 // moments, diagonals and products; the descriptor row
 template <int NE>
 __host__ __device__ constexpr int symm_mom_elems(int lmaxp, int ldg, int ntypes) {
-    return (4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kMomPw > mom_symm_elems<NE>(ntypes)
-                ? 4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kMomPw
+    return (4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kSumRow > mom_symm_elems<NE>(ntypes)
+                ? 4 * lmaxp + (NE + 1) * lmaxp + kSumCh * kSumRow
                 : mom_symm_elems<NE>(ntypes)) +
            ((ldg + 1) & ~1);
 }
@@ -1638,7 +1717,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     T* Grow = (T*)lds_raw;
     T* su = Grow + ((ldg + 1) & ~1);
     T* tab = su + 4 * lmaxp;              // [lmaxp][NE + 1]: R_e, fc
-    T* pw = tab + (NE + 1) * lmaxp;       // [kSumCh][15]
+    T* pw = tab + (NE + 1) * lmaxp;       // [kSumCh][kSumRow]
     T* Mom = su;                          // after the sums
     T* Dg = Mom + ntypes * NE * kMomK;
     T* S = Dg + ntypes * NE;
