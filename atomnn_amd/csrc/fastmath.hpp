@@ -1,4 +1,4 @@
-// FP64 exponential and cutoff cosine of the per-entry loops.
+// FP64 exponential and cutoff cosine of the per-entry loops, and the networks' tanh.
 //
 // The per-entry kernels are bound by VALU issue, and most of their instructions were the library's exp (about 30
 // with the range checks and a register move per polynomial coefficient, which the compiler keeps in VGPRs) and
@@ -40,6 +40,36 @@ __device__ __forceinline__ double exp_f64(double x) {
     q = fma(q, r, 1.0);
     q = fma(q, r, 1.0);
     return ldexp(q, (int)n);
+}
+
+// tanh z = -m / (2 + m) with m = e^(-2|z|) - 1, sign of z.  With 2^n and r as above, m = 2^n (e^r - 1) + (2^n - 1):
+// nothing cancels (n = 0 near z = 0, where m = e^r - 1 = r (1 + r q)).  The quotient's divisor lies in [1, 2], so
+// the reciprocal needs no scaling: v_rcp_f64 and two Newton steps, and a correction of the product.  About 35
+// instructions (expm1 and the compiler's division: about 90).
+__device__ __forceinline__ double tanh_f64(double z) {
+    double x = -2.0 * fabs(z);
+    x = x < -1000.0 ? -1000.0 : x;  // (a NaN stays one)
+    const double n = rint(x * 1.4426950408889634);
+    double r = fma(n, -0.6931471805599453, x);
+    r = fma(n, -2.3190468138462996e-17, r);
+    double q = 2.5117605919396305e-08;
+    q = fma_sc(q, r, 2.7630856171049715e-07);
+    q = fma_sc(q, r, 2.755721721092878e-06);
+    q = fma_sc(q, r, 2.4801491260699277e-05);
+    q = fma_sc(q, r, 0.00019841269916209367);
+    q = fma_sc(q, r, 0.001388888894557356);
+    q = fma_sc(q, r, 0.008333333333307848);
+    q = fma_sc(q, r, 0.04166666666652186);
+    q = fma_sc(q, r, 0.166666666666667);
+    q = fma_sc(q, r, 0.5000000000000012);
+    const double p = fma(r * r, q, r);  // e^r - 1
+    const double s = ldexp(1.0, (int)n), m = fma(s, p, s - 1.0), d = 2.0 + m;
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    y = fma(fma(-d, y, 1.0), y, y);
+    double t = -m * y;
+    t = fma(fma(-d, t, -m), y, t);
+    return copysign(t, z);
 }
 
 // sin(pi x) and cos(pi x) for 0 <= x <= 1.  With w = x below 1/4 and w = 1/2 - x above (both exact), |w| <= 1/2,

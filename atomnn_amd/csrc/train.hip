@@ -250,6 +250,358 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_tile(
     }
 }
 
+// ------------------------------------------------------------------ gradient rows of groups of tiles
+// Forward and backward pass of consecutive 16-atom tiles of one species, one gradient row for all of them, for
+// networks of H = 1 or 2 tanh layers of at most U = 32 or 64 units and at most 16 NI <= 128 inputs (train_group_shape).
+// Two teams of U / 16 wavefronts take the tiles in turn; each wavefront owns one 16-column tile of every hidden layer
+// and keeps, for all its tiles, layer 0's weights in registers as MFMA operands (layer 1's in LDS, where both
+// directions and teams read them) and its part of the weight gradient as MFMA accumulators: dz^T a of a tile is K = 16
+// more steps of the same product.  dz of a wavefront's own columns is already the B operand of its gradient products,
+// so LDS holds, besides, only what crosses wavefronts: inputs, a_0, dz_1.  At the end the second team's sums are added
+// to the first's, through LDS, and the block writes one row.
+//   ROWSEED false: rows of one structure, seed outw (the reduction weights the row by the structure's dcdo)
+//   ROWSEED true: seed dcdo[structure] outw per row
+// k_train_tile reads the weights from L2 for every tile, its LDS rows start in one bank, and it writes a row of every
+// parameter per tile, in 8-byte pieces 512 bytes apart: 155 us on 32768 atoms (16 structures, 3 species, 84-64-64-1;
+// 2080 tiles) and 30 us more to add its rows; here 68 and 6 us.  Of the 68, 45 are the tiles (10 on each CU; their 96
+// products of 64 cycles per wavefront are 25 us, the rest the tanh, staging and barriers between them), 10 the
+// plan's, the atoms' and the weights' loads at the start, 5 the row at the end.  Measured: one team with a block or two on
+// a CU 70 and 68 us, with the library's expm1 and quotient in tanh 82.
+// Registers: U = 64 leaves a wavefront 256, which H = 2 with more than 96 inputs does not fit; those networks keep
+// k_train_tile, as do other depths, activations and widths.
+// Sum over the 16 lanes of a DPP row, on every lane.
+__device__ __forceinline__ double row16_sum(double x) {
+    auto ror = [](double y, auto ctrl) {
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(y), ctrl.value, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(y), ctrl.value, 0xf, 0xf, false);
+        return __hiloint2double(hi, lo);
+    };
+    x += ror(x, std::integral_constant<int, 0x128>{});
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    return x + ror(x, std::integral_constant<int, 0x121>{});
+}
+template <int NI>
+__host__ __device__ constexpr int tg_ldi() {
+    return 16 * NI + 4;  // LDS rows: the 16 rows of a K-step start in different banks
+}
+template <int H, int NI, int U>
+__host__ __device__ constexpr int tg_team_elems() {  // of one team: inputs (two buffers), a_0, dz_1, energies, seeds
+    return 2 * 16 * tg_ldi<NI>() + (H - 1) * 2 * 16 * (U + 4) + U + 2 * 16;
+}
+template <int H, int NI, int U>
+__host__ __device__ constexpr int tg_lds_elems() {
+    constexpr int run = (H - 1) * U * (U + 4) + 2 * 16 * NI + 2 * tg_team_elems<H, NI, U>();
+    constexpr int sum = (4 * (NI + (H - 1) * U / 16) + 4) * 4 * U;  // the second team's accumulators at the end
+    return run > sum ? run : sum;
+}
+
+template <int H, int NI, int U, bool ROWSEED>
+__global__ __launch_bounds__(8 * U, U / 32) void k_train_group(
+    const TrainPlan* __restrict__ tp, const double* __restrict__ Wm, const double* __restrict__ par, TrainTiles tt,
+    TrainTiles tr, const int* __restrict__ gtile, const int* __restrict__ batom, const int* __restrict__ bslot,
+    const int* __restrict__ bstruct, const double* __restrict__ G, int ldg, double* __restrict__ out,
+    const double* __restrict__ dcdo, double* __restrict__ partial) {
+    extern __shared__ __align__(16) double tsh[];
+    constexpr int kThreads = 4 * U, ldi = tg_ldi<NI>(), ldu = U + 4, KI = 4 * NI, KH = U / 4, MH = U / 16;
+    constexpr int kPer = kThreads / 16, NV = 16 * NI / kPer;  // threads and inputs of a row in the staging
+    const int g = blockIdx.x;
+    const int s = train_species(tr, tp->T, g);
+    const TrainNet& N = tp->net[s];
+    const int nin = N.nin, nin_pad = N.nin_pad, n0 = N.nodes[0], n1 = N.nodes[H - 1];
+    const double outw = N.outw, outb = N.outb;
+    const int a0 = tt.atom_start[s], M = tt.atom_start[s + 1] - a0, ts0 = tt.tile_start[s];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = __lane_id();
+    const int team = wid / (U / 16), wv = wid - team * (U / 16), tid = wv * kWave + lane, li = lane & 15, lk = lane >> 4;
+    double* W1 = tsh;                                       // [U][ldu] (H = 2): layer 1's weights, zero padded
+    double* sinw = W1 + (H - 1) * U * ldu;                  // [2][16 NI] inpw, inpb
+    double* ins = sinw + 2 * 16 * NI + team * tg_team_elems<H, NI, U>();  // [2][16][ldi]
+    double* A0 = ins + 2 * 16 * ldi;                        // [16][ldu] (H = 2)
+    double* Z1 = A0 + (H - 1) * 16 * ldu;                   // [16][ldu] (H = 2)
+    double* ep = Z1 + (H - 1) * 16 * ldu;                   // [U / 16][16] energies of each wavefront's columns
+    double* seed = ep + U;                                  // [2][16]
+    const int w0 = N.wpad[0], w1 = H == 2 ? N.wpad[1] : w0;  // padded hidden widths (the last one: w1)
+    const int col = wv * 16 + li;
+    const bool on0 = col < w0, on1 = col < w1;  // units past a layer's width carry zeros (tanh 0 = 0)
+    const int t0 = gtile[g], t1 = gtile[g + 1];
+    // Staging of a tile's scaled inputs, kPer threads a row: the row's atom two of the team's tiles ahead, its
+    // descriptors loaded a tile ahead (in flight over that tile's products), written to the other buffer before the
+    // next tile.
+    const int sr = tid / kPer, sk0 = tid - sr * kPer;
+    auto atom_of = [&](int t) {
+        const int row = (t - ts0) * 16 + sr;
+        return t < t1 && row < M ? batom[a0 + row] : -1;  // -1: padding row
+    };
+    double sv[NV];
+    auto load = [&](int src) {
+        const double* gr = G + (int64_t)max(src, 0) * ldg;
+        int sk = sk0;
+        asm volatile("" : "+v"(sk));  // (addresses computed each time: kept over the loop they would spill)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) sv[j] = gr[min(sk + kPer * j, nin - 1)];
+    };
+    auto stage = [&](int t, int b, int src) {
+        int sk = sk0;
+        asm volatile("" : "+v"(sk));
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int k = sk + kPer * j;
+            ins[(b * 16 + sr) * ldi + k] = src >= 0 ? sinw[k] * (sv[j] + sinw[16 * NI + k]) : 0.0;
+        }
+        if (sk == 0)
+            seed[b * 16 + sr] = src < 0 ? 0.0
+                                        : (ROWSEED ? dcdo[bstruct[a0 + (t - ts0) * 16 + sr]] * outw : outw);
+    };
+    int src = atom_of(t0 + team), next = atom_of(t0 + team + 2);
+    load(src);
+    {
+        const double *iw = Wm + N.inpw_off, *ib = Wm + N.inpb_off;
+        for (int k = threadIdx.x; k < 16 * NI; k += 2 * kThreads) {
+            sinw[k] = k < nin ? iw[k] : 0.0;
+            sinw[16 * NI + k] = k < nin ? ib[k] : 0.0;
+        }
+    }
+    // weights: layer 0's forward operands of this wavefront's columns in registers, layer 1 in LDS for both directions
+    // (loads at clamped addresses, so that all are in flight together)
+    double f0[KI];
+    {
+        const double* w = par + N.woff[0] + (int64_t)(on0 ? col : 0) * nin_pad;
+#pragma unroll
+        for (int q = 0; q < KI; ++q) f0[q] = w[min(4 * q + lk, nin_pad - 1)];
+    }
+    if constexpr (H == 2) {  // each team half of the K-steps
+        const double* w = par + N.woff[1] + (int64_t)(on1 ? col : 0) * w0;
+        double f1[KH / 2];
+#pragma unroll
+        for (int q = 0; q < KH / 2; ++q) f1[q] = w[min(4 * (2 * q + team) + lk, w0 - 1)];
+#pragma unroll
+        for (int q = 0; q < KH / 2; ++q) {
+            const int k = 4 * (2 * q + team) + lk;
+            W1[col * ldu + k] = on1 && k < w0 ? f1[q] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < KI; ++q) f0[q] = on0 && 4 * q + lk < nin_pad ? f0[q] : 0.0;
+    const double bias0 = on0 ? par[N.boff[0] + col] : 0.0, bias1 = H == 2 && on1 ? par[N.boff[1] + col] : 0.0;
+    const double wo = on1 ? par[N.woff[H] + col] : 0.0, bo = par[N.boff[H]];
+    d4_t g0[NI], g1[H == 2 ? MH : 1];
+#pragma unroll
+    for (int m = 0; m < NI; ++m) g0[m] = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < (H == 2 ? MH : 1); ++m) g1[m] = d4_t{0.0, 0.0, 0.0, 0.0};
+    double gb0 = 0.0, gb1 = 0.0, gwo = 0.0, gbo = 0.0;
+    __syncthreads();
+    stage(t0 + team, 0, src);
+    __syncthreads();
+    const int nt = (t1 - t0 + 1) / 2;  // tiles of a team; with an odd count the second team's last one is all padding
+    for (int i = 0; i < nt; ++i) {
+        const int t = t0 + team + 2 * i, b = i & 1;
+        const double* in = ins + b * 16 * ldi;
+        src = next;
+        next = atom_of(t + 4);
+        load(src);
+        int slot = -1;  // where the energy of row `lane` goes
+        if (!ROWSEED && wv == team && lane < 16 && t < t1) {
+            const int row = (t - ts0) * 16 + lane, at = a0 + min(row, M - 1);
+            const int q = bslot[at];
+            slot = row < M && batom[at] >= 0 ? q : -1;
+        }
+        double av[4], d0[4], d1[4], z[4];
+        // layer 0
+        {
+            d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < KI; ++q)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(in[li * ldi + 4 * q + lk], f0[q], acc, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) z[v] = acc[v] + bias0;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) train_act<false>(NEU_TANH, z[v], av[v], d0[v]);
+        }
+        if constexpr (H == 2) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) A0[(4 * v + lk) * ldu + col] = av[v];
+            double w[KH / 4];  // a quarter of the weights, read ahead of the barrier
+#pragma unroll
+            for (int q = 0; q < KH / 4; ++q) w[q] = W1[col * ldu + 4 * q + lk];
+            __syncthreads();
+            d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < KH; ++q)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A0[li * ldu + 4 * q + lk],
+                                                           q < KH / 4 ? w[q] : W1[col * ldu + 4 * q + lk], acc, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) z[v] = acc[v] + bias1;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) train_act<false>(NEU_TANH, z[v], av[v], d1[v]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) d1[v] = d0[v];
+        }
+        // output layer (linear, one unit): energy terms, its gradient, and the first backward step
+        double dz[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const double sd = seed[b * 16 + 4 * v + lk];
+            const double e = row16_sum(wo * av[v]);
+            if (li == 0) ep[wv * 16 + 4 * v + lk] = e;
+            gwo += sd * av[v];
+            dz[v] = sd * wo * d1[v];
+            gb1 += dz[v];
+            if constexpr (H == 2) Z1[(4 * v + lk) * ldu + col] = dz[v];
+        }
+        stage(t + 2, b ^ 1, src);
+        __syncthreads();
+        gbo += seed[b * 16 + li];
+        if (wv == team && lane < 16) {  // outputs (the teams' on different SIMDs)
+            double e = 0.0;
+#pragma unroll
+            for (int n = 0; n < MH; ++n) e += ep[n * 16 + lane];
+            if (slot >= 0) out[slot] = outb + (bo + e) * outw;
+        }
+        if constexpr (H == 2) {
+            // layer 1's weight gradient a_0^T dz_1 (rows: layer-0 units), and dz_0 = (dz_1 W_1) .* d_0
+#pragma unroll
+            for (int m = 0; m < MH; ++m)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    g1[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(A0[(4 * q + lk) * ldu + 16 * m + li], dz[q], g1[m], 0, 0, 0);
+            d4_t acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < KH; ++q)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Z1[li * ldu + 4 * q + lk], W1[(4 * q + lk) * ldu + col], acc, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                dz[v] = acc[v] * d0[v];
+                gb0 += dz[v];
+            }
+        }
+        // layer 0's weight gradient ins^T dz_0 (rows: inputs)
+#pragma unroll
+        for (int m = 0; m < NI; ++m)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                g0[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(in[(4 * q + lk) * ldi + 16 * m + li], dz[q], g0[m], 0, 0, 0);
+        __syncthreads();  // the next tile overwrites A0, Z1, ep, and this buffer one tile later
+    }
+    // the second team's sums added to the first's
+    auto each = [&](auto f) {
+        int q = 0;
+#pragma unroll
+        for (int m = 0; m < NI; ++m)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) g0[m][v] = f(g0[m][v], q++);
+        if constexpr (H == 2) {
+#pragma unroll
+            for (int m = 0; m < MH; ++m)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) g1[m][v] = f(g1[m][v], q++);
+            gb0 = f(gb0, q++);
+        }
+        gb1 = f(gb1, q++);
+        gwo = f(gwo, q++);
+        gbo = f(gbo, q++);
+    };
+    if (team == 1) each([&](double x, int q) { return tsh[q * kThreads + tid] = x; });
+    __syncthreads();
+    if (team == 1) return;
+    each([&](double x, int q) { return x + tsh[q * kThreads + tid]; });
+    // the row, in the reference's parameter order
+    double* prow = partial + tr.pbase[s] + (int64_t)(g - tr.tile_start[s]) * N.nparams;
+    auto quarters = [](double v) {
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    gwo = quarters(gwo);
+    gb1 = quarters(gb1);
+    if constexpr (H == 2) {
+        gb0 = quarters(gb0);
+        if (lk == 0 && col < n0) prow[N.rb[0] + col] = gb0;
+        if (lk == 0 && col < n1) prow[N.rb[1] + col] = gb1;
+        if (lk == 0 && col < n1) prow[N.rw[2] + col] = gwo;
+        double* pw = prow + N.rw[1] + lk * n1 + col;
+#pragma unroll
+        for (int m = 0; m < MH; ++m)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (16 * m + 4 * v + lk < n0 && col < n1) pw[(16 * m + 4 * v) * n1] = g1[m][v];
+    } else {
+        if (lk == 0 && col < n0) prow[N.rb[0] + col] = gb1;
+        if (lk == 0 && col < n0) prow[N.rw[1] + col] = gwo;
+    }
+    double* pw = prow + N.rw[0] + lk * n0 + col;
+#pragma unroll
+    for (int m = 0; m < NI; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (16 * m + 4 * v + lk < nin && col < n0) pw[(16 * m + 4 * v) * n0] = g0[m][v];
+    if (wv == 0) {  // the output bias: the sum of the seeds (one a row, on every 16 lanes)
+        gbo = row16_sum(gbo);
+        if (lane == 0) prow[N.rb[H]] = gbo;
+    }
+}
+
+// Hidden layers (1 or 2), inputs in units of 16 (4, 5, 6 or 8) and units (32 or 64) of k_train_group for a model; false
+// where it does not apply.
+struct GroupShape {
+    int h, ni, u;
+};
+static bool train_group_shape(const TrainPlan& p, GroupShape& r) {
+    r.h = p.net[0].L - 1;
+    int in = 0, w = 0;
+    if (r.h < 1 || r.h > 2) return false;
+    for (int t = 0; t < p.T; ++t) {
+        const TrainNet& n = p.net[t];
+        if (n.L - 1 != r.h || n.act != NEU_TANH) return false;
+        for (int l = 0; l < r.h; ++l) w = std::max(w, n.wpad[l]);
+        in = std::max(in, n.nin_pad / 16);
+    }
+    if (in > (r.h == 2 && w > 32 ? 6 : 8) || w > 64) return false;
+    r.ni = in <= 4 ? 4 : (in <= 6 ? in : 8);
+    r.u = w <= 32 ? 32 : 64;
+    return true;
+}
+
+struct GroupArgs {
+    int ngroups;
+    const TrainPlan* tp;
+    const double *Wm, *par;
+    TrainTiles tt, tr;
+    const int *gtile, *batom, *bslot, *bstruct;
+    const double* G;
+    int ldg;
+    double* out;
+    const double* dcdo;
+    double* partial;
+};
+template <int H, int NI, int U, bool RS>
+static hipError_t launch_group_t(const GroupArgs& a, hipStream_t st) {
+    const size_t lds = 8 * (size_t)tg_lds_elems<H, NI, U>();
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k_train_group<H, NI, U, RS>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_train_group<H, NI, U, RS>), dim3(a.ngroups), dim3(8 * U), lds, st, a.tp, a.Wm, a.par, a.tt, a.tr,
+                       a.gtile, a.batom, a.bslot, a.bstruct, a.G, a.ldg, a.out, a.dcdo, a.partial);
+    return hipGetLastError();
+}
+template <int H, int U, bool RS>
+static hipError_t launch_group_n(int ni, const GroupArgs& a, hipStream_t st) {
+    if (ni == 4) return launch_group_t<H, 4, U, RS>(a, st);
+    if (ni == 5) return launch_group_t<H, 5, U, RS>(a, st);
+    if (ni == 8) {
+        if constexpr (H == 1 || U == 32) return launch_group_t<H, 8, U, RS>(a, st);
+        return hipErrorInvalidValue;
+    }
+    return launch_group_t<H, 6, U, RS>(a, st);
+}
+template <bool RS>
+static hipError_t launch_group(const GroupShape& p, const GroupArgs& a, hipStream_t st) {
+    if (p.h == 1) return p.u == 32 ? launch_group_n<1, 32, RS>(p.ni, a, st) : launch_group_n<1, 64, RS>(p.ni, a, st);
+    return p.u == 32 ? launch_group_n<2, 32, RS>(p.ni, a, st) : launch_group_n<2, 64, RS>(p.ni, a, st);
+}
+
 // Force training, one 16-atom tile: the gradient of dcdo out + (dout/dG . V) with respect to the
 // parameters (the energy term, and the term through which the forces depend on the network:
 // V = dL/d(dout/dG) from the descriptor tangents).  dout/dG . V is the network's tangent output
@@ -484,9 +836,11 @@ __global__ __launch_bounds__(256) void k_train_reduce1(const TrainPlan* __restri
     const int a = t0 + g * kReduceGroup, b = min(t1, a + kReduceGroup);
     double acc = 0.0;
     if (tstruct) {  // rows of single-structure tiles, weighted by their structure's dcdo
+#pragma unroll 8
         for (int t = a; t < b; ++t)
             acc += dcdo[tstruct[t]] * partial[tt.pbase[s] + (int64_t)(t - tt.tile_start[s]) * N.nparams + p];
     } else {
+#pragma unroll 8
         for (int t = a; t < b; ++t) acc += partial[tt.pbase[s] + (int64_t)(t - tt.tile_start[s]) * N.nparams + p];
     }
     grp[(int64_t)s * gstride + (int64_t)g * N.nparams + p] = acc;
@@ -638,6 +992,46 @@ class TrainSet {
         int tiles = 0;
         int64_t pb = 0;  // partial elements of all tiles
     };
+
+    // Groups of consecutive tiles of k_train_group: within each run of tiles (one structure's atoms of a species, or
+    // with no struct_t a species), at most `gsize` tiles, gsize the smallest even number (a tile for each
+    // team) that gives at most one group per CU (the kernel's residency, so one round) up to 32 tiles.  The groups' rows take the tiles' places in `rows`.
+    struct Groups {
+        TrainTiles rows;  // group ranges of the species and their row bases
+        int n = 0;
+        int64_t pb = 0;
+        std::vector<int> first;    // first tile of each group, then the tile count
+        std::vector<int> structs;  // structure of each group (struct_t given)
+    };
+    Groups make_groups(const Tiles& tl, const std::vector<int>* struct_t) const {
+        Groups r;
+        const auto build = [&](int gsize) {
+            std::memset(&r.rows, 0, sizeof(r.rows));
+            r.first.clear();
+            r.structs.clear();
+            r.pb = 0;
+            for (int t = 0; t <= kMaxSpecies; ++t) {
+                r.rows.tile_start[t] = (int)r.first.size();
+                r.rows.pbase[t] = r.pb;
+                if (t >= T_) continue;
+                for (int k = tl.tt.tile_start[t]; k < tl.tt.tile_start[t + 1];) {
+                    int e = k + 1;
+                    while (e < tl.tt.tile_start[t + 1] && e - k < gsize && (!struct_t || (*struct_t)[e] == (*struct_t)[k])) ++e;
+                    r.first.push_back(k);
+                    if (struct_t) r.structs.push_back((*struct_t)[k]);
+                    r.pb += plan_.net[t].nparams;
+                    k = e;
+                }
+            }
+            r.n = (int)r.first.size();
+        };
+        for (int gsize = 2 * std::max(1, std::min(16, tl.tiles / (2 * owner_.num_cus))); gsize <= 32; gsize += 2) {
+            build(gsize);
+            if (r.n <= owner_.num_cus) break;
+        }
+        r.first.push_back(tl.tiles);
+        return r;
+    }
 
     void check_args(const char* fn, const double* x, int nbatch, const int* batch, int loss, double delta,
                     const double* err) const {
@@ -836,10 +1230,23 @@ class TrainSet {
                 }
             }
             tiles_ = make_tiles(atom_s, slot_s, struct_s, stream_);
-            if (one_pass_) {
-                std::vector<int> ts;
+            std::vector<int> ts;
+            if (one_pass_)
                 for (int t = 0; t < T_; ++t)
                     for (size_t k = 0; k < struct_s[t].size(); k += 16) ts.push_back(struct_s[t][k]);
+            grouped_ = grad && tiles_.tiles > 0 && train_group_shape(plan_, gshape_);
+            if (grouped_) {
+                groups_ = make_groups(tiles_, one_pass_ ? &ts : nullptr);
+                // rows beyond one buffer: tile by tile, in chunks
+                grouped_ = (int64_t)groups_.n * maxnp <= owner_.train_chunk_elems;
+            }
+            if (grouped_) {
+                ts = groups_.structs;
+                d_gtile_.reserve(4 * groups_.first.size());
+                HIPCHK(hipMemcpyAsync(d_gtile_.p, groups_.first.data(), 4 * groups_.first.size(), hipMemcpyHostToDevice,
+                                      stream_));
+            }
+            if (one_pass_) {
                 d_tstruct_.reserve(4 * std::max<size_t>(ts.size(), 1));
                 HIPCHK(hipMemcpyAsync(d_tstruct_.p, ts.data(), 4 * ts.size(), hipMemcpyHostToDevice, stream_));
             }
@@ -871,7 +1278,15 @@ class TrainSet {
         const double* par = (const double*)d_par_.p;
         const int *ba = (const int*)d_batom_.p, *bsl = (const int*)d_bslot_.p, *bst = (const int*)d_bstruct_.p;
         const double* Gp = (const double*)d_G_.p;
-        if (one_pass_) {
+        GroupArgs ga{};
+        if (grouped_) {
+            d_partial_.reserve(8 * (size_t)groups_.pb);
+            ga = GroupArgs{groups_.n, tpp, Wm,   par,  tl.tt,  groups_.rows, (const int*)d_gtile_.p,         ba,
+                           bsl,       bst, Gp,   ldg_, (double*)d_out_.p,    (const double*)d_dcdo_.p,       (double*)d_partial_.p};
+        }
+        if (one_pass_ && grouped_) {
+            HIPCHK(launch_group<false>(gshape_, ga, stream_));
+        } else if (one_pass_) {
             d_partial_.reserve(8 * (size_t)std::max<int64_t>(tl.pb, 1));
             if (tl.tiles > 0)
                 launch_tile<3>(gen_, dim3(tl.tiles), lds, stream_, tpp, Wm, par, tl.tt, 0, ba, bsl, bst, Gp, ldg_,
@@ -886,7 +1301,11 @@ class TrainSet {
         HIPCHK(hipGetLastError());
         if (grad) {
             HIPCHK(hipMemsetAsync(d_grad_.p, 0, 8 * (size_t)total(), stream_));
-            if (one_pass_) {
+            if (grouped_) {
+                if (!one_pass_) HIPCHK(launch_group<true>(gshape_, ga, stream_));
+                reduce_rows(tl, groups_.rows, 0, groups_.n, stream_, one_pass_ ? (const int*)d_tstruct_.p : nullptr,
+                            (const double*)d_dcdo_.p);
+            } else if (one_pass_) {
                 reduce_rows(tl, tl.tt, 0, tl.tiles, stream_, (const int*)d_tstruct_.p, (const double*)d_dcdo_.p);
             } else {
                 sum_tiles(tl, stream_, [&](const TrainTiles& tc, int c0, int c1) {
@@ -1103,6 +1522,10 @@ class TrainSet {
     Tiles tiles_;
     bool one_pass_ = false;
     DevMem d_tstruct_;
+    bool grouped_ = false;  // the tiles' rows by k_train_group
+    GroupShape gshape_{};
+    Groups groups_;
+    DevMem d_gtile_;
     std::unique_ptr<Engine> ws_;  // workspace of the force passes
     // workspaces that keep the neighbour rows and descriptors of force-training chunks
     std::vector<std::pair<std::vector<int>, std::unique_ptr<Engine>>> fcache_;
