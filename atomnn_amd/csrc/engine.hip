@@ -1379,6 +1379,48 @@ void Engine::resident_fetch(uint32_t flags, nnp_result* res) {
     }
 }
 
+// Descriptors of n atoms to the caller's rows of ldg values, through the two halves of a page-locked buffer of
+// bounded size: the copy of one part runs while the part before it is moved to the caller's rows.
+// (3001 atoms, 2 MB: 283 us with a pageable copy into a new vector and a loop over the values, 239 us so.)
+void Engine::fetch_descriptors(int n, double* G, int ldg) {
+    const size_t lg = (size_t)pb.plan.ldg, row = lg * 8, width = std::min<size_t>(lg, (size_t)std::max(ldg, 0));
+    const int part = (int)std::min<size_t>((size_t)n, std::max<size_t>(1, kDescriptorPart / row));
+    h_down.reserve(2 * part * row);
+    struct Events {
+        hipStream_t st;
+        hipEvent_t e[2] = {nullptr, nullptr};
+        ~Events() {
+            (void)hipStreamSynchronize(st);  // (an exception: no copy into the buffer stays in flight)
+            for (hipEvent_t x : e)
+                if (x) (void)hipEventDestroy(x);
+        }
+    } ev{stream};
+    for (hipEvent_t& x : ev.e) HIPCHK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+    const int parts = (n + part - 1) / part;
+    for (int k = 0; k <= parts; ++k) {
+        if (k < parts) {
+            const size_t a = (size_t)k * part, m = std::min<size_t>(part, n - a);
+            HIPCHK(hipMemcpyAsync((char*)h_down.p + (k & 1) * part * row, (const char*)d_G.p + a * row, m * row,
+                                  hipMemcpyDeviceToHost, stream));
+            HIPCHK(hipEventRecord(ev.e[k & 1], stream));
+        }
+        if (k == 0) continue;
+        HIPCHK(hipEventSynchronize(ev.e[(k - 1) & 1]));
+        const size_t a = (size_t)(k - 1) * part, m = std::min<size_t>(part, n - a);
+        const char* h = (const char*)h_down.p + ((k - 1) & 1) * part * row;
+        if (ldg <= 0) continue;
+        if ((size_t)ldg == lg) {
+            std::memcpy(G + a * lg, h, m * row);
+            continue;
+        }
+        for (size_t i = 0; i < m; ++i) {
+            double* g = G + (a + i) * ldg;
+            std::memcpy(g, h + i * row, width * 8);
+            std::fill(g + width, g + ldg, 0.0);
+        }
+    }
+}
+
 void Engine::fetch(Strucs ss, uint32_t flags, nnp_result* res) {
     int mc = download(false, flags & NNP_FORCE, false);
     if ((defer_count && mc > maxp) || (speculated && mc > lmaxp)) {
@@ -1557,12 +1599,7 @@ int nnp_symm(nnp_model* m, const nnp_structure* s, double* G, int ldg) {
         E.upload(ss);
         E.build_neighbors(false);
         E.descriptors<double>();
-        const int n = s->natoms, lg = E.pb.plan.ldg;
-        std::vector<double> g((size_t)n * lg);
-        HIPCHK(hipMemcpyAsync(g.data(), E.d_G.p, g.size() * 8, hipMemcpyDeviceToHost, E.stream));
-        HIPCHK(hipStreamSynchronize(E.stream));
-        for (int i = 0; i < n; ++i)
-            for (int k = 0; k < ldg; ++k) G[(size_t)i * ldg + k] = k < lg ? g[(size_t)i * lg + k] : 0.0;
+        E.fetch_descriptors(s->natoms, G, ldg);
         return NNP_OK;
     });
 }

@@ -69,6 +69,9 @@ struct HostPinned {
     void release();
 };
 
+// Bytes of descriptors moved to the caller at a time (two such parts are staged).
+constexpr size_t kDescriptorPart = 512 << 10;
+
 struct NeighborArgs {
     const DevStruc* S;
     const int* atom_struc;
@@ -151,6 +154,7 @@ class Engine {
     void bind_scratch(void* base, size_t bytes, const nnp_structure& s);
     std::vector<int> sp_fill;
     void run(Strucs ss, uint32_t flags);
+    void fetch_descriptors(int n, double* G, int ldg);
     void fetch(Strucs ss, uint32_t flags, nnp_result* res);
 
     // device-resident batches: upload once, enqueue passes, fetch results

@@ -820,6 +820,22 @@ __global__ __launch_bounds__(256) void k_train_struct(const double* __restrict__
     }
 }
 
+// Network parameters from the reference's order (x, page-locked host memory read in place: one launch in place of a
+// transposition on the host and a copy) to the training buffer, whose padding stays zero.
+__global__ __launch_bounds__(256) void k_train_params(const TrainPlan* __restrict__ tp, const int64_t* __restrict__ goff,
+                                                      const double* __restrict__ x, double* __restrict__ par) {
+    const TrainNet& N = tp->net[blockIdx.y];
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= N.nparams) return;
+    const double v = x[goff[blockIdx.y] + p];
+    for (int l = 0; l < N.L; ++l) {
+        const int nodes = N.nodes[l], in_real = l == 0 ? N.nin : N.nodes[l - 1], in_pad = l == 0 ? N.nin_pad : N.wpad[l - 1];
+        const int b = p - N.rb[l], w = p - N.rw[l];
+        if (b >= 0 && b < nodes) par[N.boff[l] + b] = v;
+        if (w >= 0 && w < in_real * nodes) par[N.woff[l] + (int64_t)(w % nodes) * in_pad + w / nodes] = v;
+    }
+}
+
 // Gradient rows summed in two fixed-order levels (all rows of a level in parallel):
 // level 1: groups of kReduceGroup consecutive tiles of a species, each summed in tile order into
 // grp[s][g][p]; level 2: grad[goff_s + p] (+)= the groups in order.
@@ -923,7 +939,11 @@ class TrainSet {
             goff_[t + 1] = goff_[t] + N.nparams;
         }
         npar_dev_ = pofs;
-        hpar_.assign(npar_dev_, 0.0);
+        // parameter, gradient and staging memory (sizes known here, so that no pass allocates it); padding weights are zero
+        d_par_.reserve(8 * (size_t)npar_dev_);
+        d_res_.reserve(8 * (size_t)(total() + 3 * n));
+        h_io_.reserve(8 * (size_t)(2 * total() + 3 * n));
+        HIPCHK(hipMemcpy(d_par_.p, std::vector<double>(npar_dev_, 0.0).data(), 8 * (size_t)npar_dev_, hipMemcpyHostToDevice));
         d_plan_.reserve(sizeof(TrainPlan));
         HIPCHK(hipMemcpy(d_plan_.p, &plan_, sizeof(TrainPlan), hipMemcpyHostToDevice));
         d_goff_.reserve(sizeof(int64_t) * (T_ + 1));
@@ -962,6 +982,12 @@ class TrainSet {
         HIPCHK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     }
     ~TrainSet() {
+        if (stream_) (void)hipStreamSynchronize(stream_);
+        if (ws_) (void)hipStreamSynchronize(ws_->stream);
+        for (DevMem* m : {&d_plan_, &d_goff_, &d_G_, &d_par_, &d_out_, &d_dcdo_, &d_res_, &d_partial_, &d_grp_, &d_fref_,
+                          &d_gF_, &d_V_, &d_tstruct_, &d_gtile_})
+            m->release();
+        h_io_.release();
         if (stream_) (void)hipStreamDestroy(stream_);
     }
 
@@ -995,7 +1021,8 @@ class TrainSet {
 
     // Groups of consecutive tiles of k_train_group: within each run of tiles (one structure's atoms of a species, or
     // with no struct_t a species), at most `gsize` tiles, gsize the smallest even number (a tile for each
-    // team) that gives at most one group per CU (the kernel's residency, so one round) up to 32 tiles.  The groups' rows take the tiles' places in `rows`.
+    // team) that gives at most one group per CU (the kernel's residency, so one round) up to 32 tiles.  The groups'
+    // rows take the tiles' places in `rows`.
     struct Groups {
         TrainTiles rows;  // group ranges of the species and their row bases
         int n = 0;
@@ -1045,28 +1072,65 @@ class TrainSet {
     }
 
     // parameters: reference order -> padded row-major layers, uploaded on stream st
-    void pack_params(const double* x, hipStream_t st) {
-        for (int t = 0; t < T_; ++t) {
-            const TrainNet& N = plan_.net[t];
-            const double* y = x + goff_[t];
-            for (int l = 0; l < N.L; ++l) {
-                const int in_pad = l == 0 ? N.nin_pad : N.wpad[l - 1];
-                const int in_real = l == 0 ? N.nin : N.nodes[l - 1];
-                for (int n = 0; n < N.nodes[l]; ++n) {
-                    hpar_[N.boff[l] + n] = y[N.rb[l] + n];
-                    for (int m = 0; m < in_real; ++m) hpar_[N.woff[l] + (int64_t)n * in_pad + m] = y[N.rw[l] + m * N.nodes[l] + n];
-                }
-            }
-        }
-        d_par_.reserve(8 * (size_t)npar_dev_);
-        HIPCHK(hipMemcpyAsync(d_par_.p, hpar_.data(), 8 * (size_t)npar_dev_, hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));  // hpar_ is reused by the next call
+    // Staging of one call: [x, total][results: gradient, then three values a structure].  One kernel reads x in place and
+    // one copy brings every result; with the parameters transposed on the host, four to fifteen pageable copies, and
+    // the tiles and reference values of a chunk sent again on each call, a call waited more than it computed: 194 us
+    // for 16 x 2048 atoms and 310 us for the force training of 24 structures of up to 700, now 121 and 180 us.
+    void pack_params(const double* x, int nbatch, hipStream_t st) {
+        h_io_.reserve(8 * (size_t)(2 * total() + 3 * (int64_t)nbatch));
+        d_res_.reserve(8 * (size_t)(total() + 3 * (int64_t)nbatch));
+        grad_started_ = false;
+        std::memcpy(h_io_.p, x, 8 * (size_t)total());
+        int maxnp = 1;
+        for (int t = 0; t < T_; ++t) maxnp = std::max(maxnp, plan_.net[t].nparams);
+        hipLaunchKernelGGL(k_train_params, dim3((maxnp + 255) / 256, T_), dim3(256), 0, st, (const TrainPlan*)d_plan_.p,
+                           (const int64_t*)d_goff_.p, (const double*)h_io_.p, (double*)d_par_.p);
+        HIPCHK(hipGetLastError());
     }
+    // Values q (0: losses, 1: squared energy residuals, 2: squared force residuals) of the call's structures.
+    double* res(int q, int nbatch) const { return (double*)d_res_.p + total() + (int64_t)q * nbatch; }
+    // The results in host memory: the gradient at [0], res(q) at [total + q nbatch].
+    const double* fetch_results(int nbatch, int nq, double* grad, hipStream_t st) {
+        const int64_t o = grad ? 0 : total(), n = total() + (int64_t)nq * nbatch - o;
+        double* h = (double*)h_io_.p + total();
+        if (grad && !grad_started_) HIPCHK(hipMemsetAsync(d_res_.p, 0, 8 * (size_t)total(), st));
+        HIPCHK(hipMemcpyAsync(h + o, (const double*)d_res_.p + o, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        if (grad) std::memcpy(grad, h, 8 * (size_t)total());
+        return h + total();
+    }
+    // A call that ends by an exception leaves nothing in flight on its stream (the staging memory is written again
+    // by the next call).
+    struct Settle {
+        hipStream_t st;
+        ~Settle() {
+            if (std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(st);
+        }
+    };
 
     // Species tiles of 16 atoms over the given (source row, slot, structure) lists per species,
     // uploaded into d_batom_, d_bslot_, d_bstruct_ on stream st.
+    // What a batch's tiles read: atoms, slots and structures by species, first slots, reference energies, first
+    // reference force of each structure (force training).
+    struct TileArrays {
+        DevMem atom, slot, strct, bstart, eref, fstart;
+        TileArrays() = default;
+        TileArrays(const TileArrays&) = delete;
+        ~TileArrays() {
+            for (DevMem* m : {&atom, &slot, &strct, &bstart, &eref, &fstart}) m->release();
+        }
+    };
+    // Force training's state of a chunk of structures: workspace and tiles.
+    struct Chunk {
+        std::vector<int> key;
+        std::unique_ptr<Engine> own;  // null: the scratch workspace
+        Tiles tl;
+        TileArrays ta;
+        bool settled = false;  // its rows' reaction tables are known to miss nothing
+    };
+
     Tiles make_tiles(const std::vector<std::vector<int>>& atom_s, const std::vector<std::vector<int>>& slot_s,
-                     const std::vector<std::vector<int>>& struct_s, hipStream_t st) {
+                     const std::vector<std::vector<int>>& struct_s, hipStream_t st, TileArrays& ta) {
         Tiles r;
         std::memset(&r.tt, 0, sizeof(r.tt));
         hbatom_.clear();
@@ -1086,19 +1150,19 @@ class TrainSet {
             }
         }
         const size_t nba = std::max<size_t>(hbatom_.size(), 1);
-        d_batom_.reserve(4 * nba);
-        d_bslot_.reserve(4 * nba);
-        d_bstruct_.reserve(4 * nba);
-        HIPCHK(hipMemcpyAsync(d_batom_.p, hbatom_.data(), 4 * hbatom_.size(), hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(d_bslot_.p, hbslot_.data(), 4 * hbslot_.size(), hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(d_bstruct_.p, hbstruct_.data(), 4 * hbstruct_.size(), hipMemcpyHostToDevice, st));
+        ta.atom.reserve(4 * nba);
+        ta.slot.reserve(4 * nba);
+        ta.strct.reserve(4 * nba);
+        HIPCHK(hipMemcpyAsync(ta.atom.p, hbatom_.data(), 4 * hbatom_.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(ta.slot.p, hbslot_.data(), 4 * hbslot_.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(ta.strct.p, hbstruct_.data(), 4 * hbstruct_.size(), hipMemcpyHostToDevice, st));
         return r;
     }
 
     // Gradient rows of every tile, in chunks of tiles (at most the model's train_chunk_elems row
     // elements at a time, 2^28 = 2 GB by default):
     // launch(tc, c0, c1) writes the rows of tiles [c0, c1) at the shifted bases of tc; the rows are
-    // then added into d_grad_ in a fixed order (groups of consecutive tiles, then the groups).
+    // then added into the gradient in a fixed order (groups of consecutive tiles, then the groups).
     template <typename F>
     void sum_tiles(const Tiles& tl, hipStream_t st, F&& launch) {
         if (tl.tiles == 0) return;
@@ -1123,7 +1187,7 @@ class TrainSet {
         }
     }
 
-    // d_grad_ += the rows of tiles [c0, c1) (bases tc), optionally weighted by dcdo[tstruct[tile]].
+    // The gradient (d_res_; set by a call's first rows) += the rows of tiles [c0, c1) (bases tc), optionally weighted by dcdo[tstruct[tile]].
     void reduce_rows(const Tiles& tl, const TrainTiles& tc, int c0, int c1, hipStream_t st, const int* tstruct,
                      const double* dcdo) {
         (void)tl;
@@ -1138,8 +1202,9 @@ class TrainSet {
         hipLaunchKernelGGL(k_train_reduce1, dim3(pblocks, gmax, T_), dim3(256), 0, st, (const TrainPlan*)d_plan_.p, tc, c0,
                            c1, (const double*)d_partial_.p, gmax, gstride, (double*)d_grp_.p, tstruct, dcdo);
         hipLaunchKernelGGL(k_train_reduce2, dim3(pblocks, T_), dim3(256), 0, st, (const TrainPlan*)d_plan_.p, tc, c0, c1,
-                           (const double*)d_grp_.p, gstride, (const int64_t*)d_goff_.p, (double*)d_grad_.p, 1);
+                           (const double*)d_grp_.p, gstride, (const int64_t*)d_goff_.p, (double*)d_res_.p, grad_started_ ? 1 : 0);
         HIPCHK(hipGetLastError());
+        grad_started_ = true;
     }
 
     // A tile kernel's dynamic LDS within the device's per-workgroup limit (above 64 KiB the kernel
@@ -1165,7 +1230,8 @@ class TrainSet {
 
     void error(const double* x, int nbatch, const int* batch, int loss, double delta, double* err, double* grad) {
         check_args("nnp_train_error", x, nbatch, batch, loss, delta, err);
-        pack_params(x, stream_);
+        const Settle settle{stream_};
+        pack_params(x, nbatch, stream_);
         int64_t maxnp = 1;
         for (int t = 0; t < T_; ++t) maxnp = std::max<int64_t>(maxnp, plan_.net[t].nparams);
         // Tiles: with the gradient, single-structure tiles (each structure's atoms of a species
@@ -1229,7 +1295,7 @@ class TrainSet {
                     struct_s[t].swap(pst);
                 }
             }
-            tiles_ = make_tiles(atom_s, slot_s, struct_s, stream_);
+            tiles_ = make_tiles(atom_s, slot_s, struct_s, stream_, ta_);
             std::vector<int> ts;
             if (one_pass_)
                 for (int t = 0; t < T_; ++t)
@@ -1250,21 +1316,19 @@ class TrainSet {
                 d_tstruct_.reserve(4 * std::max<size_t>(ts.size(), 1));
                 HIPCHK(hipMemcpyAsync(d_tstruct_.p, ts.data(), 4 * ts.size(), hipMemcpyHostToDevice, stream_));
             }
-            d_bstart_.reserve(4 * (size_t)(nbatch + 1));
-            d_out_.reserve(8 * (size_t)std::max(bstart[nbatch], 1));
-            HIPCHK(hipMemcpyAsync(d_bstart_.p, bstart.data(), 4 * (size_t)(nbatch + 1), hipMemcpyHostToDevice, stream_));
+            std::vector<double> eb(nbatch);
+            for (int b = 0; b < nbatch; ++b) eb[b] = eref_[batch[b]];
+            ta_.eref.reserve(8 * (size_t)nbatch);
+            HIPCHK(hipMemcpyAsync(ta_.eref.p, eb.data(), 8 * (size_t)nbatch, hipMemcpyHostToDevice, stream_));
+            ta_.bstart.reserve(4 * (size_t)(nbatch + 1));
+            natoms_batch_ = bstart[nbatch];
+            HIPCHK(hipMemcpyAsync(ta_.bstart.p, bstart.data(), 4 * (size_t)(nbatch + 1), hipMemcpyHostToDevice, stream_));
             HIPCHK(hipStreamSynchronize(stream_));  // the host vectors above go out of scope
             tiles_key_ = key;
         }
         const Tiles& tl = tiles_;
-        std::vector<double> eb(nbatch);
-        for (int b = 0; b < nbatch; ++b) eb[b] = eref_[batch[b]];
-        d_eref_.reserve(8 * (size_t)nbatch);
+        d_out_.reserve(8 * (size_t)std::max(natoms_batch_, 1));
         d_dcdo_.reserve(8 * (size_t)nbatch);
-        d_loss_.reserve(8 * (size_t)nbatch);
-        d_dE2_.reserve(8 * (size_t)nbatch);
-        d_grad_.reserve(8 * (size_t)total());
-        HIPCHK(hipMemcpyAsync(d_eref_.p, eb.data(), 8 * (size_t)nbatch, hipMemcpyHostToDevice, stream_));
         size_t lds = 0;
         for (int t = 0; t < T_; ++t) lds = std::max(lds, train_lds_bytes(plan_.net[t]));
         for (int md = 0; md < 4; md += (md == 1 ? 2 : 1)) {  // modes 0, 1, 3
@@ -1276,7 +1340,7 @@ class TrainSet {
         const double* Wm = (const double*)owner_.d_w64.p;
         const TrainPlan* tpp = (const TrainPlan*)d_plan_.p;
         const double* par = (const double*)d_par_.p;
-        const int *ba = (const int*)d_batom_.p, *bsl = (const int*)d_bslot_.p, *bst = (const int*)d_bstruct_.p;
+        const int *ba = (const int*)ta_.atom.p, *bsl = (const int*)ta_.slot.p, *bst = (const int*)ta_.strct.p;
         const double* Gp = (const double*)d_G_.p;
         GroupArgs ga{};
         if (grouped_) {
@@ -1296,11 +1360,10 @@ class TrainSet {
                            (double*)d_out_.p, nullptr, nullptr, nullptr);
         }
         hipLaunchKernelGGL(k_train_struct, dim3(nbatch), dim3(256), 0, stream_, (const double*)d_out_.p,
-                           (const int*)d_bstart_.p, (const double*)d_eref_.p, loss, delta, (double*)d_dcdo_.p,
-                           (double*)d_loss_.p, (double*)d_dE2_.p);
+                           (const int*)ta_.bstart.p, (const double*)ta_.eref.p, loss, delta, (double*)d_dcdo_.p,
+                           res(0, nbatch), res(1, nbatch));
         HIPCHK(hipGetLastError());
         if (grad) {
-            HIPCHK(hipMemsetAsync(d_grad_.p, 0, 8 * (size_t)total(), stream_));
             if (grouped_) {
                 if (!one_pass_) HIPCHK(launch_group<true>(gshape_, ga, stream_));
                 reduce_rows(tl, groups_.rows, 0, groups_.n, stream_, one_pass_ ? (const int*)d_tstruct_.p : nullptr,
@@ -1314,11 +1377,8 @@ class TrainSet {
                 });
             }
         }
-        std::vector<double> lv(nbatch), e2(nbatch);
-        HIPCHK(hipMemcpyAsync(lv.data(), d_loss_.p, 8 * (size_t)nbatch, hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipMemcpyAsync(e2.data(), d_dE2_.p, 8 * (size_t)nbatch, hipMemcpyDeviceToHost, stream_));
-        if (grad) HIPCHK(hipMemcpyAsync(grad, d_grad_.p, 8 * (size_t)total(), hipMemcpyDeviceToHost, stream_));
-        HIPCHK(hipStreamSynchronize(stream_));
+        const double* lv = fetch_results(nbatch, 2, grad, stream_);
+        const double* e2 = lv + nbatch;
         err[0] = err[1] = 0.0;
         for (int b = 0; b < nbatch; ++b) {
             err[0] += lv[b];
@@ -1339,7 +1399,8 @@ class TrainSet {
         if (!ws_) ws_ = std::make_unique<Engine>(owner_, 1001);
         const hipStream_t st = ws_->stream;  // every chunk's work is ordered on this stream
         const bool all_images = flags & NNP_ALL_IMAGES;
-        pack_params(x, st);
+        const Settle settle{st};
+        pack_params(x, nbatch, st);
         size_t lds = 0, flds = 0;
         for (int t = 0; t < T_; ++t) {
             lds = std::max(lds, train_lds_bytes(plan_.net[t]));
@@ -1348,57 +1409,41 @@ class TrainSet {
         check_lds(lds, gen_ ? (const void*)k_train_tile<2, true> : (const void*)k_train_tile<2, false>);
         if (grad) check_lds(flds, gen_ ? (const void*)k_train_force_tile<true> : (const void*)k_train_force_tile<false>);
         const double* Wm = (const double*)owner_.d_w64.p;
-        if (grad) {
-            d_grad_.reserve(8 * (size_t)total());
-            HIPCHK(hipMemsetAsync(d_grad_.p, 0, 8 * (size_t)total(), st));
-        }
-        err[0] = err[1] = err[2] = 0.0;
         int k0 = 0;
         while (k0 < nbatch) {
             // a chunk of whole structures, at most ~128k atoms (one structure if larger)
             int k1 = k0;
             int64_t atoms = 0;
             while (k1 < nbatch && (k1 == k0 || atoms + natoms_[batch[k1]] <= (1 << 17))) atoms += natoms_[batch[k1++]];
-            const int nb = k1 - k0;
-            std::vector<nnp_structure> cs(nb);
-            std::vector<int> bstart(nb + 1, 0);
-            std::vector<int64_t> fstart(nb);
-            std::vector<double> eb(nb);
-            for (int b = 0; b < nb; ++b) {
-                const int sb = batch[k0 + b];
-                cs[b].natoms = natoms_[sb];
-                cs[b].type = types_.data() + aoff_[sb];
-                cs[b].pos = hpos_.data() + 3 * aoff_[sb];
-                cs[b].cell = hopen_[sb] ? nullptr : hcell_.data() + 9 * (size_t)sb;
-                bstart[b + 1] = bstart[b] + natoms_[sb];
-                fstart[b] = aoff_[sb];
-                eb[b] = eref_[sb];
-            }
+            const int nb = k1 - k0, n = (int)atoms;
             // The structures do not move between calls: a chunk seen before keeps its neighbour
-            // rows and descriptors in a workspace of its own (up to the model's train_cache_atoms
+            // rows, descriptors and tiles in a workspace of its own (up to the model's train_cache_atoms
             // option in all, 2^20 by default);
             // otherwise the scratch workspace builds them.
             std::vector<int> key(batch + k0, batch + k1);
             key.push_back(all_images ? 1 : 0);
-            Engine* Ep = nullptr;
+            Chunk* C = nullptr;
             for (auto& c : fcache_)
-                if (c.first == key) Ep = c.second.get();
-            if (!Ep) {
+                if (c->key == key) C = c.get();
+            if (!C) {
+                HIPCHK(hipStreamSynchronize(st));  // (the scratch workspace's last chunk)
+                auto fresh = std::make_unique<Chunk>();
                 const bool keep = fcache_atoms_ + atoms <= owner_.train_cache_atoms;
+                if (keep) fresh->own = std::make_unique<Engine>(owner_, 1002);
+                build_chunk(*fresh, batch + k0, nb, all_images, keep ? *fresh->own : *ws_, st);
                 if (keep) {
-                    fcache_.emplace_back(key, std::make_unique<Engine>(owner_, 1002));
+                    fresh->key = key;
+                    fcache_.push_back(std::move(fresh));
                     fcache_atoms_ += atoms;
-                    Ep = fcache_.back().second.get();
+                    C = fcache_.back().get();
                 } else {
-                    Ep = ws_.get();
+                    scratch_ = std::move(fresh);
+                    C = scratch_.get();
                 }
-                Engine& B = *Ep;
-                B.upload(cs);
-                B.build_neighbors(all_images);
-                B.descriptors<double>();
-                if (keep) HIPCHK(hipStreamSynchronize(B.stream));
             }
-            Engine& E = *Ep;
+            Engine& E = C->own ? *C->own : *ws_;
+            const Tiles& tl = C->tl;
+            const TileArrays& ta = C->ta;
             // the chunk's kernels, the workspace's force kernels included, run in order on st
             struct OnStream {
                 Engine& e;
@@ -1406,59 +1451,42 @@ class TrainSet {
                 OnStream(Engine& w, hipStream_t s) : e(w), own(w.stream) { e.stream = s; }
                 ~OnStream() { e.stream = own; }
             } on_stream(E, st);
-            const int n = bstart[nb];
-            // species tiles over the workspace atoms (source row = slot = workspace index)
-            std::vector<std::vector<int>> atom_s(T_), slot_s(T_), struct_s(T_);
-            for (int b = 0; b < nb; ++b)
-                for (int i = bstart[b]; i < bstart[b + 1]; ++i) {
-                    const int t = types_[aoff_[batch[k0 + b]] + (i - bstart[b])];
-                    atom_s[t].push_back(i);
-                    slot_s[t].push_back(i);
-                    struct_s[t].push_back(b);
-                }
-            tiles_key_.clear();  // the energy path's cached tiles are overwritten
-            const Tiles tl = make_tiles(atom_s, slot_s, struct_s, st);
-            d_bstart_.reserve(4 * (size_t)(nb + 1));
-            d_fstart_.reserve(8 * (size_t)nb);
-            d_eref_.reserve(8 * (size_t)nb);
             d_out_.reserve(8 * (size_t)n);
             d_dcdo_.reserve(8 * (size_t)nb);
-            d_loss_.reserve(8 * (size_t)nb);
-            d_dE2_.reserve(8 * (size_t)nb);
-            d_f2_.reserve(8 * (size_t)nb);
             d_gF_.reserve(8 * 3 * (size_t)n);
             d_V_.reserve(8 * (size_t)n * ldg_);
             E.d_dEdG.reserve(8 * (size_t)n * ldg_);
-            HIPCHK(hipMemcpyAsync(d_bstart_.p, bstart.data(), 4 * (size_t)(nb + 1), hipMemcpyHostToDevice, st));
-            HIPCHK(hipMemcpyAsync(d_fstart_.p, fstart.data(), 8 * (size_t)nb, hipMemcpyHostToDevice, st));
-            HIPCHK(hipMemcpyAsync(d_eref_.p, eb.data(), 8 * (size_t)nb, hipMemcpyHostToDevice, st));
             // outputs and dout/dG at x, then the forces by the model's force kernels
             if (tl.tiles > 0)
                 launch_tile<2>(gen_, dim3(tl.tiles), lds, st,
                                    (const TrainPlan*)d_plan_.p, Wm, (const double*)d_par_.p, tl.tt, 0,
-                                   (const int*)d_batom_.p, (const int*)d_bslot_.p, (const int*)d_bstruct_.p,
+                                   (const int*)ta.atom.p, (const int*)ta.slot.p, (const int*)ta.strct.p,
                                    (const double*)E.d_G.p, ldg_, (double*)d_out_.p, nullptr, nullptr,
                                    (double*)E.d_dEdG.p);
             HIPCHK(hipGetLastError());
             E.force_terms<double>();
             // reactions: the missed-reaction counter is cleared here (a cached chunk has no
-            // neighbour launch in this call); a miss switches the chunk's workspace to receiver rows
-            HIPCHK(hipMemsetAsync((int*)E.d_maxcnt.p + 1, 0, 4, st));
+            // neighbour launch in this call); a miss switches the chunk's workspace to receiver rows.  What is
+            // missed depends on the rows alone, so a kept chunk is checked once.
+            if (!C->settled) HIPCHK(hipMemsetAsync((int*)E.d_maxcnt.p + 1, 0, 4, st));
             E.assemble<double>();
-            for (int attempt = 0;; ++attempt) {
+            for (int attempt = 0; !C->settled; ++attempt) {
                 int c[4] = {0, 0, 0, 0};
                 HIPCHK(hipMemcpyAsync(c, E.d_maxcnt.p, 16, hipMemcpyDeviceToHost, st));
                 HIPCHK(hipStreamSynchronize(st));
-                if (!E.reactions_redo(c)) break;
+                if (!E.reactions_redo(c)) {
+                    C->settled = true;
+                    break;
+                }
                 if (attempt == 3) throw std::runtime_error("force assembly: receiver rows did not converge");
                 E.assemble<double>();
             }
             hipLaunchKernelGGL(k_train_struct, dim3(nb), dim3(256), 0, st, (const double*)d_out_.p,
-                               (const int*)d_bstart_.p, (const double*)d_eref_.p, loss, delta, (double*)d_dcdo_.p,
-                               (double*)d_loss_.p, (double*)d_dE2_.p);
+                               (const int*)ta.bstart.p, (const double*)ta.eref.p, loss, delta, (double*)d_dcdo_.p,
+                               res(0, nbatch) + k0, res(1, nbatch) + k0);
             hipLaunchKernelGGL(k_train_fresid, dim3(nb), dim3(256), 0, st, (const double*)E.d_F.p,
-                               (const double*)d_fref_.p, (const int*)d_bstart_.p, (const int64_t*)d_fstart_.p, beta,
-                               (double*)d_gF_.p, (double*)d_f2_.p);
+                               (const double*)d_fref_.p, (const int*)ta.bstart.p, (const int64_t*)ta.fstart.p, beta,
+                               (double*)d_gF_.p, res(2, nbatch) + k0);
             HIPCHK(hipGetLastError());
             if (grad) {
                 HIPCHK(launch_symm_jvp(E.shape, owner_.pb.plan.generic, (const DevPlan*)E.d_plan.p,
@@ -1470,7 +1498,7 @@ class TrainSet {
                 sum_tiles(tl, st, [&](const TrainTiles& tc, int c0, int c1) {
                     const TrainPlan* tpp = (const TrainPlan*)d_plan_.p;
                     const double* par = (const double*)d_par_.p;
-                    const int *ba = (const int*)d_batom_.p, *bs = (const int*)d_bstruct_.p;
+                    const int *ba = (const int*)ta.atom.p, *bs = (const int*)ta.strct.p;
                     const double *Gp = (const double*)E.d_G.p, *Vp = (const double*)d_V_.p, *dc = (const double*)d_dcdo_.p;
                     double* pp = (double*)d_partial_.p;
                     if (gen_)
@@ -1481,22 +1509,53 @@ class TrainSet {
                                            par, tc, c0, ba, bs, Gp, Vp, ldg_, dc, pp);
                 });
             }
-            std::vector<double> lv(nb), e2(nb), f2(nb);
-            HIPCHK(hipMemcpyAsync(lv.data(), d_loss_.p, 8 * (size_t)nb, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipMemcpyAsync(e2.data(), d_dE2_.p, 8 * (size_t)nb, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipMemcpyAsync(f2.data(), d_f2_.p, 8 * (size_t)nb, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
-            for (int b = 0; b < nb; ++b) {
-                err[0] += lv[b] + 0.5 * beta * f2[b];
-                err[1] += e2[b];
-                err[2] += f2[b];
-            }
             k0 = k1;
         }
-        if (grad) {
-            HIPCHK(hipMemcpyAsync(grad, d_grad_.p, 8 * (size_t)total(), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+        const double* lv = fetch_results(nbatch, 3, grad, st);
+        const double *e2 = lv + nbatch, *f2 = e2 + nbatch;
+        err[0] = err[1] = err[2] = 0.0;
+        for (int b = 0; b < nbatch; ++b) {
+            err[0] += lv[b] + 0.5 * beta * f2[b];
+            err[1] += e2[b];
+            err[2] += f2[b];
         }
+    }
+
+    // The chunk of nb structures: its neighbour rows and descriptors in B, its tiles and reference values on st.
+    void build_chunk(Chunk& C, const int* batch, int nb, bool all_images, Engine& B, hipStream_t st) {
+        std::vector<nnp_structure> cs(nb);
+        std::vector<int> bstart(nb + 1, 0);
+        std::vector<int64_t> fstart(nb);
+        std::vector<double> eb(nb);
+        // species tiles over the workspace atoms (source row = slot = workspace index)
+        std::vector<std::vector<int>> atom_s(T_), struct_s(T_);
+        for (int b = 0; b < nb; ++b) {
+            const int sb = batch[b];
+            cs[b].natoms = natoms_[sb];
+            cs[b].type = types_.data() + aoff_[sb];
+            cs[b].pos = hpos_.data() + 3 * aoff_[sb];
+            cs[b].cell = hopen_[sb] ? nullptr : hcell_.data() + 9 * (size_t)sb;
+            bstart[b + 1] = bstart[b] + natoms_[sb];
+            fstart[b] = aoff_[sb];
+            eb[b] = eref_[sb];
+            for (int i = 0; i < natoms_[sb]; ++i) {
+                const int t = types_[aoff_[sb] + i];
+                atom_s[t].push_back(bstart[b] + i);
+                struct_s[t].push_back(b);
+            }
+        }
+        B.upload(cs);
+        B.build_neighbors(all_images);
+        B.descriptors<double>();
+        C.tl = make_tiles(atom_s, atom_s, struct_s, st, C.ta);
+        C.ta.bstart.reserve(4 * (size_t)(nb + 1));
+        C.ta.fstart.reserve(8 * (size_t)nb);
+        C.ta.eref.reserve(8 * (size_t)nb);
+        HIPCHK(hipMemcpyAsync(C.ta.bstart.p, bstart.data(), 4 * (size_t)(nb + 1), hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(C.ta.fstart.p, fstart.data(), 8 * (size_t)nb, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(C.ta.eref.p, eb.data(), 8 * (size_t)nb, hipMemcpyHostToDevice, st));
+        HIPCHK(hipStreamSynchronize(st));  // the host vectors go out of scope
+        if (B.stream != st) HIPCHK(hipStreamSynchronize(B.stream));
     }
 
   private:
@@ -1507,10 +1566,11 @@ class TrainSet {
     std::vector<int64_t> goff_;
     std::vector<int> natoms_, types_;
     std::vector<int64_t> aoff_;
-    std::vector<double> eref_, hpar_;
+    std::vector<double> eref_;
     hipStream_t stream_ = nullptr;
-    DevMem d_plan_, d_goff_, d_G_, d_par_, d_batom_, d_bslot_, d_bstruct_, d_bstart_, d_eref_, d_out_, d_dcdo_, d_loss_,
-        d_dE2_, d_grad_, d_partial_, d_grp_, d_fref_, d_fstart_, d_f2_, d_gF_, d_V_;
+    DevMem d_plan_, d_goff_, d_G_, d_par_, d_out_, d_dcdo_, d_res_, d_partial_, d_grp_, d_fref_, d_gF_, d_V_;
+    HostPinned h_io_;
+    bool grad_started_ = false;  // the call's gradient holds its first rows
     std::vector<double> hpos_, hcell_;
     std::vector<char> hopen_;
     std::vector<int> hbatom_, hbslot_, hbstruct_;
@@ -1520,6 +1580,8 @@ class TrainSet {
     // tiles of the last energy-training call (batch + mode) and whether they are single-structure
     std::vector<int> tiles_key_;
     Tiles tiles_;
+    TileArrays ta_;
+    int natoms_batch_ = 0;
     bool one_pass_ = false;
     DevMem d_tstruct_;
     bool grouped_ = false;  // the tiles' rows by k_train_group
@@ -1528,7 +1590,8 @@ class TrainSet {
     DevMem d_gtile_;
     std::unique_ptr<Engine> ws_;  // workspace of the force passes
     // workspaces that keep the neighbour rows and descriptors of force-training chunks
-    std::vector<std::pair<std::vector<int>, std::unique_ptr<Engine>>> fcache_;
+    std::vector<std::unique_ptr<Chunk>> fcache_;
+    std::unique_ptr<Chunk> scratch_;
     int64_t fcache_atoms_ = 0;
 };
 
