@@ -63,15 +63,18 @@ __device__ __forceinline__ void cell_diff(const DevStruc& s, double dx, double d
     }
 }
 
+__device__ __forceinline__ void image_vec(const DevStruc& s, int a, int b, int c, double& x, double& y, double& z) {
+    x = (double)a * s.Rv[0] + (double)b * s.Rv[3] + (double)c * s.Rv[6];
+    y = (double)a * s.Rv[1] + (double)b * s.Rv[4] + (double)c * s.Rv[7];
+    z = (double)a * s.Rv[2] + (double)b * s.Rv[5] + (double)c * s.Rv[8];
+}
 // image vector R_n = a Rv0 + b Rv1 + c Rv2 for linear index n (neighbor.cpp:87-95)
 __device__ __forceinline__ void image_vec(const DevStruc& s, int n, double& x, double& y, double& z) {
     const int w2 = 2 * s.shell[2] + 1, w1 = 2 * s.shell[1] + 1;
     const int c = n % w2 - s.shell[2];
     const int b = (n / w2) % w1 - s.shell[1];
     const int a = n / (w2 * w1) - s.shell[0];
-    x = (double)a * s.Rv[0] + (double)b * s.Rv[3] + (double)c * s.Rv[6];
-    y = (double)a * s.Rv[1] + (double)b * s.Rv[4] + (double)c * s.Rv[7];
-    z = (double)a * s.Rv[2] + (double)b * s.Rv[5] + (double)c * s.Rv[8];
+    image_vec(s, a, b, c, x, y, z);
 }
 
 // Exclusive prefix sum over the wavefront in six DPP adds: shifts by 1, 2, 4 and 8 inside each row of 16
@@ -155,87 +158,148 @@ __device__ __forceinline__ void clear_counters(const PassCounters& pc) {
 }
 
 // ------------------------------------------------------------------ all-pairs search
-__global__ __launch_bounds__(kWave) void k_neigh_allpairs(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
+// One centre a block.  Wavefront w takes the atoms 64 (4 r + w) to 64 (4 r + w) + 63 of round r, one a lane: difference
+// vector and box of images within reach.  The images of all of them are then spread over the lanes in (atom, image)
+// order, twice: to count what each atom keeps and find its nearest image, and to write the entries, whose places the
+// counts give (scans inside the wavefront, the wavefronts' totals through LDS), next to each other.  A lane that walks
+// its own atom's images instead costs the wavefront the longest walk, in a chain of FP64 latencies: about 110
+// images are within reach of a centre, all of them on two lanes of a two-atom cell (20 uneven cells of up to 512 atoms:
+// 24.5 us, now 9.2; one of 64 atoms: 9.7 us, now 8.2; four wavefronts a centre instead of one make no difference while
+// each lane walks its own images).
+constexpr int kPairWaves = 4;
+struct PairChunk {  // a wavefront's 64 atoms
+    double b[3][kWave];              // difference vector
+    unsigned long long mind[kWave];  // bits of the smallest distance
+    int off[kWave], lo[3][kWave], ext[2][kWave];  // first image, box of images (lowest indexes, last two extents)
+    int type[kWave], kept[kWave], minn[kWave];
+};
+__global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                           const double* __restrict__ pos, const int* __restrict__ type,
                                                           const int* __restrict__ centres, double rc2, int maxp,
                                                           int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                           int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
                                                           unsigned short* __restrict__ row_tab, unsigned short* __restrict__ nbr_key, PassCounters pc) {
     clear_counters(pc);
+    __shared__ PairChunk chunk[kPairWaves];
+    __shared__ int wtot[2][kPairWaves];
     const int i = centres[blockIdx.x];
     const DevStruc& s = S[atom_struc[i]];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool one = s.natoms <= kWave;  // (uniform)
+    if (one && w > 0) return;
     const int li = i - s.atom0;
     const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
     const int64_t row = (int64_t)i * maxp;
     const int tw = row_tab_width(s.natoms);
+    PairChunk& L = chunk[w];
+    const int w1 = 2 * s.shell[1] + 1, w2 = 2 * s.shell[2] + 1;
+    const bool periodic = s.periodic;
+    const double fro = s.fro;
+    const auto ordered = [] {  // LDS writes of some lanes before reads of others of the same wavefront
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+    };
     int written = 0;
-    for (int j0 = 0; j0 < s.natoms; j0 += kWave) {
-        const int j = j0 + lane;
+    for (int j0 = 0, buf = 0; j0 < s.natoms; j0 += kWave * kPairWaves, buf ^= 1) {
+        const int jw = j0 + w * kWave, j = jw + lane;
         const bool valid = j < s.natoms;
         double bx = 0, by = 0, bz = 0;
-        int tj = 0;
-        int mine = 0;
-        double mind = s.fro;
-        int minn = -1;
+        // images of this j that can be within rc (open structures: the single image 0)
+        ImgRange g{{0, 0, 0}, {-1, -1, -1}};
         if (valid) {
             const int gj = s.atom0 + j;
-            tj = type[gj];
+            L.type[lane] = type[gj];
             const double dx = xi - pos[3 * gj], dy = yi - pos[3 * gj + 1], dz = zi - pos[3 * gj + 2];
-            if (s.periodic) {
+            if (periodic) {
                 cell_diff(s, dx, dy, dz, bx, by, bz);
+                g = img_range(s, bx, by, bz);
             } else {
                 bx = dx;
                 by = dy;
                 bz = dz;
+                g = ImgRange{{0, 0, 0}, {0, 0, 0}};
             }
         }
-        // images of this j that can be within rc (open structures: the single image 0)
-        ImgRange g{{0, 0, 0}, {-1, -1, -1}};
-        if (valid) g = s.periodic ? img_range(s, bx, by, bz) : ImgRange{{0, 0, 0}, {0, 0, 0}};
-        const int w1 = 2 * s.shell[1] + 1, w2 = 2 * s.shell[2] + 1;
-        for (int a = g.lo[0]; a <= g.hi[0]; ++a)
-            for (int b = g.lo[1]; b <= g.hi[1]; ++b)
-                for (int c = g.lo[2]; c <= g.hi[2]; ++c) {
-                    const int n = ((a + s.shell[0]) * w1 + (b + s.shell[1])) * w2 + (c + s.shell[2]);
-                    double ix = 0, iy = 0, iz = 0;
-                    if (s.periodic) image_vec(s, n, ix, iy, iz);
-                    const double rx = bx - ix, ry = by - iy, rz = bz - iz;
-                    const double d2 = rx * rx + ry * ry + rz * rz;
-                    const bool keep = (j != li) ? (d2 <= rc2) : (1e-6 < d2 && d2 <= rc2);
-                    if (keep) {
-                        ++mine;
-                        const double d = sqrt(d2);
-                        if (j != li && s.periodic && d < mind) {
-                            mind = d;
-                            minn = n;
-                        }
-                    }
-                }
+        const int e0 = max(0, g.hi[0] - g.lo[0] + 1), e1 = max(0, g.hi[1] - g.lo[1] + 1), e2 = max(0, g.hi[2] - g.lo[2] + 1);
+        int images;  // of the wavefront's atoms
+        L.off[lane] = wave_excl_scan(e0 * e1 * e2, lane, images);
+        L.b[0][lane] = bx;
+        L.b[1][lane] = by;
+        L.b[2][lane] = bz;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) L.lo[q][lane] = g.lo[q];
+        L.ext[0][lane] = e1;
+        L.ext[1][lane] = e2;
+        L.kept[lane] = 0;
+        L.mind[lane] = __double_as_longlong(fro);  // (distances are positive: their bits order as they do)
+        L.minn[lane] = INT_MAX;
+        ordered();
+        // image q of the wavefront's: its atom (the last whose images begin at or before q), offset and vector
+        const auto image = [&](int q, int& k, int& n, double& rx, double& ry, double& rz) {
+            k = 0;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+                if (L.off[k + o] <= q) k += o;
+            const int t = q - L.off[k], f1 = L.ext[0][k], f2 = L.ext[1][k];
+            const int u = t / f2, v = u / f1;
+            const int a = L.lo[0][k] + v, b = L.lo[1][k] + u - v * f1, c = L.lo[2][k] + t - u * f2;
+            n = ((a + s.shell[0]) * w1 + (b + s.shell[1])) * w2 + (c + s.shell[2]);
+            double ix = 0, iy = 0, iz = 0;
+            if (periodic) image_vec(s, a, b, c, ix, iy, iz);
+            rx = L.b[0][k] - ix;
+            ry = L.b[1][k] - iy;
+            rz = L.b[2][k] - iz;
+            const double d2 = rx * rx + ry * ry + rz * rz;
+            return d2 <= rc2 && (jw + k != li || 1e-6 < d2) ? d2 : -1.0;  // -1: not kept
+        };
+        for (int q = lane; q < images; q += kWave) {
+            int k, n;
+            double rx, ry, rz;
+            const double d2 = image(q, k, n, rx, ry, rz);
+            if (d2 < 0) continue;
+            atomicAdd(&L.kept[k], 1);
+            if (periodic && jw + k != li) atomicMin(&L.mind[k], (unsigned long long)__double_as_longlong(sqrt(d2)));
+        }
+        ordered();
+        const int mine = L.kept[lane];
         int tot;
         int at = written + wave_excl_scan(mine, lane, tot);
+        if (!one) {
+            if (lane == 0) wtot[buf][w] = tot;
+            __syncthreads();  // (the other buffer's readers passed the barrier before)
+            tot = 0;
+#pragma unroll
+            for (int v = 0; v < kPairWaves; ++v) {
+                const int c = wtot[buf][v];
+                if (v < w) at += c;
+                tot += c;
+            }
+        }
         // the row's index table: atom j opens slot j / width when it is the slot's first
         if (valid && j % tw == 0) row_tab[(int64_t)i * kRowTab + j / tw] = (unsigned short)min(at, maxp);
-        if (mine > 0) {
-            for (int a = g.lo[0]; a <= g.hi[0]; ++a)
-                for (int b = g.lo[1]; b <= g.hi[1]; ++b)
-                    for (int c = g.lo[2]; c <= g.hi[2]; ++c) {
-                        const int n = ((a + s.shell[0]) * w1 + (b + s.shell[1])) * w2 + (c + s.shell[2]);
-                        double ix = 0, iy = 0, iz = 0;
-                        if (s.periodic) image_vec(s, n, ix, iy, iz);
-                        const double rx = bx - ix, ry = by - iy, rz = bz - iz;
-                        const double d2 = rx * rx + ry * ry + rz * rz;
-                        const bool keep = (j != li) ? (d2 <= rc2) : (1e-6 < d2 && d2 <= rc2);
-                        if (keep) {
-                            if (at < maxp)
-                                put_entry(row + at, j, n, tj, n == minn, rx, ry, rz, sqrt(d2), nbr_j, nbr_key, nbr_meta,
-                                          nbr_r);
-                            ++at;
-                        }
-                    }
+        int put = __builtin_amdgcn_readfirstlane(at);  // (lane 0's: the wavefront's first entry)
+        for (int q0 = 0; q0 < images; q0 += kWave) {
+            int k = 0, n = 0;
+            double rx = 0, ry = 0, rz = 0, d2 = -1.0;
+            if (q0 + lane < images) d2 = image(q0 + lane, k, n, rx, ry, rz);
+            const bool keep = d2 >= 0;
+            const double d = keep ? sqrt(d2) : 0.0;
+            // the nearest image, the first of equally near ones (images of an atom come in increasing n)
+            const bool near = keep && periodic && jw + k != li && d < fro &&
+                              (unsigned long long)__double_as_longlong(d) == L.mind[k];
+            if (near) atomicMin(&L.minn[k], n);
+            ordered();
+            const uint64_t mask = __ballot(keep);
+            const int e = put + __popcll(mask & ((1ull << lane) - 1));
+            if (keep && e < maxp)
+                put_entry(row + e, jw + k, n, L.type[k], near && n == L.minn[k], rx, ry, rz, d, nbr_j, nbr_key, nbr_meta,
+                          nbr_r);
+            put += __popcll(mask);
         }
+        ordered();  // (before the next round's atoms are staged)
         written += tot;
     }
+    if (w > 0) return;
     const int q0 = (s.natoms + tw - 1) / tw;  // slots past the last atom
     if (lane >= q0 && lane < kRowTab) row_tab[(int64_t)i * kRowTab + lane] = (unsigned short)min(written, maxp);
     if (lane == 0) {
@@ -858,7 +922,7 @@ hipError_t launch_neighbors(const NeighborArgs& a, hipStream_t st) {
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.npair > 0) {
-        hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave), 0, st, a.S, a.atom_struc, a.pos, a.type,
+        hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave * kPairWaves), 0, st, a.S, a.atom_struc, a.pos, a.type,
                            a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
