@@ -42,19 +42,9 @@ constexpr double kBoltzmann = 8.617333262e-5;  // eV / K
 // math/special.hpp:46-47, mod(x, 0, 1)
 __device__ __forceinline__ double mod01(double x) { return fmod(fmod(x, 1.0) + 1.0, 1.0); }
 
-// The first half kick and the drift of a step in one launch: v += c_i F with c_i = dt / (2 m_i)
-// (A/fs per eV/A), then x += v dt and, with wrap, back into the cell (Cell::returnToCell,
-// struc/cell.cpp:84-94).
-__global__ __launch_bounds__(256) void k_kick_drift(double* __restrict__ x, double* __restrict__ v,
-                                                   const double* __restrict__ F, const double* __restrict__ c, double dt,
-                                                   int n, const DevStruc* __restrict__ S, int wrap) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const double ci = c[i];
-    const double vx = v[3 * i] + ci * F[3 * i], vy = v[3 * i + 1] + ci * F[3 * i + 1], vz = v[3 * i + 2] + ci * F[3 * i + 2];
-    v[3 * i] = vx;
-    v[3 * i + 1] = vy;
-    v[3 * i + 2] = vz;
+// Atom i moved by v dt, returned to the cell with wrap.
+__device__ __forceinline__ void drift(double* __restrict__ x, int i, double vx, double vy, double vz, double dt,
+                                      const DevStruc* __restrict__ S, int wrap) {
     double px = x[3 * i] + vx * dt, py = x[3 * i + 1] + vy * dt, pz = x[3 * i + 2] + vz * dt;
     const DevStruc& s = S[0];
     if (wrap && s.periodic) {
@@ -68,6 +58,43 @@ __global__ __launch_bounds__(256) void k_kick_drift(double* __restrict__ x, doub
     x[3 * i] = px;
     x[3 * i + 1] = py;
     x[3 * i + 2] = pz;
+}
+
+// The first half kick and the drift of a step in one launch: v += c_i F with c_i = dt / (2 m_i)
+// (A/fs per eV/A), then x += v dt and, with wrap, back into the cell (Cell::returnToCell,
+// struc/cell.cpp:84-94).
+__global__ __launch_bounds__(256) void k_kick_drift(double* __restrict__ x, double* __restrict__ v,
+                                                   const double* __restrict__ F, const double* __restrict__ c, double dt,
+                                                   int n, const DevStruc* __restrict__ S, int wrap) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const double ci = c[i];
+    const double vx = v[3 * i] + ci * F[3 * i], vy = v[3 * i + 1] + ci * F[3 * i + 1], vz = v[3 * i + 2] + ci * F[3 * i + 2];
+    v[3 * i] = vx;
+    v[3 * i + 1] = vy;
+    v[3 * i + 2] = vz;
+    drift(x, i, vx, vy, vz, dt, S, wrap);
+}
+
+// Between two steps of a block: the second half kick of one (rounded as by itself), the first half kick and drift of the
+// next, and the pass's maxima; the kinetic energy of a step that the block goes on from has no reader.  4096
+// atoms: 5.0 us for k_kick_kinetic (a grid-wide sum) and 4.5 for k_kick_drift, 4.7 us here, and one launch less.
+__global__ __launch_bounds__(256) void k_kick_step(double* __restrict__ x, double* __restrict__ v,
+                                                   const double* __restrict__ F, const double* __restrict__ c, double dt,
+                                                   int n, const DevStruc* __restrict__ S, int wrap,
+                                                   const int* __restrict__ maxcnt, int* __restrict__ maxseen) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 3 && maxcnt[i] > maxseen[i]) maxseen[i] = maxcnt[i];
+    if (i >= n) return;
+    const double ci = c[i], fx = F[3 * i], fy = F[3 * i + 1], fz = F[3 * i + 2];
+    double vx = v[3 * i] + ci * fx, vy = v[3 * i + 1] + ci * fy, vz = v[3 * i + 2] + ci * fz;
+    vx = vx + ci * fx;
+    vy = vy + ci * fy;
+    vz = vz + ci * fz;
+    v[3 * i] = vx;
+    v[3 * i + 1] = vy;
+    v[3 * i + 2] = vz;
+    drift(x, i, vx, vy, vz, dt, S, wrap);
 }
 
 // The second half kick and the kinetic energy in one launch: each block kicks its 256 atoms and
@@ -316,12 +343,16 @@ struct Md {
         HIPCHK(hipGetLastError());
     }
 
-    void enqueue_step(int kind) {
+    // One step; inside a block it begins where the last one ended (begun), and ends with the next one's beginning
+    // (next: its kind).
+    void enqueue_step(int kind, bool begun = false, int next = -1) {
         Engine& E = *eng;
         const int nb = (n + 255) / 256;
-        hipLaunchKernelGGL(k_kick_drift, dim3(nb), dim3(256), 0, E.stream, pos(), (double*)d_vel.p, force(),
-                           (const double*)d_half.p, dt, n, (const DevStruc*)E.d_strucs.p, kind == 2 ? 0 : 1);
-        HIPCHK(hipGetLastError());
+        if (!begun) {
+            hipLaunchKernelGGL(k_kick_drift, dim3(nb), dim3(256), 0, E.stream, pos(), (double*)d_vel.p, force(),
+                               (const double*)d_half.p, dt, n, (const DevStruc*)E.d_strucs.p, kind == 2 ? 0 : 1);
+            HIPCHK(hipGetLastError());
+        }
         if (kind == 0) {
             E.enqueue_pass(flags);
         } else {
@@ -334,6 +365,13 @@ struct Md {
             }
             refresh(kind == 1 ? 1 : 0);
             E.enqueue_pass(flags, true);
+        }
+        if (next >= 0) {
+            hipLaunchKernelGGL(k_kick_step, dim3(nb), dim3(256), 0, E.stream, pos(), (double*)d_vel.p, force(),
+                               (const double*)d_half.p, dt, n, (const DevStruc*)E.d_strucs.p, next == 2 ? 0 : 1,
+                               (const int*)E.d_maxcnt.p, (int*)d_maxseen.p);
+            HIPCHK(hipGetLastError());
+            return;
         }
         hipLaunchKernelGGL(k_kick_kinetic, dim3(nb), dim3(256), 0, E.stream, (double*)d_vel.p, force(),
                            (const double*)d_half.p, (const double*)d_mass.p, n, (double*)d_bsum.p,
@@ -375,7 +413,8 @@ struct Md {
         Engine& E = *eng;
         if (!execb)
             capture(graphb, execb, [&]() {
-                for (int q = 0; q < len; ++q) enqueue_step(use_list ? (q == 0 ? 1 : 2) : 0);
+                for (int q = 0; q < len; ++q)
+                    enqueue_step(use_list ? (q == 0 ? 1 : 2) : 0, q > 0, q + 1 == len ? -1 : (use_list ? 2 : 0));
             });
         HIPCHK(hipGraphLaunch(execb, E.stream));
     }
