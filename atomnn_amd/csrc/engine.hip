@@ -430,8 +430,7 @@ Engine::Engine(const Engine& o, int) : host(o.host), pb(o.pb), shape(o.shape) {
 size_t Engine::workspace_bytes() const {
     size_t b = 0;
     for (const DevMem* m : {&d_up, &d_cnt, &d_nbrj, &d_meta, &d_nbrr, &d_maxcnt, &d_abin, &d_bcount, &d_bstart,
-                            &d_brank, &d_bpos, &d_rowtab, &d_key, &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount,
-                            &d_rlist, &d_out, &d_mom})
+                            &d_G, &d_dEdG, &d_X, &d_eatom, &d_F, &d_E, &d_sstart, &d_rcount, &d_rlist, &d_out, &d_mom})
         b += m->cap;
     return b;
 }
@@ -704,18 +703,32 @@ void Engine::build_neighbors(bool all_images) {
         const size_t ent = (size_t)ntot * maxp;
         if (ent >= (size_t)1 << 31) throw std::invalid_argument("batch too large for 32-bit entry indices");
         d_cnt.reserve((size_t)ntot * 4);
-        d_nbrj.reserve(ent * 4);
+        // (the keys and index tables lie behind the indices: a device allocation costs tens of us)
+        const size_t o_key = (ent * 4 + 255) & ~size_t(255), b_key = ent * sizeof(unsigned short),
+                     o_tab = (o_key + b_key + 255) & ~size_t(255), b_tab = (size_t)ntot * kRowTab * sizeof(unsigned short);
+        d_nbrj.reserve(d_nbrj.bound ? ent * 4 : o_tab + b_tab);
+        if (d_nbrj.bound) {
+            d_rowtab.reserve(b_tab);
+            d_key.reserve(b_key);
+        } else {
+            d_key.bind((char*)d_nbrj.p + o_key, b_key);
+            d_rowtab.bind((char*)d_nbrj.p + o_tab, b_tab);
+        }
         d_meta.reserve(ent * 4);
         d_nbrr.reserve(ent * sizeof(double4));
-        d_rowtab.reserve((size_t)ntot * kRowTab * sizeof(unsigned short));
-        d_key.reserve(ent * sizeof(unsigned short));
         if (!d_maxcnt.p) {  // counters the current mode does not write are read back as zero
             d_maxcnt.reserve(64);
             HIPCHK(hipMemsetAsync(d_maxcnt.p, 0, 64, stream));
         }
         d_work.reserve(64);
         if (nbins > 0) {
-            d_abin.reserve((size_t)ntot * 4);
+            // (the ranks and bin-ordered positions behind the bins)
+            const size_t o_pos = ((size_t)ntot * 8 + 255) & ~size_t(255), b_pos = (size_t)ntot * sizeof(float4);
+            d_abin.reserve(d_abin.bound ? (size_t)ntot * 4 : o_pos + b_pos);
+            if (!d_abin.bound) {
+                d_brank.bind((char*)d_abin.p + (size_t)ntot * 4, (size_t)ntot * 4);
+                d_bpos.bind((char*)d_abin.p + o_pos, b_pos);
+            }
             const size_t count_cap = d_bcount.cap;
             d_bcount.reserve((size_t)nbins * 4);
             // the bin counters are zero between passes: the scan clears what it has read

@@ -193,7 +193,7 @@ class Server {
             // batch from empty buffers (the device may still be short of memory)
             if (held > lane_budget_ || status == NNP_ENOMEM) {
                 (void)hipStreamSynchronize(E.stream);
-                for (DevMem* m : {&E.d_nbrj, &E.d_key, &E.d_meta, &E.d_nbrr, &E.d_X, &E.d_G, &E.d_dEdG, &E.d_mom}) m->release();
+                for (DevMem* m : {&E.d_nbrj, &E.d_key, &E.d_rowtab, &E.d_meta, &E.d_nbrr, &E.d_X, &E.d_G, &E.d_dEdG, &E.d_mom}) m->release();
                 E.mom_fresh = 0;
             }
             const double t = steady_now();
