@@ -158,34 +158,38 @@ __device__ __forceinline__ void clear_counters(const PassCounters& pc) {
 }
 
 // ------------------------------------------------------------------ all-pairs search
-// One centre a block.  Wavefront w takes the atoms 64 (4 r + w) to 64 (4 r + w) + 63 of round r, one a lane: difference
-// vector and box of images within reach.  The images of all of them are then spread over the lanes in (atom, image)
-// order, twice: to count what each atom keeps and find its nearest image, and to write the entries, whose places the
-// counts give (scans inside the wavefront, the wavefronts' totals through LDS), next to each other.  A lane that walks
-// its own atom's images instead costs the wavefront the longest walk, in a chain of FP64 latencies: about 110
-// images are within reach of a centre, all of them on two lanes of a two-atom cell (20 uneven cells of up to 512 atoms:
-// 24.5 us, now 9.2; one of 64 atoms: 9.7 us, now 8.2; four wavefronts a centre instead of one make no difference while
-// each lane walks its own images).
-constexpr int kPairWaves = 4;
+// One centre a block.  Wavefront w takes the atoms 64 (W r + w) to 64 (W r + w) + 63 of round r, one a lane: difference
+// vector and box of images within reach.  Where no atom has two images in its box (open structures, cells at least
+// two cutoffs across) each lane takes its own.  Otherwise the images of all of them are spread over the lanes in (atom,
+// image) order, twice: to count what each atom keeps and find its nearest image, and to write the entries, next to
+// each other.  Places in the row come from scans inside the wavefront and the wavefronts' totals through LDS.
+// A lane that walks its own atom's images costs the wavefront the longest walk, in a chain of FP64 latencies, twice:
+// about 110 images are within reach of a centre, all of them on two lanes of a two-atom cell.  Walked so / now: 20 uneven
+// cells of up to 512 atoms 24.5 / 9.1 us, one of 64 atoms 9.7 / 8.2, 600 of 20 atoms 51 / 29, 60 of 250 atoms 57 / 42, 512
+// of up to 512 atoms 101 / 67, open structures of 2000 and 7000 atoms 46 / 26 and 234 / 163.
+// W: four wavefronts a centre shorten the chain while the centres alone leave the chip idle; beyond kPairCentres one
+// (34,700 centres: four 140 us, one 96, before the single-image path; 4,800: 24 against 17 us).
+constexpr int kPairCentres = 2048;
 struct PairChunk {  // a wavefront's 64 atoms
     double b[3][kWave];              // difference vector
     unsigned long long mind[kWave];  // bits of the smallest distance
     int off[kWave], lo[3][kWave], ext[2][kWave];  // first image, box of images (lowest indexes, last two extents)
     int type[kWave], kept[kWave], minn[kWave];
 };
-__global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
+template <int W>
+__global__ __launch_bounds__(kWave * W) void k_neigh_allpairs(const DevStruc* __restrict__ S, const int* __restrict__ atom_struc,
                                                           const double* __restrict__ pos, const int* __restrict__ type,
                                                           const int* __restrict__ centres, double rc2, int maxp,
                                                           int* __restrict__ cnt, int* __restrict__ nbr_j,
                                                           int* __restrict__ nbr_meta, double4* __restrict__ nbr_r,
                                                           unsigned short* __restrict__ row_tab, unsigned short* __restrict__ nbr_key, PassCounters pc) {
     clear_counters(pc);
-    __shared__ PairChunk chunk[kPairWaves];
-    __shared__ int wtot[2][kPairWaves];
+    __shared__ PairChunk chunk[W];
+    __shared__ int wtot[2][W];
     const int i = centres[blockIdx.x];
     const DevStruc& s = S[atom_struc[i]];
     const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const bool one = s.natoms <= kWave;  // (uniform)
+    const bool one = W == 1 || s.natoms <= kWave;  // (uniform)
     if (one && w > 0) return;
     const int li = i - s.atom0;
     const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
@@ -200,15 +204,16 @@ __global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const Dev
         __builtin_amdgcn_wave_barrier();
     };
     int written = 0;
-    for (int j0 = 0, buf = 0; j0 < s.natoms; j0 += kWave * kPairWaves, buf ^= 1) {
+    for (int j0 = 0, buf = 0; j0 < s.natoms; j0 += kWave * W, buf ^= 1) {
         const int jw = j0 + w * kWave, j = jw + lane;
         const bool valid = j < s.natoms;
         double bx = 0, by = 0, bz = 0;
         // images of this j that can be within rc (open structures: the single image 0)
         ImgRange g{{0, 0, 0}, {-1, -1, -1}};
+        int tj = 0;
         if (valid) {
             const int gj = s.atom0 + j;
-            L.type[lane] = type[gj];
+            tj = type[gj];
             const double dx = xi - pos[3 * gj], dy = yi - pos[3 * gj + 1], dz = zi - pos[3 * gj + 2];
             if (periodic) {
                 cell_diff(s, dx, dy, dz, bx, by, bz);
@@ -221,19 +226,40 @@ __global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const Dev
             }
         }
         const int e0 = max(0, g.hi[0] - g.lo[0] + 1), e1 = max(0, g.hi[1] - g.lo[1] + 1), e2 = max(0, g.hi[2] - g.lo[2] + 1);
-        int images;  // of the wavefront's atoms
-        L.off[lane] = wave_excl_scan(e0 * e1 * e2, lane, images);
-        L.b[0][lane] = bx;
-        L.b[1][lane] = by;
-        L.b[2][lane] = bz;
+        const int mimg = e0 * e1 * e2;
+        // no atom with two images (open structures, cells at least two cutoffs across): each lane takes its own
+        const bool single = __all(mimg <= 1);
+        int images = 0, mine = 0, n1 = 0;  // images of the wavefront's atoms; with `single` this lane's
+        double rx1 = 0, ry1 = 0, rz1 = 0, d1 = 0;
+        if (single) {
+            if (mimg == 1) {
+                n1 = ((g.lo[0] + s.shell[0]) * w1 + (g.lo[1] + s.shell[1])) * w2 + (g.lo[2] + s.shell[2]);
+                double ix = 0, iy = 0, iz = 0;
+                if (periodic) image_vec(s, g.lo[0], g.lo[1], g.lo[2], ix, iy, iz);
+                rx1 = bx - ix;
+                ry1 = by - iy;
+                rz1 = bz - iz;
+                const double d2 = rx1 * rx1 + ry1 * ry1 + rz1 * rz1;
+                if (d2 <= rc2 && (j != li || 1e-6 < d2)) {
+                    mine = 1;
+                    d1 = sqrt(d2);
+                }
+            }
+        } else {
+            L.type[lane] = tj;
+            L.off[lane] = wave_excl_scan(mimg, lane, images);
+            L.b[0][lane] = bx;
+            L.b[1][lane] = by;
+            L.b[2][lane] = bz;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) L.lo[q][lane] = g.lo[q];
-        L.ext[0][lane] = e1;
-        L.ext[1][lane] = e2;
-        L.kept[lane] = 0;
-        L.mind[lane] = __double_as_longlong(fro);  // (distances are positive: their bits order as they do)
-        L.minn[lane] = INT_MAX;
-        ordered();
+            for (int q = 0; q < 3; ++q) L.lo[q][lane] = g.lo[q];
+            L.ext[0][lane] = e1;
+            L.ext[1][lane] = e2;
+            L.kept[lane] = 0;
+            L.mind[lane] = __double_as_longlong(fro);  // (distances are positive: their bits order as they do)
+            L.minn[lane] = INT_MAX;
+            ordered();
+        }
         // image q of the wavefront's: its atom (the last whose images begin at or before q), offset and vector
         const auto image = [&](int q, int& k, int& n, double& rx, double& ry, double& rz) {
             k = 0;
@@ -260,8 +286,10 @@ __global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const Dev
             atomicAdd(&L.kept[k], 1);
             if (periodic && jw + k != li) atomicMin(&L.mind[k], (unsigned long long)__double_as_longlong(sqrt(d2)));
         }
-        ordered();
-        const int mine = L.kept[lane];
+        if (!single) {
+            ordered();
+            mine = L.kept[lane];
+        }
         int tot;
         int at = written + wave_excl_scan(mine, lane, tot);
         if (!one) {
@@ -269,7 +297,7 @@ __global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const Dev
             __syncthreads();  // (the other buffer's readers passed the barrier before)
             tot = 0;
 #pragma unroll
-            for (int v = 0; v < kPairWaves; ++v) {
+            for (int v = 0; v < W; ++v) {
                 const int c = wtot[buf][v];
                 if (v < w) at += c;
                 tot += c;
@@ -277,6 +305,9 @@ __global__ __launch_bounds__(kWave * kPairWaves) void k_neigh_allpairs(const Dev
         }
         // the row's index table: atom j opens slot j / width when it is the slot's first
         if (valid && j % tw == 0) row_tab[(int64_t)i * kRowTab + j / tw] = (unsigned short)min(at, maxp);
+        if (single && mine && at < maxp)
+            put_entry(row + at, j, n1, tj, j != li && periodic && d1 < fro, rx1, ry1, rz1, d1, nbr_j, nbr_key, nbr_meta,
+                      nbr_r);
         int put = __builtin_amdgcn_readfirstlane(at);  // (lane 0's: the wavefront's first entry)
         for (int q0 = 0; q0 < images; q0 += kWave) {
             int k = 0, n = 0;
@@ -922,8 +953,12 @@ hipError_t launch_neighbors(const NeighborArgs& a, hipStream_t st) {
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.npair > 0) {
-        hipLaunchKernelGGL(k_neigh_allpairs, dim3(a.npair), dim3(kWave * kPairWaves), 0, st, a.S, a.atom_struc, a.pos, a.type,
-                           a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
+        if (a.npair <= kPairCentres)
+            hipLaunchKernelGGL(k_neigh_allpairs<4>, dim3(a.npair), dim3(kWave * 4), 0, st, a.S, a.atom_struc, a.pos, a.type,
+                               a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
+        else
+            hipLaunchKernelGGL(k_neigh_allpairs<1>, dim3(a.npair), dim3(kWave), 0, st, a.S, a.atom_struc, a.pos, a.type,
+                               a.pair_centres, a.rc2, a.maxp, a.cnt, a.nbr_j, a.nbr_meta, a.nbr_r, a.row_tab, a.nbr_key, pc);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.ntot > 0 && a.count_max) return launch_count_max(a.cnt, a.ntot, a.maxcnt, st);
