@@ -285,23 +285,21 @@ static float bf16_value(uint16_t h) {
     return x;
 }
 
-// A layer's FP32 weights as the B operand of v_mfma_f32_16x16x32_bf16, split x = hi + lo + rest: for column tile jt
-// and step s of 32 in K, 64 lanes x 8 values of hi, of lo, then of the rest, where lane l holds B[32 s + 8 (l / 16) + q][16 jt + l % 16]
+// A layer's FP32 weights as the B operand of v_mfma_f32_16x16x32_bf16, split x = hi + lo: for column tile jt and
+// step s of 32 in K, 64 lanes x 8 values of hi, then of lo, where lane l holds B[32 s + 8 (l / 16) + q][16 jt + l % 16]
 // (zero past the layer), so a wavefront loads each operand as one 16-byte load per lane over 1 KB.
 template <class B>
 static int pack_net_bf(std::vector<uint16_t>& out, int ncol, int K, B value) {
     const int at = (int)(out.size() / 8);
     for (int jt = 0; jt < ncol / 16; ++jt)
         for (int s = 0; s < (K + 31) / 32; ++s)
-            for (int part = 0; part < 3; ++part)
+            for (int part = 0; part < 2; ++part)
                 for (int l = 0; l < 64; ++l)
                     for (int q = 0; q < 8; ++q) {
                         const int k = 32 * s + 8 * (l / 16) + q;
                         const float x = k < K ? (float)value(k, 16 * jt + l % 16) : 0.f;
                         const uint16_t hi = bf16_bits(x);
-                        const float r = x - bf16_value(hi);
-                        const uint16_t lo = bf16_bits(r);
-                        out.push_back(part == 0 ? hi : part == 1 ? lo : bf16_bits(r - bf16_value(lo)));
+                        out.push_back(part == 0 ? hi : bf16_bits(x - bf16_value(hi)));
                     }
     return at;
 }

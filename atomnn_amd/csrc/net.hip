@@ -497,14 +497,13 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mixed(const DevPlan* 
 // The mixed form for networks of H = 1 to 3 tanh layers of at most 64 units (net_bf_hidden): a block of four
 // wavefronts takes 32 atoms of a species as two 16-row MFMA tiles, and each wavefront one 16-column tile of every
 // hidden layer, so a layer's activations, derivatives and deltas of its tile stay in the wavefront's registers
-// and only the split operands of the next product go through LDS.  Besides k_net_mixed's three products of the high and
-// low parts it takes low by low and the weights' third part by high, which are MFMA work alone: the error of the
-// mixed forces falls from 1.0e-5 to 5.2e-6 of their size (300-atom cells), for 3 us on 65536 atoms.
+// and only the split operands of the next product go through LDS.  The same split products in the same order as
+// k_net_mixed (the energy's row dot products are summed in another order).
 // k_net_mixed converts and splits its operands at every use (each weight once per 16 atoms, each activation once
 // per column tile), 1984 VALU instructions per wavefront and 16 atoms, and reads the weights of the
 // backward products a 4-byte column element at a time.  Here the weights are split once per model and laid out
 // as operands (16 bytes per lane, 1 KB per wavefront), and an activation is split once, where it is computed.
-// 65536 atoms, 84-64-64-1: 130 -> 48 us; 11003 atoms 31 -> 18 us.
+// 65536 atoms, 84-64-64-1: 130 -> 46 us; 11003 atoms 31 -> 18 us.
 constexpr int kBfRows = 32;
 __host__ __device__ constexpr int bf_lda(int k) { return (k + 31) / 32 * 32 + 8; }  // rows start in different banks
 static size_t net_bf_lds_bytes(const DevNet& n) {
@@ -518,22 +517,17 @@ __device__ __forceinline__ void bf_mm(const __bf16* A, int lda, const uint4* __r
     const int li = lane & 15, lk = lane >> 4;
     const int ns = (K + 31) / 32;
     acc[0] = acc[1] = f4_t{0.f, 0.f, 0.f, 0.f};
-    const uint4* b = B + (size_t)jt * ns * 192 + lane;
+    const uint4* b = B + (size_t)jt * ns * 128 + lane;
     const __bf16* a = A + li * lda + 8 * lk;
     for (int s = 0; s < ns; ++s) {
-        const bf8_t bh = __builtin_bit_cast(bf8_t, b[s * 192]);
-        bf8_t bl{}, br{};
-        if constexpr (TERMS == 3) {
-            bl = __builtin_bit_cast(bf8_t, b[s * 192 + 64]);
-            br = __builtin_bit_cast(bf8_t, b[s * 192 + 128]);
-        }
+        const bf8_t bh = __builtin_bit_cast(bf8_t, b[s * 128]);
+        bf8_t bl{};
+        if constexpr (TERMS == 3) bl = __builtin_bit_cast(bf8_t, b[s * 128 + 64]);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             const bf8_t ah = *reinterpret_cast<const bf8_t*>(a + t * 16 * lda + 32 * s);
             if constexpr (TERMS == 3) {
                 const bf8_t al = *reinterpret_cast<const bf8_t*>(a + (kBfRows + t * 16) * lda + 32 * s);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, br, acc[t], 0, 0, 0);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bl, acc[t], 0, 0, 0);
                 acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc[t], 0, 0, 0);
                 acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc[t], 0, 0, 0);
             }
