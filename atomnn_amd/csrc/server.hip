@@ -72,14 +72,15 @@ class Server {
         for (auto& t : workers_) t.join();
     }
 
-    // Estimated device bytes of a batch of `atoms` atoms with about `p` entries per atom:
-    // neighbour rows (40 B), force terms (32 B) and per-atom arrays (descriptor and dE/dG rows, the
-    // moment table of S NE 35 values).
+    // Estimated device bytes of a batch of `atoms` atoms with about `p` entries per atom: neighbour rows (index,
+    // metadata and displacement 40 B, key 2 B) and force terms (32 B), and per-atom arrays: descriptor and dE/dG rows,
+    // the moment table of S NE 35 values, the rows' index tables (64 B), bins, ranks and bin-ordered positions (24 B),
+    // inputs, results and counters (about 124 B).
     size_t estimate(size_t atoms, double p) const {
         const size_t maxp = (size_t)std::ceil(p * 1.5 + 16);
         const int ne = owner_.shape == 0 ? 2 : (owner_.shape == 1 ? 4 : 8);  // exponents of the grid shape
         const size_t mom = (size_t)owner_.pb.plan.T * ne * 35 * 8;           // FP64 bound
-        return atoms * (maxp * 72 + (size_t)owner_.pb.plan.ldg * 16 + mom + 128) + (1 << 20);
+        return atoms * (maxp * 74 + (size_t)owner_.pb.plan.ldg * 16 + mom + 212) + (1 << 20);
     }
 
     int64_t submit(const nnp_structure& s, nnp_result* out) {
