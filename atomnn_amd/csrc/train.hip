@@ -1239,10 +1239,13 @@ class TrainSet {
         // forward + backward pass per tile gives the outputs and the gradient rows of the outputs,
         // which the reduction weights by dcdo; otherwise species tiles across structures, a forward
         // pass for the energies and a second pass with the loss seeds.  The tiles of the previous
-        // call are reused when the batch and mode repeat.
+        // call are reused when the batch, mode and row buffer repeat.
         const int mode = grad ? (owner_.train_one_pass ? 2 : 1) : 0;
         std::vector<int> key(batch, batch + nbatch);
         key.push_back(mode);
+        // (the rows that one buffer holds decide between the forms below)
+        key.push_back((int)(owner_.train_chunk_elems >> 32));
+        key.push_back((int)(owner_.train_chunk_elems & 0xffffffff));
         if (key != tiles_key_) {
             tiles_key_.clear();
             std::vector<int> bstart(nbatch + 1, 0);
