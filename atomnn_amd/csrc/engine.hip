@@ -3,12 +3,12 @@
 // Pipeline for a batch of structures (all kernels cover every atom of every structure):
 //   1. neighbour list      k_bins_small or k_bin_atoms / k_bin_scan / k_fill_bins, then
 //                          k_neigh_cells_bits (large cells), k_neigh_allpairs (small cells)
-//   2. descriptors         k_symm<T, NE, NC>                 -> G
-//   3. networks            k_net_f64 | k_net_mixed, all species' 16-atom tiles -> E_i, dE/dG
-//   4. force terms         k_force<T, NE, NC>                 -> X (per neighbour entry)
+//   2. descriptors         k_symm_mom | k_symm_pow | k_symm<T, NE, NC>  -> G
+//   3. networks            k_net_f64 | k_net_mixed32 | k_net_mixed, tiles of every species' atoms -> E_i, dE/dG
+//   4. force terms         k_force_mom | k_force_pow | k_force<T, NE, NC>  -> X (per neighbour entry)
 //   5. force assembly      k_assemble (gathers each atom's reactions from its neighbours' rows) -> F (FP64)
-//   6. energy              per structure, sum of E_i in atom order (FP64), as
-//                          NNP::energy accumulates (nnp.cpp:394-400)
+//   6. energy              per structure, sum of E_i in FP64 (NNP::energy, nnp.cpp:394-400): on the host in atom order
+//                          for a synchronous call, by energy_tail_block (strided chains, a tree) for a resident pass
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -10,8 +10,8 @@
 // and no min flags (neighbor.cpp:149-170).
 //
 // Two searches produce the same list:
-//  * all-pairs: one wavefront per centre sweeps j in chunks of 64 lanes; each lane tests
-//    the images of its j, a wave prefix sum places the kept entries in order.  Used for
+//  * all-pairs: a centre's wavefronts sweep j in chunks of 64; the (j, image) pairs within
+//    reach are spread over the lanes, prefix sums place the kept entries in order.  Used for
 //    small cells (any image shell > 0) and small structures.
 //  * cell list: for structures whose image shells are all 0 (every cell height > 2 rc) the
 //    entry of j is exactly diff(r_i, r_j) when within rc; candidates come from the 27
@@ -63,18 +63,11 @@ __device__ __forceinline__ void cell_diff(const DevStruc& s, double dx, double d
     }
 }
 
+// image vector R_n = a Rv0 + b Rv1 + c Rv2 (neighbor.cpp:87-95)
 __device__ __forceinline__ void image_vec(const DevStruc& s, int a, int b, int c, double& x, double& y, double& z) {
     x = (double)a * s.Rv[0] + (double)b * s.Rv[3] + (double)c * s.Rv[6];
     y = (double)a * s.Rv[1] + (double)b * s.Rv[4] + (double)c * s.Rv[7];
     z = (double)a * s.Rv[2] + (double)b * s.Rv[5] + (double)c * s.Rv[8];
-}
-// image vector R_n = a Rv0 + b Rv1 + c Rv2 for linear index n (neighbor.cpp:87-95)
-__device__ __forceinline__ void image_vec(const DevStruc& s, int n, double& x, double& y, double& z) {
-    const int w2 = 2 * s.shell[2] + 1, w1 = 2 * s.shell[1] + 1;
-    const int c = n % w2 - s.shell[2];
-    const int b = (n / w2) % w1 - s.shell[1];
-    const int a = n / (w2 * w1) - s.shell[0];
-    image_vec(s, a, b, c, x, y, z);
 }
 
 // Exclusive prefix sum over the wavefront in six DPP adds: shifts by 1, 2, 4 and 8 inside each row of 16
@@ -680,8 +673,9 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
 // search took 18.0 us on 4096 atoms (2 species, rc 6) and 205 us on 16 x 4096 atoms (rc 6.5); with the filter
 // 10.9 us and 102 us (728 instead of 1516 VALU instructions per centre).
 //
-// The filter must keep everything Cell::diff would.  A cell-list structure has every height > 2 rc, so an
-// entry within rc has fractional components |f| <= rc / h < 1/2 and is the image that rounding picks; the FP32
+// The filter must keep everything Cell::diff would.  A cell-list structure has every height h > 2 rc: its last image
+// shell is 0, so V / (|Rv0| |Rv1|) > 2 rc over the two longest vectors, and every height V / |Ri x Rj| is at least that.  An
+// entry within rc then has fractional components |f| <= rc / h < 1/2 and is the image that rounding picks; the FP32
 // coordinates (in [0, 1], error 2^-25) put the distance off by less than 4e-7 ||R||_F, and the filter adds
 // 1e-6 ||R||_F.  Where some rc / h is within 1e-4 of 1/2 the rounding could take the other image, and
 // where a row could hold more than the register batches (maxp > 192) or the filter lists more than they

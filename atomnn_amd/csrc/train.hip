@@ -1071,7 +1071,7 @@ class TrainSet {
             if (batch[b] < 0 || batch[b] >= nst) throw std::invalid_argument(std::string(fn) + ": structure out of range");
     }
 
-    // parameters: reference order -> padded row-major layers, uploaded on stream st
+    // Parameters from the reference's order to padded row-major layers, on stream st.
     // Staging of one call: [x, total][results: gradient, then three values a structure].  One kernel reads x in place and
     // one copy brings every result; with the parameters transposed on the host, four to fifteen pageable copies, and
     // the tiles and reference values of a chunk sent again on each call, a call waited more than it computed: 194 us
@@ -1108,8 +1108,6 @@ class TrainSet {
         }
     };
 
-    // Species tiles of 16 atoms over the given (source row, slot, structure) lists per species,
-    // uploaded into d_batom_, d_bslot_, d_bstruct_ on stream st.
     // What a batch's tiles read: atoms, slots and structures by species, first slots, reference energies, first
     // reference force of each structure (force training).
     struct TileArrays {
@@ -1129,6 +1127,8 @@ class TrainSet {
         bool settled = false;  // its rows' reaction tables are known to miss nothing
     };
 
+    // Species tiles of 16 atoms over the given (source row, slot, structure) lists per species,
+    // uploaded into ta's tables on stream st.
     Tiles make_tiles(const std::vector<std::vector<int>>& atom_s, const std::vector<std::vector<int>>& slot_s,
                      const std::vector<std::vector<int>>& struct_s, hipStream_t st, TileArrays& ta) {
         Tiles r;
@@ -1183,14 +1183,14 @@ class TrainSet {
             }
             launch(tc, c0, c1);
             HIPCHK(hipGetLastError());
-            reduce_rows(tl, tc, c0, c1, st, nullptr, nullptr);
+            reduce_rows(tc, c0, c1, st, nullptr, nullptr);
         }
     }
 
-    // The gradient (d_res_; set by a call's first rows) += the rows of tiles [c0, c1) (bases tc), optionally weighted by dcdo[tstruct[tile]].
-    void reduce_rows(const Tiles& tl, const TrainTiles& tc, int c0, int c1, hipStream_t st, const int* tstruct,
+    // The gradient (d_res_; set by a call's first rows) += the rows of tiles [c0, c1) (bases tc), optionally weighted by
+    // dcdo[tstruct[tile]].
+    void reduce_rows(const TrainTiles& tc, int c0, int c1, hipStream_t st, const int* tstruct,
                      const double* dcdo) {
-        (void)tl;
         if (c1 <= c0) return;
         int64_t maxnp = 1;
         for (int t = 0; t < T_; ++t) maxnp = std::max<int64_t>(maxnp, plan_.net[t].nparams);
@@ -1369,10 +1369,10 @@ class TrainSet {
         if (grad) {
             if (grouped_) {
                 if (!one_pass_) HIPCHK(launch_group<true>(gshape_, ga, stream_));
-                reduce_rows(tl, groups_.rows, 0, groups_.n, stream_, one_pass_ ? (const int*)d_tstruct_.p : nullptr,
+                reduce_rows(groups_.rows, 0, groups_.n, stream_, one_pass_ ? (const int*)d_tstruct_.p : nullptr,
                             (const double*)d_dcdo_.p);
             } else if (one_pass_) {
-                reduce_rows(tl, tl.tt, 0, tl.tiles, stream_, (const int*)d_tstruct_.p, (const double*)d_dcdo_.p);
+                reduce_rows(tl.tt, 0, tl.tiles, stream_, (const int*)d_tstruct_.p, (const double*)d_dcdo_.p);
             } else {
                 sum_tiles(tl, stream_, [&](const TrainTiles& tc, int c0, int c1) {
                     launch_tile<1>(gen_, dim3(c1 - c0), lds, stream_, tpp, Wm, par, tc, c0, ba, bsl, bst, Gp, ldg_,
