@@ -671,7 +671,7 @@ __global__ __launch_bounds__(kWave) void k_neigh_cells(const DevStruc* __restric
 // Bound by the VALU instructions it issues and the latency of its loads.  Cell::diff is about 60 FP64
 // operations; on every candidate and again on every set bit (a lane per bitmap word, most lanes idle) the
 // search took 18.0 us on 4096 atoms (2 species, rc 6) and 205 us on 16 x 4096 atoms (rc 6.5); with the filter
-// 10.9 us and 102 us (728 instead of 1516 VALU instructions per centre).
+// 11 us and 104 us (744 instead of 1516 VALU instructions per centre of the latter).
 //
 // The filter must keep everything Cell::diff would.  A cell-list structure has every height h > 2 rc: its last image
 // shell is 0, so V / (|Rv0| |Rv1|) > 2 rc over the two longest vectors, and every height V / |Ri x Rj| is at least that.  An

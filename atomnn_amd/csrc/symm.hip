@@ -1692,8 +1692,8 @@ static hipError_t launch_force_mom_t(const DevPlan* plan, const double* rfe, con
 // the sums on the vector unit (k_symm: per-lane monomials over half-waves, functions over lanes, the cutoff once per
 // species and once more for the angular factors) FP64 took 2203 VALU instructions per centre at P = 45 (2
 // species, NE = 4, 16 radial functions) and FP32 2048 at P = 69 (3 species, NE = 2, 12): 29.2 us on 4096 atoms, 240 us
-// on 16 x 4096.  Here 1018 and 973 instructions, 21.5 us and 163 us (of which exp_f64, sincospi_f64, entries staged in
-// registers, K-steps unrolled over a chunk and products with uniform trip counts: 1663 -> 1018, 26.1 -> 21.5 us), and at
+// on 16 x 4096.  Here 1115 and 1004 instructions, 21.5 us and 155 us (of which exp_f64, sincospi_f64, entries staged in
+// registers, K-steps unrolled over a chunk and products with uniform trip counts: 1663 -> 1115, 26.1 -> 21.5 us), and at
 // row head room (molecular dynamics) 34.7 -> 22 us: the moments take the entries' LDS after the sums, 7.2 instead of 9.9 KB
 // a centre.
 // LDS in elements of T: the entries (u, d), their B values and a chunk of power rows, then, in their place, the
