@@ -92,6 +92,27 @@ __device__ __forceinline__ double train_act_d2(int act, double z, double a) {
     return act == NEU_LINEAR ? 0.0 : -2.0 * a * (1.0 - a * a);
 }
 
+// Sum over the 16 lanes of a DPP row, on every lane.
+__device__ __forceinline__ double row16_sum(double x) {
+    auto ror = [](double y, auto ctrl) {
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(y), ctrl.value, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(y), ctrl.value, 0xf, 0xf, false);
+        return __hiloint2double(hi, lo);
+    };
+    x += ror(x, std::integral_constant<int, 0x128>{});
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    return x + ror(x, std::integral_constant<int, 0x121>{});
+}
+// The output unit's sum over 16 of its inputs, one a lane of a DPP row.  Every kernel adds the inputs in this order, 16 at a
+// time, and forms the output by train_out, so that a call gives the same errors with and without the gradient, whichever
+// kernel takes the tiles.
+__device__ __forceinline__ double train_unit_part(double w, double a) {
+#pragma clang fp contract(off)
+    return row16_sum(w * a);
+}
+__device__ __forceinline__ double train_out(double outb, double outw, double z) { return fma(z, outw, outb); }
+
 // LDS: ins [16][nin_pad], then per layer A_l [16][wpad_l] and D_l [16][wpad_l] (dadz; dcdz in the
 // backward pass, in place).
 static size_t train_lds_bytes(const TrainNet& n) {
@@ -141,7 +162,18 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_tile(
     for (int l = 0; l < N.L; ++l) {
         const double* prev = l == 0 ? ins : A[l - 1];
         const int in_pad = l == 0 ? N.nin_pad : N.wpad[l - 1], wp = N.wpad[l];
-        const int act = l == N.L - 1 ? NEU_LINEAR : N.act;
+        if (l == N.L - 1) {  // linear, one unit: four rows a wavefront
+            static_assert(kTrainWaves * 4 == 16, "a tile's 16 rows");
+            const int row = 4 * wv + lk;
+            double e = 0.0;
+            for (int n = 0; n < in_pad; n += 16) e += train_unit_part(par[N.woff[l] + n + li], prev[row * in_pad + n + li]);
+            for (int n = li; n < wp; n += 16) {
+                A[l][row * wp + n] = n == 0 ? par[N.boff[l]] + e : 0.0;
+                D[l][row * wp + n] = 1.0;
+            }
+            __syncthreads();
+            break;
+        }
         for (int jt = wv; jt < wp / 16; jt += kTrainWaves) {
             const d4_t acc = tile_mm_f64<true>(prev, in_pad, par + N.woff[l], in_pad, in_pad, jt, li, lk);
             const int col = jt * 16 + li;
@@ -149,7 +181,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_tile(
             for (int v = 0; v < 4; ++v) {
                 const int row = 4 * v + lk;
                 double av, dv;
-                train_act<GEN>(act, acc[v] + par[N.boff[l] + col], av, dv);
+                train_act<GEN>(N.act, acc[v] + par[N.boff[l] + col], av, dv);
                 A[l][row * wp + col] = av;
                 D[l][row * wp + col] = dv;
             }
@@ -159,7 +191,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_tile(
     const int L = N.L;
     if constexpr (MODE != 1) {
         if (tid < 16 && r0 + tid < M && batom[a0 + r0 + tid] >= 0)
-            out[bslot[a0 + r0 + tid]] = N.outb + A[L - 1][tid * N.wpad[L - 1]] * N.outw;
+            out[bslot[a0 + r0 + tid]] = train_out(N.outb, N.outw, A[L - 1][tid * N.wpad[L - 1]]);
     }
     if constexpr (MODE == 0) {
         return;
@@ -269,18 +301,6 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_tile(
 // a CU 70 and 68 us, with the library's expm1 and quotient in tanh 82.
 // Registers: U = 64 leaves a wavefront 256, which H = 2 with more than 96 inputs does not fit; those networks keep
 // k_train_tile, as do other depths, activations and widths.
-// Sum over the 16 lanes of a DPP row, on every lane.
-__device__ __forceinline__ double row16_sum(double x) {
-    auto ror = [](double y, auto ctrl) {
-        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(y), ctrl.value, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(y), ctrl.value, 0xf, 0xf, false);
-        return __hiloint2double(hi, lo);
-    };
-    x += ror(x, std::integral_constant<int, 0x128>{});
-    x += ror(x, std::integral_constant<int, 0x124>{});
-    x += ror(x, std::integral_constant<int, 0x122>{});
-    return x + ror(x, std::integral_constant<int, 0x121>{});
-}
 template <int NI>
 __host__ __device__ constexpr int tg_ldi() {
     return 16 * NI + 4;  // LDS rows: the 16 rows of a K-step start in different banks
@@ -443,7 +463,7 @@ __global__ __launch_bounds__(8 * U, U / 32) void k_train_group(
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const double sd = seed[b * 16 + 4 * v + lk];
-            const double e = row16_sum(wo * av[v]);
+            const double e = train_unit_part(wo, av[v]);
             if (li == 0) ep[wv * 16 + 4 * v + lk] = e;
             gwo += sd * av[v];
             dz[v] = sd * wo * d1[v];
@@ -457,7 +477,7 @@ __global__ __launch_bounds__(8 * U, U / 32) void k_train_group(
             double e = 0.0;
 #pragma unroll
             for (int n = 0; n < MH; ++n) e += ep[n * 16 + lane];
-            if (slot >= 0) out[slot] = outb + (bo + e) * outw;
+            if (slot >= 0) out[slot] = train_out(outb, outw, bo + e);
         }
         if constexpr (H == 2) {
             // layer 1's weight gradient a_0^T dz_1 (rows: layer-0 units), and dz_0 = (dz_1 W_1) .* d_0
