@@ -177,7 +177,9 @@ int nnp_profile_read(nnp_model* m, double* ms, int64_t* calls, int nstage);
  *   "moments"   bit 0: descriptor angular sums by the moment expansion, bit 1: the angular
  *               force terms by it (default 3, both); clear bits take the triplet loops; models
  *               outside its domain (integer zeta <= 4, |lambda| <= 1, one exponent table per
- *               centre species) take the triplet loops whatever the bits
+ *               centre species) visit the pairs whatever the bits: in the power-ladder kernels
+ *               for zeta 1, 2, 4, 8, 16 with lambda +-1 and up to four exponents, else in the
+ *               triplet loops
  *   "force_waves"  1 = one wavefront per centre in the force-term kernel (default), 2 = two
  *               wavefronts split a centre's exponents, radial functions and moment entries
  *               (moment path on fast-path models only)
